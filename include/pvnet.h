@@ -36,11 +36,11 @@ enum { PVNET_RELU = 1, PVNET_F32OUT = 2, PVNET_GATHER = 4 };
  * ntaps*cin.  If relu_of is not NULL the result is multiplied by (relu_of[m][n] > 0) (the
  * backward of a ReLU whose output is relu_of).  flags: PVNET_RELU applies max(., 0);
  * PVNET_F32OUT writes float instead of bf16.  y may be a channel slice of a wider tensor.
- * 3x3x3 convolutions with 16, 32, 48 or 64 outputs (or multiples of 48 or 64) on grids of whole
- * 16 x 4 x 4 bricks (x, y, z; 16 x 8 x 4 where the halo fits) stage each brick and its halo in
- * LDS once; PVNET_GATHER keeps them on the per-tap gathering kernel (the same result bit for bit,
- * for comparison).  Pointwise convolutions with cin <= 32 and cout <= 64 take their matrix-core
- * operands straight from global memory (no LDS); PVNET_GATHER keeps them on the tiled kernel
+ * 3x3x3 convolutions whose rows can be written four channels at a time (cout and ldy multiples of 4,
+ * y aligned to 8 bytes, 16 with PVNET_F32OUT, relu_of likewise) march through z with their input
+ * planes in LDS; PVNET_GATHER keeps them on the per-tap gathering kernel (the same result bit for
+ * bit, for comparison), which also takes the shapes that fit no plan.  Pointwise convolutions with
+ * cin <= 32 and cout <= 64 take their matrix-core operands straight from global memory (no LDS); PVNET_GATHER keeps them on the tiled kernel
  * (again the same result bit for bit). */
 typedef struct {
     pvnet_shape s;

@@ -19,6 +19,7 @@
 #include <cmath>
 #include <cstdint>
 #include <string>
+#include <type_traits>
 
 #include "../../include/pvnet.h"
 
@@ -244,158 +245,8 @@ __global__ __launch_bounds__(256) void k_conv_pw(pvnet_conv a, int M) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// 3x3x3 convolution with 16 NT output channels per block (NT = 1..4 column tiles; grid.y takes
-// further groups of 16 NT channels) on grids of whole 16 x 4 x 4
-// bricks: each block stages one brick of one box with its one-voxel halo (18 x 6 x 6 voxels, all
-// cin channels) in LDS once and runs the k-steps of k_conv_fwd over it, where k_conv_fwd gathers
-// every tap's rows from L2 again.  The k-steps, their operands and their order are those of
-// k_conv_fwd, so each output is the same bit for bit.  Wave wv computes brick plane z = wv as 4
-// MFMA row tiles (y = tile) of 16 voxels (x = MFMA row).  The halo is stored chunk-major
-// (halo[chunk][voxel], a chunk = 8 channels, 16 bytes), so the 16 lanes that read one A fragment
-// row group address 16 consecutive 16-byte rows: one pass over the 64 banks.
-
-// bricks of BRX x BY x BRZ voxels (BY = 4 or 8, one wave per 4 rows of a plane), halo HLX x (BY + 2)
-// x HLZ
-constexpr int BRX = 16, BRZ = 4;
-constexpr int HLX = BRX + 2, HLZ = BRZ + 2;
-template <int BY>
-constexpr int hl_vox() { return HLX * (BY + 2) * HLZ; }
-
-// step table: entry 4 s + g = the halo offset of k-values s * 32 + 8 g .. + 7 relative to the
-// output voxel (chunk * HLV + tap shift), plus BR_TAB_BIAS; 0 where they lie beyond K
-constexpr int BR_TAB_BIAS = 1 << 20;
-
-// WL: the block's weight rows are staged in LDS after the step table (row pitch kpad + 8 bf16, an
-// odd number of 16-byte units, so the 16 rows one fragment reads fall on distinct banks), instead
-// of being read from global memory one step ahead.
-template <int NT, int BY, bool WL>
-__global__ __launch_bounds__(64 * BY) void k_conv_fwd_brick(pvnet_conv a, int K) {
-    constexpr int HLY = BY + 2, HLV = hl_vox<BY>(), NTH = 64 * BY;
-    extern __shared__ uint4 halo[];  // [cin / 8 chunks][HLV voxels], the step table, WL: weights
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    const int zz = wv % BRZ, yq = wv / BRZ;  // this wave: plane zz, rows 4 yq .. 4 yq + 3
-    const int g = lane >> 4, c16 = lane & 15;
-    const int d = a.s.d, h = a.s.h, w = a.s.w;
-    const int nbx = w / BRX, nby = h / BY, nbz = d / BRZ;
-    int bid = xcd_tile(blockIdx.x, gridDim.x);
-    const int bx = bid % nbx;
-    bid /= nbx;
-    const int by = bid % nby;
-    bid /= nby;
-    const int bz = bid % nbz;
-    const int box = bid / nbz;
-    const int x0 = bx * BRX, y0 = by * BY, z0 = bz * BRZ;
-    const int n0 = blockIdx.y * 16 * NT;
-    const int cch = a.cin >> 3;
-    const int nsteps = a.kpad / BK;
-    int* tab = reinterpret_cast<int*>(halo + HLV * cch);
-    for (int i = t; i < 4 * nsteps; i += NTH) {
-        const int k = (i >> 2) * BK + (i & 3) * 8;
-        int v = 0;
-        if (k < K) {
-            const int tap = k / a.cin, ci = k - tap * a.cin;
-            int dz, dy, dx;
-            tap_offset(27, tap, dz, dy, dx);
-            v = (ci >> 3) * HLV + (dz * HLY + dy) * HLX + dx + BR_TAB_BIAS;
-        }
-        tab[i] = v;
-    }
-    uint4* wl = reinterpret_cast<uint4*>(tab + 4 * nsteps);
-    const int WP = 4 * nsteps + 1;  // 16-byte units per weight row in LDS
-    if constexpr (WL) {
-        for (int i = t; i < 16 * NT * 4 * nsteps; i += NTH) {
-            const int row = i / (4 * nsteps), col = i - row * (4 * nsteps);
-            wl[row * WP + col] = *(const uint4*)(a.w + (int64_t)(n0 + row) * a.kpad + col * 8);
-        }
-    }
-    for (int i = t; i < HLV * cch; i += NTH) {
-        const int ch = i / HLV, v = i - ch * HLV;
-        const int x = x0 - 1 + v % HLX, y = y0 - 1 + (v / HLX) % HLY, z = z0 - 1 + v / (HLX * HLY);
-        uint4 val = make_uint4(0, 0, 0, 0);
-        if ((unsigned)x < (unsigned)w && (unsigned)y < (unsigned)h && (unsigned)z < (unsigned)d) {
-            const int64_t m = (((int64_t)box * d + z) * h + y) * w + x;
-            val = *(const uint4*)(a.x + m * a.ldx + ch * 8);
-        }
-        halo[i] = val;
-    }
-    __syncthreads();
-
-    f32x4 acc[4][NT];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < NT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // halo voxel of (c16, tile 0, wv); tile i adds i rows.  Only the last step can reach beyond K
-    // (kpad - K < 32), so the others run without a check, each prefetching the next step's table
-    // entry and weight fragments.
-    const int vox = ((zz + 1) * HLY + 4 * yq + 1) * HLX + c16 + 1 - BR_TAB_BIAS;
-    const uint16_t* wrow[NT];
-#pragma unroll
-    for (int j = 0; j < NT; j++) wrow[j] = a.w + (int64_t)(n0 + 16 * j + c16) * a.kpad + g * 8;
-    // weight fragment of column tile j at step s
-    auto wfrag = [&](int j, int s) -> bf16x8 {
-        if constexpr (WL)
-            return *reinterpret_cast<const bf16x8*>(&wl[(16 * j + c16) * WP + 4 * s + g]);
-        else
-            return *(const bf16x8*)(wrow[j] + s * BK);
-    };
-    int tv = tab[g];
-    bf16x8 bfr[NT];
-#pragma unroll
-    for (int j = 0; j < NT; j++) bfr[j] = wfrag(j, 0);
-    for (int s = 0; s + 1 < nsteps; s++) {
-        const int tvn = tab[4 * (s + 1) + g];
-        bf16x8 bn[NT];
-#pragma unroll
-        for (int j = 0; j < NT; j++) bn[j] = wfrag(j, s + 1);
-        const int base = vox + tv;
-        uint4 r[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) r[i] = halo[base + i * HLX];
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int j = 0; j < NT; j++)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(&r[i]), bfr[j],
-                                                                    acc[i][j], 0, 0, 0);
-        tv = tvn;
-#pragma unroll
-        for (int j = 0; j < NT; j++) bfr[j] = bn[j];
-    }
-    {
-        const int base = vox + tv;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            uint4 r = make_uint4(0, 0, 0, 0);
-            if (tv) r = halo[base + i * HLX];
-#pragma unroll
-            for (int j = 0; j < NT; j++)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(&r), bfr[j],
-                                                                    acc[i][j], 0, 0, 0);
-        }
-    }
-
-    const bool relu = a.flags & PVNET_RELU, f32out = a.flags & PVNET_F32OUT;
-#pragma unroll
-    for (int j = 0; j < NT; j++) {
-        const int n = n0 + 16 * j + c16;
-        const float bias = a.bias ? a.bias[n] : 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                // MFMA row 4 g + e: voxel x0 + 4 g + e of row y0 + 4 yq + i in plane z0 + zz
-                const int64_t m = (((int64_t)box * d + z0 + zz) * h + y0 + 4 * yq + i) * w + x0 + 4 * g + e;
-                float v = acc[i][j][e] + bias;
-                if (relu) v = v < 0.f ? 0.f : v;
-                if (a.relu_of && !bf_pos(a.relu_of[m * a.ldr + n])) v = 0.f;
-                if (f32out)
-                    ((float*)a.y)[m * a.ldy + n] = v;
-                else
-                    ((uint16_t*)a.y)[m * a.ldy + n] = f2bf(v);
-            }
-    }
-}
+// 3x3x3 convolutions on the matrix cores, plane by plane
+#include "conv_march.hpp"
 
 // ---------------------------------------------------------------------------------------------
 // weight gradient: block tile BN output channels x 64 k-values, reduction over its voxel chunk in
@@ -1177,63 +1028,14 @@ int pvnet_conv_fwd(const pvnet_conv* c, void* stream) {
     if (M >= (int64_t)1 << 31) return fail(1, "pvnet_conv_fwd: too many voxels");
     hipStream_t st = (hipStream_t)stream;
     const int K = c->ntaps * c->cin;
-    // tiles: 256-voxel blocks for narrow outputs on large grids; 64-channel tiles only when the
-    // grid still has >= 2048 blocks (the K loop is long, so the device needs many blocks in flight)
+    // tiles of the gathering kernel: 256-voxel blocks for narrow outputs on large grids; 64-channel tiles
+    // only when the grid still has >= 2048 blocks (the K loop is long, so the device needs many blocks in
+    // flight)
     const int mt = blocks_for(M, 128);
-    // brick kernel: 16 NT channels per block, NT = cout / 16 up to 4 (48 and 96: NT = 3); bricks of
-    // 16 x 8 x 4 voxels where their halo fits LIM of LDS, else 16 x 4 x 4
-    const size_t tab_bytes = (size_t)(c->kpad / BK) * 4 * sizeof(int);
-    const size_t halo8 = (size_t)hl_vox<8>() * c->cin * 2 + tab_bytes, halo4 = (size_t)hl_vox<4>() * c->cin * 2 + tab_bytes;
-    const int bnt = c->cout % 16 ? 0 : c->cout <= 64 ? c->cout / 16 : c->cout % 48 == 0 ? 3 : c->cout % 64 == 0 ? 4 : 0;
-    const bool bok = bnt && c->ntaps == 27 && !(c->flags & PVNET_GATHER) && c->s.d % BRZ == 0 && c->s.w % BRX == 0 &&
-                     M >= (int64_t)256 * 2048;
-    // the first of (16 x 8 x 4, weights in LDS), (16 x 8 x 4), (16 x 4 x 4, weights in LDS),
-    // (16 x 4 x 4) whose LDS fits LIM: the taller brick first (more waves per CU for the same
-    // LDS), then the weights in LDS (no global load in the k-loop).  A workgroup may take all
-    // 160 KB of a CU's LDS; LIM = 112 KB measured best on the warm-start network's layers (taller
-    // bricks pay even at one block per CU, weights in LDS only while about two blocks fit)
-    const size_t wbytes = (size_t)16 * bnt * (2 * (size_t)c->kpad + 16);
-    const size_t LIM = 112 * 1024;
-    bool by8 = false, wl = false;
-    size_t lds = 0;
-    if (bok && c->s.h % 8 == 0 && halo8 + wbytes <= LIM) {
-        by8 = wl = true;
-        lds = halo8 + wbytes;
-    } else if (bok && c->s.h % 8 == 0 && halo8 <= LIM) {
-        by8 = true;
-        lds = halo8;
-    } else if (bok && c->s.h % 4 == 0 && halo4 + wbytes <= LIM) {
-        wl = true;
-        lds = halo4 + wbytes;
-    } else if (bok && c->s.h % 4 == 0 && halo4 <= LIM) {
-        lds = halo4;
-    }
-    if (lds) {
-        const unsigned nbr = (unsigned)(M / (BRX * (by8 ? 8 : 4) * BRZ));
-        const dim3 gb(nbr, c->cout / (16 * bnt));
-#define PVNET_BRICK(NTV, BYV)                                                                         \
-    do {                                                                                              \
-        if (wl)                                                                                       \
-            hipLaunchKernelGGL((k_conv_fwd_brick<NTV, BYV, true>), gb, dim3(64 * BYV), lds, st, *c, K);  \
-        else                                                                                          \
-            hipLaunchKernelGGL((k_conv_fwd_brick<NTV, BYV, false>), gb, dim3(64 * BYV), lds, st, *c, K); \
-    } while (0)
-        if (by8) {
-            switch (bnt) {
-                case 1: PVNET_BRICK(1, 8); break;
-                case 2: PVNET_BRICK(2, 8); break;
-                case 3: PVNET_BRICK(3, 8); break;
-                default: PVNET_BRICK(4, 8); break;
-            }
-        } else {
-            switch (bnt) {
-                case 1: PVNET_BRICK(1, 4); break;
-                case 2: PVNET_BRICK(2, 4); break;
-                case 3: PVNET_BRICK(3, 4); break;
-                default: PVNET_BRICK(4, 4); break;
-            }
-        }
-#undef PVNET_BRICK
+    MarchPlan mp;
+    if (march_ok(*c) && march_plan(*c, mp)) {
+        const unsigned nblk = (unsigned)mp.ntx * mp.nty * mp.nzs * mp.ng * c->s.nb;
+        hipLaunchKernelGGL(march_kernel(mp), dim3(nblk), dim3(64 * (mp.wx * mp.wn + mp.roll)), mp.lds, st, *c, mp);
     } else if (c->ntaps == 1 && K <= BK && c->cout <= 64 && !(c->flags & PVNET_GATHER)) {
         const dim3 gp((unsigned)((M + 64 * PWT - 1) / (64 * PWT)));
         switch ((c->cout + 15) / 16) {

@@ -508,26 +508,28 @@ inline bool march_search(const MarchKey& c, MarchPlan& best) {
     return best_cost > 0;
 }
 
-// The plan of a shape, kept per thread for the shapes used last (a plan is a pure function of the key).
-inline bool march_plan(const pvnet_conv& c, MarchPlan& p) {
+// The plan of a shape, kept per thread for the shapes used last (a plan is a pure function of its key).
+template <class Plan, class Search>
+bool kept_plan(const MarchKey& key, Plan& p, Search search) {
     struct Slot {
         MarchKey key;
-        MarchPlan plan;
+        Plan plan;
         int ok;  // 0 empty, 1 plan, 2 no plan fits
     };
     constexpr int SLOTS = 128;
     thread_local Slot slots[SLOTS];
-    const MarchKey key{c.s, c.cin, c.cout};
     uint32_t hsh = 2166136261u;
-    for (int32_t v : {c.s.nb, c.s.d, c.s.h, c.s.w, c.cin, c.cout}) hsh = (hsh ^ (uint32_t)v) * 16777619u;
+    for (int32_t v : {key.s.nb, key.s.d, key.s.h, key.s.w, key.cin, key.cout}) hsh = (hsh ^ (uint32_t)v) * 16777619u;
     Slot& sl = slots[(hsh ^ (hsh >> 15)) % SLOTS];
     if (!sl.ok || !(sl.key == key)) {
         sl.key = key;
-        sl.ok = march_search(key, sl.plan) ? 1 : 2;
+        sl.ok = search(key, sl.plan) ? 1 : 2;
     }
     p = sl.plan;
     return sl.ok == 1;
 }
+
+inline bool march_plan(const pvnet_conv& c, MarchPlan& p) { return kept_plan<MarchPlan>(MarchKey{c.s, c.cin, c.cout}, p, march_search); }
 
 // The marching kernels take 3x3x3 convolutions whose outputs (and ReLU mask) can be accessed four channels at a
 // time; PVNET_GATHER keeps k_conv_fwd.

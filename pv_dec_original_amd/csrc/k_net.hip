@@ -247,6 +247,7 @@ __global__ __launch_bounds__(256) void k_conv_pw(pvnet_conv a, int M) {
 // ---------------------------------------------------------------------------------------------
 // 3x3x3 convolutions on the matrix cores, plane by plane
 #include "conv_march.hpp"
+#include "wgrad_march.hpp"
 
 // ---------------------------------------------------------------------------------------------
 // weight gradient: block tile BN output channels x 64 k-values, reduction over its voxel chunk in
@@ -365,192 +366,6 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(pvnet_wgrad a, int M, int K,
             const int n = n0 + j * 16 + g * 4 + e;
             if (n < a.cout) a.ws[((int64_t)split * a.cout + n) * K + kk] = acc[j][e];
         }
-}
-
-// ---------------------------------------------------------------------------------------------
-// weight gradient of a 16- or 32-output 3x3x3 convolution on grids of whole 8 x 8 x 4 bricks.
-// Block `split` reduces a contiguous run of bricks; per brick it stages dy^T once (16 or 32 rows of
-// 256 voxels) and holds its MFMA A fragments (8 per 16 rows, 32 voxels each) in registers for
-// every tap, so that each B fragment feeds one MFMA per 16 output channels, then stages
-// the input one 8-channel group at a time as three channel-major copies, one per x shift dx, of
-// the brick's rows with their z/y halo: X[dx][ci][zh][yh] = the 8 voxels x0 + dx + (0..7) of row
-// (z0 - 1 + zh, y0 - 1 + yh), one 16-byte LDS row.  A B fragment (32 voxels x 16 k-columns) is
-// then one aligned 16-byte read per lane.  A 16-column C tile pairs the taps 2p and 2p + 1 of the
-// group's 8 channels (14 tiles, the last half empty); wave w owns tiles w, w + 4, ...
-//
-// LDS rows are 16 bytes; the 64 banks span 16 rows.  The channel stride of 65 rows (= 1 mod 16)
-// puts the 8 channels a half of a 16-lane group reads on 8 consecutive bank groups, and the copy
-// stride of 520 rows (= 8 mod 16) puts the other half, the next tap's copy, on the other 8; dy^T
-// rows are 33 apart (= 1 mod 16) for the same reason.
-
-constexpr int WBRX = 8, WBRY = 8, WBRZ = 4;  // weight-gradient bricks
-constexpr int WBX_CH = 65;                 // rows per channel (6 x 10 + 5)
-constexpr int WBX_CPY = 8 * WBX_CH;        // rows per dx copy
-constexpr int WBX_ROWS = 3 * WBX_CPY;      // input rows
-constexpr int WBX_ZERO = 40;               // zero rows after them (row offsets within a tile <= 37)
-constexpr int WBD_P = 33;                  // dy^T row pitch in 16-byte rows (256 voxels + 1)
-constexpr int WB_SPLITS = 1024;            // blocks (partial rows) at most along the voxels
-constexpr int WB_NGB = 2;                  // 8-channel groups per block
-
-// column c of the 8x8 bf16 block r (rows = voxels, 16-bit halves = channels): 8 voxels of channel c
-template <int c>
-__device__ __forceinline__ uint4 tcol(const uint4 (&r)[8]) {
-    const uint32_t* rw = reinterpret_cast<const uint32_t*>(r);
-    uint32_t o[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const uint32_t lo = rw[(2 * k) * 4 + (c >> 1)], hi = rw[(2 * k + 1) * 4 + (c >> 1)];
-        o[k] = (c & 1) ? ((lo >> 16) | (hi & 0xffff0000u)) : ((lo & 0xffffu) | (hi << 16));
-    }
-    return make_uint4(o[0], o[1], o[2], o[3]);
-}
-
-template <int c = 0>
-__device__ __forceinline__ void store_cols(const uint4 (&r)[8], uint4* dst, int stride) {
-    if constexpr (c < 8) {
-        dst[c * stride] = tcol<c>(r);
-        store_cols<c + 1>(r, dst, stride);
-    }
-}
-
-// block (split, gy): bricks split * per .. ; channel groups gy * NGB + (0 .. NGB - 1); NR row tiles
-// of 16 output channels (cout = 16 NR).  The grid is one-dimensional, ngy blocks per split: the
-// blocks of one split take consecutive slots of one XCD, so that they walk the same bricks at the
-// same time through one L2 (each reads its own channels of the same input rows).
-//
-// dboff >= 0 (16-output layers): the blocks of the first channel group also sum dy over their
-// bricks for the bias gradient, as one more MFMA per fragment with B = ones in their first wave,
-// into the row ws[dboff + split * cout ..] (the split sums reduce those rows like the weights').
-template <int NGB, int NR>
-__global__ __launch_bounds__(256) void k_conv_wgrad_brick(pvnet_wgrad a, int K, int nbricks, int per, int ngy,
-                                                          int64_t dboff) {
-    // X ends in WBX_ZERO zero rows: the lanes of the empty half of the last tap pair read there
-    __shared__ uint4 X[WBX_ROWS + WBX_ZERO];
-    __shared__ uint4 DY[16 * NR * WBD_P];
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    const int g = lane >> 4, c16 = lane & 15;
-    const int d = a.s.d, h = a.s.h, w = a.s.w;
-    const int nbx = w / WBRX, nby = h / WBRY, nbz = d / WBRZ;
-    const int slot = xcd_tile(blockIdx.x, gridDim.x);
-    const int split = slot / ngy, cg0 = (slot % ngy) * NGB;
-    const int ngrp = min(NGB, a.cin / 8 - cg0);
-    const int b0 = split * per, b1 = min(nbricks, b0 + per);
-
-    f32x4 acc[NGB][4][NR];
-#pragma unroll
-    for (int j = 0; j < NGB; j++)
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int rt = 0; rt < NR; rt++) acc[j][i][rt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const bool dob = NR == 1 && dboff >= 0 && cg0 == 0 && wv == 0;  // wave-uniform
-    f32x4 accb = f32x4{0.f, 0.f, 0.f, 0.f};
-    bf16x8 ones;
-#pragma unroll
-    for (int e = 0; e < 8; e++) ones[e] = (__bf16)1.0f;
-
-    const int cl = c16 & 7;  // this lane's channel within the group; its tap is 2 p + (c16 >> 3)
-    if (t < WBX_ZERO) X[WBX_ROWS + t] = make_uint4(0, 0, 0, 0);  // ordered by the first barrier
-
-    for (int b = b0; b < b1; b++) {
-        int bid = b;
-        const int bx = bid % nbx;
-        bid /= nbx;
-        const int by = bid % nby;
-        bid /= nby;
-        const int bz = bid % nbz;
-        const int64_t box = bid / nbz;
-        const int x0 = bx * WBRX, y0 = by * WBRY, z0 = bz * WBRZ;
-
-        // dy task (row rr, channel chunk nc): dy^T rows n = 8 nc .. 8 nc + 7 at voxels 8 rr ..
-        for (int u = t; u < 64 * NR; u += 256) {
-            const int rr = u / (2 * NR), nc = u % (2 * NR);
-            const int64_t row = ((box * d + z0 + (rr >> 3)) * h + y0 + (rr & 7)) * (int64_t)w + x0;
-            uint4 q[8];
-#pragma unroll
-            for (int i = 0; i < 8; i++) q[i] = *(const uint4*)(a.dy + (row + i) * a.lddy + nc * 8);
-            store_cols(q, DY + nc * 8 * WBD_P + rr, WBD_P);
-        }
-#pragma unroll
-        for (int j = 0; j < NGB; j++) {
-            if (j >= ngrp) break;  // block-uniform
-            const int cg = cg0 + j;
-            if (j > 0) __syncthreads();  // the previous group's reads of X are done
-            if (t < 180) {
-                // input task (dx, zh, yh): 8 voxels x 8 channels, written as 8 channel rows
-                const int dxi = t / 60, zh = (t / 10) % 6, yh = t % 10;
-                const int z = z0 - 1 + zh, y = y0 - 1 + yh;
-                const bool zy = (unsigned)z < (unsigned)d && (unsigned)y < (unsigned)h;
-                const int64_t row = ((box * d + z) * h + y) * (int64_t)w;
-                uint4 r[8];
-#pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    const int x = x0 + i + dxi - 1;
-                    r[i] = make_uint4(0, 0, 0, 0);
-                    if (zy && (unsigned)x < (unsigned)w) r[i] = *(const uint4*)(a.x + (row + x) * a.ldx + cg * 8);
-                }
-                store_cols(r, X + dxi * WBX_CPY + zh * 10 + yh, WBX_CH);
-            }
-            __syncthreads();
-            // A fragments: dy^T[n = 16 rt + c16][voxels 32 s + 8 g .. + 7] of brick row 4 s + g
-            bf16x8 af[NR][8];
-#pragma unroll
-            for (int rt = 0; rt < NR; rt++)
-#pragma unroll
-                for (int s2 = 0; s2 < 8; s2++)
-                    af[rt][s2] = *reinterpret_cast<const bf16x8*>(&DY[(16 * rt + c16) * WBD_P + 4 * s2 + g]);
-            if (NR == 1 && dob && j == 0) {
-                // every column of dy^T x ones is the sum of dy over the brick's voxels
-#pragma unroll
-                for (int s2 = 0; s2 < 8; s2++)
-                    accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[0][s2], ones, accb, 0, 0, 0);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int p = wv + 4 * i;
-                if (p >= 14) break;
-                const int tap = 2 * p + (c16 >> 3);
-                int dz, dy, dx;
-                tap_offset(27, tap < 27 ? tap : 0, dz, dy, dx);
-                const int base = tap < 27 ? (dx + 1) * WBX_CPY + cl * WBX_CH + (1 + dz) * 10 + (1 + dy) : WBX_ROWS;
-#pragma unroll
-                for (int s2 = 0; s2 < 8; s2++) {
-                    const int r = 4 * s2 + g;  // brick row: z = r / 8, y = r % 8
-                    const uint4 v = X[base + (r >> 3) * 10 + (r & 7)];
-#pragma unroll
-                    for (int rt = 0; rt < NR; rt++)
-                        acc[j][i][rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                            af[rt][s2], *reinterpret_cast<const bf16x8*>(&v), acc[j][i][rt], 0, 0, 0);
-                }
-            }
-        }
-        __syncthreads();  // X and DY are restaged for the next brick
-    }
-
-    // D[4 g + e][c16] of row tile rt: n = 16 rt + 4 g + e; column c16 of tile p -> k = tap * cin +
-    // 8 cg + (c16 & 7)
-#pragma unroll
-    for (int j = 0; j < NGB; j++) {
-        if (j >= ngrp) break;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int p = wv + 4 * i;
-            if (p >= 14) break;
-            const int tap = 2 * p + (c16 >> 3);
-            if (tap >= 27) continue;
-            const int k = tap * a.cin + (cg0 + j) * 8 + cl;
-#pragma unroll
-            for (int rt = 0; rt < NR; rt++)
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    a.ws[((int64_t)split * 16 * NR + 16 * rt + 4 * g + e) * K + k] = acc[j][i][rt][e];
-        }
-    }
-    // D[4 g + e][c16] = sum over this block's voxels of dy[.][4 g + e], the same in every column
-    if (dob && c16 == 0) {
-#pragma unroll
-        for (int e = 0; e < 4; e++) a.ws[dboff + (int64_t)split * 16 + 4 * g + e] = accb[e];
-    }
 }
 
 // column sums of dy over a chunk of voxels per block: part[blk][n].  Thread t sums the 8-channel
@@ -958,16 +773,9 @@ int kpad_of(int ntaps, int c) { return (ntaps * c + BK - 1) / BK * BK; }
 struct WgradPlan {
     int ktiles, ntiles, bn, nsplit, mchunk, cblk, cchunk;
     int64_t ws_main, ws_total;
-    bool brick;        // k_conv_wgrad_brick (nsplit blocks of `per` bricks each)
-    int nbricks, per;
+    bool march;  // k_wgrad_march
+    WgradMarch mp;
 };
-
-// the brick kernel takes 16-output 3x3x3 layers with up to 48 input channels on grids of whole
-// bricks; PVNET_GATHER keeps them on k_conv_wgrad
-bool wgrad_brick_ok(const pvnet_shape& s, int ntaps, int cin, int cout) {
-    return ntaps == 27 && (cout == 16 || cout == 32) && cin % 8 == 0 && s.d % WBRZ == 0 && s.h % WBRY == 0 &&
-           s.w % WBRX == 0;
-}
 
 int wgrad_bn(int cout) { return cout <= 16 ? 16 : (cout <= 32 || cout % 64 != 0) ? 32 : 64; }
 
@@ -985,18 +793,15 @@ WgradPlan plan_wgrad(const pvnet_shape& s, int ntaps, int cin, int cout, int fla
     p.mchunk = (int)(per * 128);
     p.nsplit = (int)((M + p.mchunk - 1) / p.mchunk);
     p.ws_main = (int64_t)p.nsplit * cout * K;
-    p.brick = !(flags & PVNET_GATHER) && wgrad_brick_ok(s, ntaps, cin, cout);
-    if (p.brick) {
-        p.nbricks = (int)(M / (WBRX * WBRY * WBRZ));
-        const int ns2 = std::min(p.nbricks, WB_SPLITS);
-        p.per = (p.nbricks + ns2 - 1) / ns2;
-        p.nsplit = (p.nbricks + p.per - 1) / p.per;
+    p.march = ntaps == 27 && !(flags & PVNET_GATHER) && wgrad_march_plan(s, cin, cout, p.mp);
+    if (p.march) {
+        p.nsplit = p.mp.splits;
         p.ws_main = (int64_t)p.nsplit * cout * K;
     }
     p.cchunk = (int)std::max<int64_t>(256, ((M + 1023) / 1024 + 255) & ~(int64_t)255);  // ~1024 blocks
     p.cblk = (int)((M + p.cchunk - 1) / p.cchunk);
-    // the bias rows: one per column-sum block, or one per split when the brick kernel sums them
-    p.ws_total = p.ws_main + (int64_t)std::max(p.cblk, p.brick ? p.nsplit : 0) * cout;
+    // the bias rows: one per column-sum block, or one per split when the marching kernel sums them
+    p.ws_total = p.ws_main + (int64_t)std::max(p.cblk, p.march ? p.nsplit : 0) * cout;
     return p;
 }
 
@@ -1074,30 +879,14 @@ int pvnet_conv_wgrad(const pvnet_wgrad* a, void* stream) {
     const int64_t M = voxels(a->s);
     if (M % 32) return fail(1, "pvnet_conv_wgrad: voxel count must be a multiple of 32");
     if (M >= (int64_t)1 << 31) return fail(1, "pvnet_conv_wgrad: too many voxels");
+    if (a->db && a->cout > 256) return fail(1, "pvnet_conv_wgrad: bias gradient needs cout <= 256");
     hipStream_t st = (hipStream_t)stream;
-    const WgradPlan p = plan_wgrad(a->s, a->ntaps, a->cin, a->cout, a->flags);
+    const WgradPlan p = plan_wgrad(a->s, a->ntaps, a->cin, a->cout, a->flags | (wgrad_march_ok(*a) ? 0 : PVNET_GATHER));
     const int K = a->ntaps * a->cin;
     dim3 grid(p.ktiles, p.ntiles, p.nsplit);
-    int nsplit = p.nsplit;
-    bool fused_db = false;
-    if (p.brick) {
-        // one round of resident blocks along the voxels (at most the plan's WB_SPLITS partial rows)
-        const int ng = a->cin / 8;
-        void (*kern)(pvnet_wgrad, int, int, int, int, int64_t) =
-            a->cout == 32 ? (ng == 1 ? k_conv_wgrad_brick<1, 2> : k_conv_wgrad_brick<WB_NGB, 2>)
-                          : (ng == 1 ? k_conv_wgrad_brick<1, 1> : k_conv_wgrad_brick<WB_NGB, 1>);
-        int dev = 0, cus = 0, occ = 0;
-        NET_HIP(hipGetDevice(&dev));
-        NET_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        NET_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kern, 256, 0));
-        const int gy = ng == 1 ? 1 : (ng + WB_NGB - 1) / WB_NGB;
-        // one round of resident blocks (at most the plan's WB_SPLITS partial rows)
-        const int want = std::max(1, std::min({p.nbricks, WB_SPLITS, std::max(1, cus * occ / gy)}));
-        const int per = (p.nbricks + want - 1) / want;
-        nsplit = (p.nbricks + per - 1) / per;
-        // 16-output layers sum the bias gradient in the same pass (rows after the weight partials)
-        fused_db = a->db && a->cout == 16;
-        hipLaunchKernelGGL(kern, dim3(nsplit * gy), dim3(256), 0, st, *a, K, p.nbricks, per, gy,
+    const bool fused_db = a->db && p.march;  // the bias sums come with the weights'
+    if (p.march) {
+        hipLaunchKernelGGL(wgrad_march_kernel(p.mp), dim3(p.mp.splits * p.mp.ns * p.mp.nf), dim3(256), p.mp.lds, st, *a, p.mp,
                            fused_db ? p.ws_main : (int64_t)-1);
     } else if (p.bn == 16)
         hipLaunchKernelGGL(k_conv_wgrad<16>, grid, dim3(256), 0, st, *a, (int)M, K, p.mchunk);
@@ -1107,15 +896,14 @@ int pvnet_conv_wgrad(const pvnet_wgrad* a, void* stream) {
         hipLaunchKernelGGL(k_conv_wgrad<64>, grid, dim3(256), 0, st, *a, (int)M, K, p.mchunk);
     NET_LAUNCH();
     const int64_t len = (int64_t)a->cout * K;
-    const SumJob jw{a->ws, a->dw, len, (int64_t)K, (int64_t)K, nsplit, (int)blocks_for(len, SUM_COLS)};
+    const SumJob jw{a->ws, a->dw, len, (int64_t)K, (int64_t)K, p.nsplit, (int)blocks_for(len, SUM_COLS)};
     SumJob jb{nullptr, nullptr, 0, 1, 1, 0, 0};
     if (fused_db) {
-        jb = SumJob{a->ws + p.ws_main, a->db, (int64_t)a->cout, (int64_t)a->cout, (int64_t)a->cout, nsplit,
+        jb = SumJob{a->ws + p.ws_main, a->db, (int64_t)a->cout, (int64_t)a->cout, (int64_t)a->cout, p.nsplit,
                     (int)blocks_for(a->cout, SUM_COLS)};
     } else if (a->db) {
         // the bias column sums read only dy: they run before the split sums, whose launch then
         // reduces the weight and the bias partials together
-        if (a->cout > 256 || a->cout % 8) return fail(1, "pvnet_conv_wgrad: bias gradient needs cout <= 256, a multiple of 8");
         float* part = a->ws + p.ws_main;
         hipLaunchKernelGGL(k_colsum, dim3(p.cblk), dim3(256), 0, st, a->dy, a->lddy, a->cout, (int)M, p.cchunk, part);
         NET_LAUNCH();

@@ -1,0 +1,250 @@
+// wgrad_march.hpp — weight gradients of 3x3x3 convolutions that march through z (gfx950).
+//
+//   dw[n][tap][ci] = sum over voxels m of dy[m][n] x[m + off(tap)][ci]
+//
+// The reduction index is the voxel.  A block walks runs of planes of a tx x ty tile with the planes of both
+// tensors copied straight into LDS, channels innermost as in memory, and reads the MFMA operands (eight
+// voxels of one channel per lane) with the transposing LDS read, so nothing is transposed in registers.  The
+// tensor with the fewer channels per block is the one that is shifted by the taps:
+//   sum_m dy[m] x[m + off] = sum_m' dy[m' - off] x[m'],
+// so a block takes 16 output channels of dy (planes z-1 .. z+1 with a halo) against 16 CF input channels of x
+// (its own voxels only), and a wave reads CF + 7 fragments for 7 CF MFMAs.  Wave v owns the shifts v, v + 4, ..
+// (7 of them; the 28th is a repeat that is not written), so every sum is complete within its wave.  Blocks are
+// splits of the voxels, summed by k_sum_splits.  The bias gradient is one more MFMA per dy fragment of the
+// centre tap, with ones for x.
+//
+// What bounds it: at CF = 1 the LDS (8 KB of fragments for 7 MFMAs), at CF = 3 the matrix cores and the LDS
+// alike.  Measured against the kernels it replaces (register transposes, one LDS copy of x per x shift or a
+// gather per tap; split sums included), us per call, batch x grid, channels in -> out: 8 x 96^3 48->16
+// 1032 -> 307, 16->16 346 -> 172, 8->16 200 -> 172; 8 x 48^3 96->32 301 -> 163, 32->32 114 -> 80;
+// 8 x 24^3 224->64 339 -> 127, 64->64 115 -> 55; 8 x 12^3 160->160 111 -> 62; 3 x 20 x 18 x 28 64->160 92 -> 50.
+#pragma once
+
+struct WgradMarch {
+    int32_t tx, ty, ntx, nty;   // tile (divides the plane) and tiles per plane
+    int32_t zseg, nzs;          // planes per run, runs per box
+    int32_t hx, hp, gr;         // halo row pitch and size; 32-voxel groups of a tile
+    int32_t su, fu;             // LDS units (16 bytes) of one dy and one x plane
+    int32_t cf, ns, nf;         // 16-channel tiles of x per block; blocks over the channels of dy and x
+    int32_t units, per, splits; // runs in all, runs per block, blocks over the voxels
+    int32_t lds;
+};
+
+typedef short tr4 __attribute__((ext_vector_type(4)));
+
+// 4 voxels (rows of 16 channels, 32 bytes apart) x this lane's channel: lane 16 q + c of the wave addresses
+// row 4 q + c / 4, channels 4 (c % 4) .. + 3, and receives channel c of rows 4 q .. 4 q + 3
+__device__ __forceinline__ uint2 tr_read(const char* lds) {
+    const tr4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) tr4*)(uintptr_t)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)lds);
+    return *reinterpret_cast<const uint2*>(&v);
+}
+
+template <int CF>
+__global__ __launch_bounds__(256, 3) void k_wgrad_march(const pvnet_wgrad a, const WgradMarch p, const int64_t dboff) {
+    extern __shared__ uint4 wm_sm[];
+    const int t = threadIdx.x, lane = t & 63, g = lane >> 4, c16 = lane & 15;
+    const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int d = a.s.d, h = a.s.h, w = a.s.w, K = 27 * a.cin;
+    const int slot = xcd_tile(blockIdx.x, gridDim.x);
+    const int split = slot / (p.ns * p.nf), r0 = slot - split * (p.ns * p.nf);
+    const int s0 = (r0 % p.ns) * 16, f0 = (r0 / p.ns) * 16 * CF;  // first channel of dy, of x
+    const int vox = p.tx * p.ty, sl32 = p.gr * 32, nuS = 2 * p.hp, nuF = 2 * CF * sl32;
+    uint4* Fs = wm_sm + 4 * p.su;
+    int* vtab = reinterpret_cast<int*>(Fs + 2 * p.fu);
+    int *soS = vtab + sl32, *soF = soS + nuS;
+    const uint32_t ldsS = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint4*)wm_sm, ldsF = ldsS + 16u * 4u * (uint32_t)p.su;
+    const char* smS = reinterpret_cast<const char*>(wm_sm);
+    const char* smF = reinterpret_cast<const char*>(Fs);
+
+    // slot -> byte offset of its own voxel in a dy plane (slots beyond the tile: the first voxel's)
+    for (int i = t; i < sl32; i += 256) {
+        const int v = i < vox ? i : 0, y = v / p.tx, x = v - y * p.tx;
+        vtab[i] = 32 * ((y + 1) * p.hx + x + 1);
+    }
+
+    f32x4 acc[7][CF];
+#pragma unroll
+    for (int i = 0; i < 7; i++)
+#pragma unroll
+        for (int f = 0; f < CF; f++) acc[i][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // the bias gradient: wave 1 (it owns the centre tap), in the blocks of the first x channels
+    const bool dob = dboff >= 0 && wv == 1 && f0 == 0;
+    f32x4 accb = f32x4{0.f, 0.f, 0.f, 0.f};
+    bf16x8 ones;
+#pragma unroll
+    for (int e = 0; e < 8; e++) ones[e] = (__bf16)1.0f;
+
+    const int rowv = 4 * g + (c16 >> 2), colb = (c16 & 3) * 8;  // this lane's row within 16 voxels, byte column
+    const int u1 = min(p.units, (split + 1) * p.per);
+    for (int u = split * p.per; u < u1; u++) {
+        int r = u;
+        const int zq = r % p.nzs;
+        r /= p.nzs;
+        const int x0 = (r % p.ntx) * p.tx;
+        r /= p.ntx;
+        const int y0 = (r % p.nty) * p.ty;
+        const int64_t box = r / p.nty;
+        const int z0 = zq * p.zseg, z1 = min(d, z0 + p.zseg);
+        __syncthreads();  // the previous run is done with the LDS
+        // element offset of every unit within its plane (-1: zero)
+        for (int i = t; i < nuS; i += 256) {
+            const int v = i >> 1, ch = s0 + 8 * (i & 1);
+            const int hy = v / p.hx, x = x0 - 1 + v - hy * p.hx, y = y0 - 1 + hy;
+            soS[i] = (unsigned)x < (unsigned)w && (unsigned)y < (unsigned)h && ch < a.cout ? (y * w + x) * a.lddy + ch : -1;
+        }
+        for (int i = t; i < nuF; i += 256) {
+            const int cp = i / (2 * sl32), q = i - cp * 2 * sl32, v = q >> 1, ch = f0 + 16 * cp + 8 * (q & 1);
+            const int yy = v / p.tx;
+            soF[i] = v < vox && ch < a.cin ? ((y0 + yy) * w + x0 + v - yy * p.tx) * a.ldx + ch : -1;
+        }
+        __syncthreads();
+        auto stage = [&](const uint16_t* base, int ld, int z, const int* so, int nu, uint32_t lds) {
+            const bool zin = (unsigned)z < (unsigned)d;
+            const uint16_t* pb = base + (box * d + (zin ? z : 0)) * ((int64_t)h * w) * ld;
+            for (int i = 64 * wv; i < nu; i += 256)
+                if (i + lane < nu) {
+                    const int o = so[i + lane];
+                    lds_copy16(zin && o >= 0 ? (const void*)(pb + o) : (const void*)g_march_zero,
+                               __builtin_amdgcn_readfirstlane(lds + 16u * (uint32_t)i));
+                }
+        };
+        for (int z = z0 - 1; z <= z0 + 1; z++) stage(a.dy, a.lddy, z, soS, nuS, ldsS + 16u * (uint32_t)((z & 3) * p.su));
+        stage(a.x, a.ldx, z0, soF, nuF, ldsF + 16u * (uint32_t)((z0 & 1) * p.fu));
+        march_wait();
+        march_barrier();
+        for (int z = z0; z < z1; z++) {
+            if (z + 1 < z1) {
+                stage(a.dy, a.lddy, z + 2, soS, nuS, ldsS + 16u * (uint32_t)(((z + 2) & 3) * p.su));
+                stage(a.x, a.ldx, z + 1, soF, nuF, ldsF + 16u * (uint32_t)(((z + 1) & 1) * p.fu));
+            }
+            int toff[7];  // byte offset of each shift from a voxel's own unit, wave-uniform
+#pragma unroll
+            for (int i = 0; i < 7; i++) {
+                const int s = min(wv + 4 * i, 26);
+                const int dz = s / 9, dy = s / 3 % 3, dx = s % 3;
+                toff[i] = 16 * (((z + dz - 1) & 3) * p.su) + 32 * ((dy - 1) * p.hx + dx - 1);
+            }
+            const char* fb = smF + 16 * ((z & 1) * p.fu) + 32 * rowv + colb;
+            auto group = [&](int q, bool part) {
+                const int v0 = vtab[32 * q + rowv] + colb, v1 = vtab[32 * q + 16 + rowv] + colb;
+                // in the tile's last group, elements beyond the tile are zero in both operands
+                uint2 m0 = make_uint2(~0u, ~0u), m1 = m0;
+                if (part) {
+                    auto keep = [&](int n) {
+                        return make_uint2(n >= 2 ? ~0u : n == 1 ? 0xffffu : 0u, n >= 4 ? ~0u : n == 3 ? 0xffffu : 0u);
+                    };
+                    m0 = keep(vox - (32 * q + 4 * g));
+                    m1 = keep(vox - (32 * q + 16 + 4 * g));
+                }
+                uint4 fr[CF];
+#pragma unroll
+                for (int f = 0; f < CF; f++) {
+                    const char* pf = fb + 32 * (f * sl32 + 32 * q);
+                    const uint2 lo = tr_read(pf), hi = tr_read(pf + 512);
+                    fr[f] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+                }
+#pragma unroll
+                for (int i = 0; i < 7; i++) {
+                    uint2 lo = tr_read(smS + toff[i] + v0), hi = tr_read(smS + toff[i] + v1);
+                    if (part) {
+                        lo.x &= m0.x, lo.y &= m0.y;
+                        hi.x &= m1.x, hi.y &= m1.y;
+                    }
+                    const uint4 sv = make_uint4(lo.x, lo.y, hi.x, hi.y);
+                    const bf16x8 sb = *reinterpret_cast<const bf16x8*>(&sv);
+#pragma unroll
+                    for (int f = 0; f < CF; f++)
+                        acc[i][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sb, *reinterpret_cast<const bf16x8*>(&fr[f]), acc[i][f], 0, 0, 0);
+                    if (i == 3 && dob) accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sb, ones, accb, 0, 0, 0);
+                }
+            };
+            const int whole = vox >> 5;
+            for (int q = 0; q < whole; q++) group(q, false);
+            if (whole < p.gr) group(whole, true);
+            march_wait();
+            if (z + 1 < z1) march_barrier();
+        }
+    }
+
+    // D[4 g + e][c16] of a tile pair: channel 4 g + e of dy, channel c16 of x; shift s is tap 26 - s
+#pragma unroll
+    for (int i = 0; i < 7; i++) {
+        const int tap = 26 - (wv + 4 * i);
+        if (tap < 0) continue;
+#pragma unroll
+        for (int f = 0; f < CF; f++) {
+            const int n = s0 + 4 * g, ci = f0 + 16 * f + c16;
+            if (ci >= a.cin) continue;
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (n + e < a.cout) a.ws[((int64_t)split * a.cout + n + e) * K + tap * a.cin + ci] = acc[i][f][e];
+        }
+    }
+    if (dob && c16 == 0)  // every column holds the sum of channel 4 g + e
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (s0 + 4 * g + e < a.cout) a.ws[dboff + (int64_t)split * a.cout + s0 + 4 * g + e] = accb[e];
+}
+
+typedef void (*WgradKernel)(const pvnet_wgrad, const WgradMarch, const int64_t);
+
+inline WgradKernel wgrad_march_kernel(const WgradMarch& p) {
+    return p.cf == 1 ? k_wgrad_march<1> : p.cf == 2 ? k_wgrad_march<2> : k_wgrad_march<3>;
+}
+
+// The plan of a weight gradient, from the sizes alone (the scratch size a caller asks for and the launch agree on
+// any device).  Tiles divide the plane, so that no operand needs masking inside a plane.  Every tile, run length
+// and CF that fits is priced as conv_march prices its plans: a block alone on its CU against the share of the
+// matrix cores, LDS and copies when cc blocks share it, plus the split partials' traffic; constants in clocks,
+// fitted to 22,000 timed plans of 18 layers.  The plan taken is 4% (mean) and at most 29% slower than the best
+// one timed over those.
+inline bool wgrad_march_search(const pvnet_shape& s, int cin, int cout, WgradMarch& best) {
+    constexpr int WANT = 768;  // blocks: three per CU
+    double best_cost = 0;
+    static const int cuts[] = {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32, 48};
+    const int ft = (cin + 15) / 16, st = (cout + 15) / 16;
+    for (int tx = 1; tx <= 256 && tx <= s.w; tx++) {
+        if (s.w % tx) continue;
+        for (int ty = 1; ty <= 64 && ty <= s.h; ty++) {
+            const int vox = tx * ty, gr = (vox + 31) / 32, hp = (tx + 2) * (ty + 2);
+            if (s.h % ty || vox > 512 || (vox < 32 && vox < s.w * s.h && tx < s.w)) continue;
+            for (int cf = 1; cf <= 3 && cf <= ft; cf++) {
+                const int su = (2 * hp + 63) / 64 * 64, fu = (2 * cf * gr * 32 + 63) / 64 * 64;
+                const int lds = 16 * (4 * su + 2 * fu) + 4 * (gr * 32 + 2 * hp + 2 * cf * gr * 32);
+                if (lds > 160 * 1024) continue;
+                const int nf = (ft + cf - 1) / cf;
+                const double c = std::max(1, std::min(160 * 1024 / lds, cf == 3 ? 3 : cf == 2 ? 4 : 6));
+                for (int cut : cuts) {
+                    if (cut > s.d) break;
+                    const int zseg = (s.d + cut - 1) / cut, nzs = (s.d + zseg - 1) / zseg;
+                    const int64_t units = (int64_t)s.nb * (s.w / tx) * (s.h / ty) * nzs;
+                    const int want = (int)std::max<int64_t>(1, std::min<int64_t>(units, WANT / (nf * st)));
+                    const int per = (int)((units + want - 1) / want), splits = (int)((units + per - 1) / per);
+                    const double B = (double)splits * nf * st, za = (double)s.d / nzs;
+                    const double lat = per * (4400 + 6.9 * hp + 830 * (za + 2) + za * gr * (500 + 168.0 * cf));
+                    const double thr = per * za * (gr * std::max(112.0 * cf, 32.6 * (7 + cf)) + 0.81 * (hp + cf * gr * 32));
+                    const double cc = std::min(c, std::ceil(B / 256));
+                    const double cost = (std::max(lat, thr * cc) + 0.36 * (lat + thr * cc)) * std::ceil(B / (256 * c)) +
+                                        0.2 * splits * cout * cin;
+                    if (best_cost == 0 || cost < best_cost) {
+                        best_cost = cost;
+                        best = WgradMarch{tx, ty, s.w / tx, s.h / ty, zseg, nzs, tx + 2, hp, gr, su, fu, cf, st, nf, (int)units, per, splits, lds};
+                    }
+                }
+            }
+        }
+    }
+    return best_cost > 0;
+}
+
+inline bool wgrad_march_plan(const pvnet_shape& s, int cin, int cout, WgradMarch& p) {
+    return kept_plan<WgradMarch>(MarchKey{s, cin, cout}, p, [](const MarchKey& k, WgradMarch& q) {
+        return (int64_t)k.s.nb * k.s.d * k.s.h * k.s.w < (int64_t)1 << 31 && wgrad_march_search(k.s, k.cin, k.cout, q);
+    });
+}
+
+// What one call needs beyond a plan: plane offsets fit 32 bits (as in conv_march, PVNET_GATHER and pointwise
+// layers stay on k_conv_wgrad)
+inline bool wgrad_march_ok(const pvnet_wgrad& a) {
+    return (int64_t)a.s.h * a.s.w * std::max(a.ldx, a.lddy) < (int64_t)1 << 31;
+}

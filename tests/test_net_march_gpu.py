@@ -54,3 +54,53 @@ def test_march_equals_gather(case):
     rest = out[0].clone()
     rest[:, yoff:yoff + cout] = 7.0
     assert bool((rest == 7.0).all()), "wrote outside the output slice"
+
+
+WGRAD = [
+    # shape, cin, cout, x slice (ldx, offset), dy slice (lddy, offset)
+    ((1, 1, 4, 8), 8, 8, 8, 0, 8, 0),         # one plane, one 32-voxel group
+    ((2, 3, 4, 4), 16, 16, 24, 8, 32, 16),    # half a group per tile, slices
+    ((1, 32, 5, 7), 24, 40, 24, 0, 40, 0),    # odd plane, partial channel tiles
+    ((4, 8, 37, 31), 32, 24, 32, 0, 24, 0),   # prime plane sizes: rows are the tiles
+    ((3, 7, 16, 10), 48, 16, 48, 0, 16, 0),   # three x tiles per block
+    ((1, 9, 12, 40), 64, 160, 64, 0, 160, 0),
+    ((1, 4, 8, 64), 224, 72, 224, 0, 72, 0),
+    ((1, 64, 1, 2), 8, 16, 8, 0, 16, 0),      # two voxels per plane
+]
+
+
+@pytest.mark.parametrize("case", WGRAD, ids=[f"w{i}" for i in range(len(WGRAD))])
+def test_wgrad_march_sums(case):
+    """Against 64-bit products of the same bf16 operands.  A sum of M FP32 products, each rounded to 2^-24 of
+    the running sum, strays by at most M 2^-24 of the sum of magnitudes; with at most 36,704 voxels and partial
+    sums far shorter than M that is below 1e-4 of the largest sum of magnitudes, and 1e-5 of the result's norm."""
+    import torch
+    from pv_dec_original_amd import _native as N
+    shape, cin, cout, ldx, xoff, lddy, doff = case
+    nb, d, h, w = shape
+    m = int(np.prod(shape))
+    g = torch.Generator(device="cuda")
+    g.manual_seed(11)
+    x = torch.randn((m, ldx), generator=g, device="cuda").to(torch.bfloat16)
+    dy = torch.randn((m, lddy), generator=g, device="cuda").to(torch.bfloat16)
+    sh = N.NetShape(*shape)
+    ws = torch.full((int(N.net().pvnet_wgrad_ws_floats(C.byref(sh), 27, cin, cout)),), 9.0, device="cuda")
+    st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    got = []
+    for _ in range(2):
+        dw = torch.zeros((cout, 27 * cin), device="cuda")
+        db = torch.zeros(cout, device="cuda")
+        q = N.NetWgrad(sh, 27, cin, cout, C.c_void_p(x.data_ptr() + 2 * xoff), ldx, lddy,
+                       C.c_void_p(dy.data_ptr() + 2 * doff), C.c_void_p(ws.data_ptr()), C.c_void_p(dw.data_ptr()),
+                       C.c_void_p(db.data_ptr()))
+        N.net_check(N.net().pvnet_conv_wgrad(C.byref(q), st))
+        got.append((dw, db))
+    torch.cuda.synchronize()
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), "not deterministic"
+    xd = x[:, xoff:xoff + cin].double().reshape(nb, d, h, w, cin)
+    gd = dy[:, doff:doff + cout].double()
+    pad = torch.nn.functional.pad(xd, (0, 0, 1, 1, 1, 1, 1, 1))
+    ref = torch.stack([gd.t().contiguous() @ pad[:, a:a + d, b:b + h, e:e + w].reshape(m, cin)
+                       for a in range(3) for b in range(3) for e in range(3)], dim=1).reshape(cout, 27 * cin)
+    assert float((got[0][0] - ref).norm() / ref.norm()) < 1e-5
+    assert float((got[0][1] - gd.sum(0)).norm() / gd.sum(0).norm()) < 1e-5

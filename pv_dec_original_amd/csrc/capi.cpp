@@ -131,6 +131,7 @@ struct pvlbm_sim {
     double* d_macro = nullptr;
     double* d_partials = nullptr;
     double* d_red = nullptr;
+    double* d_expand = nullptr;  // scratch of a start from a coarse field, allocated by the first one
     unsigned long long* d_gate = nullptr;
     // host copy of the triangles (link fractions), boundary slots (padded node, closure)
     std::vector<double> tri;
@@ -188,7 +189,7 @@ struct pvlbm_sim {
     ~pvlbm_sim() {
         if (stream) (void)hipStreamSynchronize(stream);
         void* ptrs[] = {d_bq, d_kind, d_aux, d_tdesc, d_pop[0], d_pop[1], d_bmask, d_bclose, d_bprof, d_brho,
-                        d_M, d_nrm, d_wss, d_tau3, d_acc, d_macro, d_partials, d_red, d_gate};
+                        d_M, d_nrm, d_wss, d_tau3, d_acc, d_macro, d_partials, d_red, d_expand, d_gate};
         for (void* p : ptrs) dfree(p);
         if (ev0) (void)hipEventDestroy(ev0);
         if (ev1) (void)hipEventDestroy(ev1);
@@ -246,6 +247,11 @@ struct pvlbm_sim {
         d_pop[1] = dalloc<char>(pop_bytes);
         HIPCHK(hipMemsetAsync(d_pop[1], 0, pop_bytes, stream));
         B = (A == d_pop[0]) ? d_pop[1] : d_pop[0];
+    }
+
+    double* ensure_expand() {
+        if (!d_expand) d_expand = dalloc<double>((size_t)expand_coarse_doubles(nx, nxp, ntiles));
+        return d_expand;
     }
 
     // Brings the state into the layout of the scheme in use (values only move: fields unchanged).
@@ -1050,37 +1056,31 @@ extern "C" int pvlbm_init_fields_coarse(pvlbm_handle h, const float* rho_c, cons
         // the coarse fields are the caller's device memory, possibly still being written on the
         // caller's stream: wait for all work on the device before this handle's stream reads them
         HIPCHK(hipDeviceSynchronize());
-        double* d_in = nullptr;
-        unsigned long long* d_cnt = nullptr;
+        // the fields go through the macro planes, node by node: the first collision reads a node's initial
+        // state there and writes its density and velocity back.  Scratch, kept with the handle: nx each of
+        // plane fluxes, targets, density offsets, then the flag and the count, then the flux partials.
+        double* d = h->ensure_expand();
+        double *d_tgt = d + h->nx, *d_drho = d_tgt + h->nx, *d_cnt = d_drho + h->nx;
         try {
-            // [4][ns] fields, then nx each: plane flux scratch, flux targets, density offsets
-            d_in = dalloc<double>((size_t)(4 * h->ns + 3 * h->nx));
-            d_cnt = dalloc<unsigned long long>(1);
-            double* d_tgt = d_in + 4 * h->ns + h->nx;
-            double* d_drho = d_tgt + h->nx;
             if (plane_flux)
                 HIPCHK(hipMemcpyAsync(d_tgt, plane_flux, sizeof(double) * h->nx, hipMemcpyHostToDevice, h->stream));
             if (plane_drho)
                 HIPCHK(hipMemcpyAsync(d_drho, plane_drho, sizeof(double) * h->nx, hipMemcpyHostToDevice, h->stream));
-            HIPCHK(hipMemsetAsync(d_cnt, 0, sizeof(unsigned long long), h->stream));
-            HIPCHK(launch_expand_coarse(rho_c, u_c, cdims[0], cdims[1], cdims[2], h->nx, h->ny, h->nz, h->nxp,
-                                        h->nyp, h->ns, umax, rho_lo, rho_hi, h->d_kind, flux_x,
-                                        plane_flux ? d_tgt : nullptr, plane_drho ? d_drho : nullptr,
-                                        d_in + 4 * h->ns, d_in, d_cnt, h->stream));
+            HIPCHK(hipMemsetAsync(d_cnt, 0, 2 * sizeof(double), h->stream));
+            HIPCHK(launch_expand_coarse(rho_c, u_c, cdims[0], cdims[1], cdims[2], h->nx, h->ny, h->nz, h->nxp, h->nyp, h->ns,
+                                        h->d_tdesc, h->ntiles, umax, rho_lo, rho_hi, flux_x, plane_flux ? d_tgt : nullptr,
+                                        plane_drho ? d_drho : nullptr, d, d_cnt + 2, reinterpret_cast<int*>(d_cnt),
+                                        h->d_macro, reinterpret_cast<unsigned long long*>(d_cnt + 1), h->stream));
             h->reset_state();
-            h->launch(F_INIT | F_MACRO | F_REDUCE, 1.0, d_in, d_in + h->ns);
+            h->launch(F_INIT | F_MACRO | F_REDUCE, 1.0, h->d_macro, h->d_macro + h->ns);
             unsigned long long cnt = 0;
-            HIPCHK(hipMemcpyAsync(&cnt, d_cnt, sizeof(cnt), hipMemcpyDeviceToHost, h->stream));
+            HIPCHK(hipMemcpyAsync(&cnt, d_cnt + 1, sizeof(cnt), hipMemcpyDeviceToHost, h->stream));
             HIPCHK(hipStreamSynchronize(h->stream));
             if (nonfinite) *nonfinite = (int64_t)cnt;
         } catch (...) {
             (void)hipStreamSynchronize(h->stream);
-            dfree(d_in);
-            dfree(d_cnt);
             throw;
         }
-        dfree(d_in);
-        dfree(d_cnt);
     });
 }
 

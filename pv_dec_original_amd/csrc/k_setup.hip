@@ -364,75 +364,138 @@ __device__ __forceinline__ float coarse_coord(int64_t i, int64_t n, int c, int& 
     return x - (float)i0;
 }
 
-__global__ void k_expand_coarse(const float* rho_c, const float* u_c, int cx, int cy, int cz, int64_t nx,
-                                int64_t ny, int64_t nz, int64_t nxp, int64_t nyp, int64_t ns, double rlo,
-                                double rhi, double* out, unsigned long long* nonfin) {
-    const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= ns) return;
-    const int64_t x = n % nxp, pr = n / nxp, y = pr % nyp, z = pr / nyp;
-    double r = 1.0, u0 = 0.0, u1 = 0.0, u2 = 0.0;
-    if (x < nx && y < ny && z < nz) {
-        int x0, x1, y0, y1, z0, z1;
-        const float fx = coarse_coord(x, nx, cx, x0, x1);
-        const float fy = coarse_coord(y, ny, cy, y0, y1);
-        const float fz = coarse_coord(z, nz, cz, z0, z1);
-        const int64_t plane = (int64_t)cx * cy * cz;
+// The field is expanded at the nodes alone, tile by tile, into the macro planes the handle already holds, and the
+// plane fluxes come from a first pass that samples u_x again instead of storing it.  On the 1024 x 512 x 512
+// aneurysm (6.45 M nodes of 268 M points, 192 x 96 x 96 coarse) the fluxes take 89 + 21 us and the fields 83 us.
+// Filling four FP64 planes of the whole box in a buffer of its own instead took 5.5 ms, and allocating and
+// freeing that buffer (9.2 GB) up to 250 ms a call.
+// Trilinear sample of the coarse field at box point (x, y, z): rho and u in FP32, false if not finite.
+struct CoarseField {
+    const float* rho;
+    const float* u;
+    int cx, cy, cz;
+    int64_t nx, ny, nz;
+};
+
+template <int C0, int C1>
+__device__ __forceinline__ void coarse_sample(const CoarseField& F, int64_t x, int64_t y, int64_t z, float (&v)[4]) {
+    int x0, x1, y0, y1, z0, z1;
+    const float fx = coarse_coord(x, F.nx, F.cx, x0, x1);
+    const float fy = coarse_coord(y, F.ny, F.cy, y0, y1);
+    const float fz = coarse_coord(z, F.nz, F.cz, z0, z1);
+    const int64_t plane = (int64_t)F.cx * F.cy * F.cz;
+#pragma unroll
+    for (int c = C0; c < C1; c++) {
+        const float* f = c == 0 ? F.rho : F.u + (c - 1) * plane;
+        auto at = [&](int zz, int yy, int xx) { return f[((int64_t)zz * F.cy + yy) * F.cx + xx]; };
+        const float a = at(z0, y0, x0) * (1.f - fx) + at(z0, y0, x1) * fx;
+        const float b = at(z0, y1, x0) * (1.f - fx) + at(z0, y1, x1) * fx;
+        const float cc = at(z1, y0, x0) * (1.f - fx) + at(z1, y0, x1) * fx;
+        const float d = at(z1, y1, x0) * (1.f - fx) + at(z1, y1, x1) * fx;
+        v[c] = (a * (1.f - fy) + b * fy) * (1.f - fz) + (cc * (1.f - fy) + d * fy) * fz;
+    }
+}
+
+__device__ __forceinline__ bool finite4(const float (&v)[4]) {
+    return isfinite(v[0]) && isfinite(v[1]) && isfinite(v[2]) && isfinite(v[3]);
+}
+
+// *flag = 1 if a coarse value is not finite or so large that a blend of finite values might not be: only
+// then can a sample be non-finite
+__global__ void k_coarse_suspect(const float* rho_c, const float* u_c, int64_t n, int* flag) {
+    bool bad = false;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < 4 * n; i += (int64_t)gridDim.x * blockDim.x) {
+        const float v = i < n ? rho_c[i] : u_c[i - n];
+        bad |= !(fabsf(v) < 1e38f);
+    }
+    if (bad) *flag = 1;
+}
+
+// the number of box points whose sample is not finite (none unless the flag is set)
+__global__ __launch_bounds__(256) void k_coarse_count(const CoarseField F, const int* flag, unsigned long long* nonfin) {
+    if (!*flag) return;
+    const int64_t n = F.nx * F.ny * F.nz;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        const int64_t r = i / F.nx;
         float v[4];
-        for (int c = 0; c < 4; c++) {
-            const float* f = c == 0 ? rho_c : u_c + (c - 1) * plane;
-            auto at = [&](int zz, int yy, int xx) { return f[((int64_t)zz * cy + yy) * cx + xx]; };
-            const float a = at(z0, y0, x0) * (1.f - fx) + at(z0, y0, x1) * fx;
-            const float b = at(z0, y1, x0) * (1.f - fx) + at(z0, y1, x1) * fx;
-            const float cc = at(z1, y0, x0) * (1.f - fx) + at(z1, y0, x1) * fx;
-            const float d = at(z1, y1, x0) * (1.f - fx) + at(z1, y1, x1) * fx;
-            v[c] = (a * (1.f - fy) + b * fy) * (1.f - fz) + (cc * (1.f - fy) + d * fy) * fz;
-        }
-        if (isfinite(v[0]) && isfinite(v[1]) && isfinite(v[2]) && isfinite(v[3])) {
-            r = fmin(fmax((double)v[0], rlo), rhi);
-            u0 = v[1];
-            u1 = v[2];
-            u2 = v[3];
-        } else {
-            atomicAdd(nonfin, 1ull);
-        }
+        coarse_sample<0, 4>(F, i % F.nx, r % F.ny, r / F.ny, v);
+        if (!finite4(v)) atomicAdd(nonfin, 1ull);
     }
-    out[n] = r;
-    out[ns + n] = u0;
-    out[2 * ns + n] = u1;
-    out[3 * ns + n] = u2;
 }
 
-// flux of u_x through each plane x over the fluid nodes: one block per plane, fixed-order sums
-__global__ __launch_bounds__(256) void k_slab_flux(const double* ux, const uint8_t* kind, int64_t ny, int64_t nz,
-                                                   int64_t nxp, int64_t nyp, double* flux) {
-    __shared__ double sh[256];
-    const int64_t x = blockIdx.x;
-    double sum = 0.0;
-    for (int64_t r = threadIdx.x; r < ny * nz; r += 256) {
-        const int64_t n = x + nxp * ((r % ny) + nyp * (r / ny));
-        if (kind[n] != 0) sum += ux[n];
-    }
-    sh[threadIdx.x] = sum;
+// Flux of u_x through each plane x over the nodes: a block walks a run of tiles, each wave adding its tiles'
+// samples into its own LDS row of XR tile columns (blockIdx.y picks them) in tile order, and writes the sum of
+// its waves' rows; k_flux_final adds the blocks.  Fixed order throughout.  Sampling u_x twice (here and in
+// k_expand_nodes) costs less than writing and re-reading the field would.
+constexpr int FLUX_XR = 16, FLUX_BLOCKS = 512;
+
+__global__ __launch_bounds__(256) void k_flux_nodes(const CoarseField F, int64_t nxp, int64_t nyp, const TileDesc* tdesc,
+                                                    int ntiles, double* part) {
+    __shared__ double sh[4][FLUX_XR * 64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    for (int i = threadIdx.x; i < 4 * FLUX_XR * 64; i += 256) (&sh[0][0])[i] = 0.0;
     __syncthreads();
-    for (int st = 128; st > 0; st >>= 1) {
-        if ((int)threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
-        __syncthreads();
+    const int nxt = (int)(nxp / 64), xt0 = blockIdx.y * FLUX_XR;
+    const int per = (ntiles + gridDim.x - 1) / gridDim.x, t1 = min(ntiles, ((int)blockIdx.x + 1) * per);
+    for (int t = blockIdx.x * per + wv; t < t1; t += 4) {
+        const int tile = tdesc[t].tile, row = tile / nxt, xt = tile - row * nxt;
+        if (xt < xt0 || xt >= xt0 + FLUX_XR || !((tdesc[t].node >> lane) & 1ull)) continue;
+        float v[4];
+        coarse_sample<0, 4>(F, 64 * xt + lane, row % (int)nyp, row / (int)nyp, v);
+        if (finite4(v)) sh[wv][64 * (xt - xt0) + lane] += (double)v[1];
     }
-    if (threadIdx.x == 0) flux[x] = sh[0];
+    __syncthreads();
+    for (int i = threadIdx.x; i < FLUX_XR * 64; i += 256) {
+        const int64_t x = 64ll * xt0 + i;
+        if (x < nxp) part[blockIdx.x * nxp + x] = ((sh[0][i] + sh[1][i]) + sh[2][i]) + sh[3][i];
+    }
 }
 
-// velocity of plane x scaled by target / flux[x] (limited to [1/4, 4]; planes without flux keep
-// theirs), then speeds clipped to umax
-__global__ void k_scale_clip(double* out, int64_t ns, int64_t nx, int64_t nxp, const double* flux, double target,
-                             const double* targets, const double* drho, double rlo, double rhi, double umax) {
-    const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= ns) return;
-    const int64_t x = n % nxp;
-    if (x < nx && targets) target = targets[x];
+// flux[x] = the blocks' sums: 8 row groups of 32 planes a block, each in ascending order, then the groups
+__global__ __launch_bounds__(256) void k_flux_final(const double* part, int nblocks, int64_t nxp, int64_t nx, double* flux) {
+    __shared__ double sh[8][32];
+    const int c = threadIdx.x & 31, r = threadIdx.x >> 5;
+    const int64_t x = (int64_t)blockIdx.x * 32 + c;
+    double s = 0.0;
+    if (x < nx)
+        for (int b = r; b < nblocks; b += 8) s += part[b * nxp + x];
+    sh[r][c] = s;
+    __syncthreads();
+    if (r == 0 && x < nx) {
+        for (int k = 1; k < 8; k++) s += sh[k][c];
+        flux[x] = s;
+    }
+}
+
+// The expanded field at the nodes, one wave per tile: the coarse sample (rest where it is not finite), its
+// density clipped, the velocity of plane x scaled by target / flux[x] (limited to [1/4, 4]; planes without flux
+// keep theirs), drho[x] added to the density, which is clipped again, speeds clipped to umax.  Only the slots of
+// nodes are written: nothing reads the others.
+__global__ __launch_bounds__(256) void k_expand_nodes(const CoarseField F, int64_t nxp, int64_t nyp, int64_t ns,
+                                                      const TileDesc* tdesc, int ntiles, double rlo, double rhi,
+                                                      const double* flux, double target, const double* targets,
+                                                      const double* drho, double umax, double* out) {
+    const int t = blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (t >= ntiles) return;
+    const int tile = tdesc[t].tile, nxt = (int)(nxp / 64), row = tile / nxt;
+    if (!((tdesc[t].node >> lane) & 1ull)) return;
+    const int64_t n = (int64_t)tile * 64 + lane, x = 64 * (tile - row * nxt) + lane;
+    float v[4];
+    coarse_sample<0, 4>(F, x, row % (int)nyp, row / (int)nyp, v);
+    double r = 1.0, u0 = 0.0, u1 = 0.0, u2 = 0.0;
+    if (finite4(v)) {
+        r = fmin(fmax((double)v[0], rlo), rhi);
+        u0 = v[1];
+        u1 = v[2];
+        u2 = v[3];
+    }
+    if (targets) target = targets[x];
     double f = 1.0;
-    if (flux && target > 0.0 && x < nx && flux[x] > 1e-12 * target) f = fmin(fmax(target / flux[x], 0.25), 4.0);
-    if (drho && x < nx) out[n] = fmin(fmax(out[n] + drho[x], rlo), rhi);
-    double u0 = out[ns + n] * f, u1 = out[2 * ns + n] * f, u2 = out[3 * ns + n] * f;
+    if (flux && target > 0.0 && flux[x] > 1e-12 * target) f = fmin(fmax(target / flux[x], 0.25), 4.0);
+    if (drho) r = fmin(fmax(r + drho[x], rlo), rhi);
+    u0 *= f;
+    u1 *= f;
+    u2 *= f;
     const double sp = sqrt(u0 * u0 + u1 * u1 + u2 * u2);
     if (sp > umax) {
         const double c = umax / sp;
@@ -440,29 +503,42 @@ __global__ void k_scale_clip(double* out, int64_t ns, int64_t nx, int64_t nxp, c
         u1 *= c;
         u2 *= c;
     }
+    out[n] = r;
     out[ns + n] = u0;
     out[2 * ns + n] = u1;
     out[3 * ns + n] = u2;
 }
 
-hipError_t launch_expand_coarse(const float* rho_c, const float* u_c, int cx, int cy, int cz, int64_t nx,
-                                int64_t ny, int64_t nz, int64_t nxp, int64_t nyp, int64_t ns, double umax,
-                                double rlo, double rhi, const uint8_t* kind, double flux_x, const double* targets,
-                                const double* drho, double* flux, double* out, unsigned long long* nonfin,
-                                hipStream_t s) {
-    const int64_t blocks = (ns + 255) / 256;
-    hipLaunchKernelGGL(k_expand_coarse, dim3((unsigned)blocks), dim3(256), 0, s, rho_c, u_c, cx, cy, cz, nx, ny,
-                       nz, nxp, nyp, ns, rlo, rhi, out, nonfin);
+int flux_blocks(int ntiles) { return ntiles < 4 * FLUX_BLOCKS ? (ntiles + 3) / 4 : FLUX_BLOCKS; }
+
+int64_t expand_coarse_doubles(int64_t nx, int64_t nxp, int ntiles) { return 3 * nx + 2 + (int64_t)flux_blocks(ntiles) * nxp; }
+
+hipError_t launch_expand_coarse(const float* rho_c, const float* u_c, int cx, int cy, int cz, int64_t nx, int64_t ny,
+                                int64_t nz, int64_t nxp, int64_t nyp, int64_t ns, const TileDesc* tdesc, int ntiles,
+                                double umax, double rlo, double rhi, double flux_x, const double* targets,
+                                const double* drho, double* flux, double* part, int* flag, double* out,
+                                unsigned long long* nonfin, hipStream_t s) {
+    const CoarseField F{rho_c, u_c, cx, cy, cz, nx, ny, nz};
+    const int64_t nc = (int64_t)cx * cy * cz;
+    hipLaunchKernelGGL(k_coarse_suspect, dim3((unsigned)(nc / 256 < 1024 ? nc / 256 + 1 : 1024)), dim3(256), 0, s, rho_c, u_c, nc, flag);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_coarse_count, dim3(2048), dim3(256), 0, s, F, flag, nonfin);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    if (ntiles <= 0) return hipSuccess;
     const bool scale = flux_x > 0.0 || targets;
     if (scale) {
-        hipLaunchKernelGGL(k_slab_flux, dim3((unsigned)nx), dim3(256), 0, s, out + ns, kind, ny, nz, nxp, nyp, flux);
+        const int nb = flux_blocks(ntiles);
+        hipLaunchKernelGGL(k_flux_nodes, dim3(nb, (unsigned)((nxp / 64 + FLUX_XR - 1) / FLUX_XR)), dim3(256), 0, s, F, nxp, nyp, tdesc, ntiles, part);
+        e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(k_flux_final, dim3((unsigned)((nx + 31) / 32)), dim3(256), 0, s, part, nb, nxp, nx, flux);
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(k_scale_clip, dim3((unsigned)blocks), dim3(256), 0, s, out, ns, nx, nxp,
-                       scale ? flux : nullptr, flux_x, targets, drho, rlo, rhi, umax);
+    hipLaunchKernelGGL(k_expand_nodes, dim3((unsigned)((ntiles + 3) / 4)), dim3(256), 0, s, F, nxp, nyp, ns, tdesc, ntiles,
+                       rlo, rhi, scale ? flux : nullptr, flux_x, targets, drho, umax, out);
     return hipGetLastError();
 }
 

@@ -134,18 +134,20 @@ hipError_t noalloc_scratch(int device, void** ptr);
 // streaming copy of `bytes` (multiple of 16) for counter calibration
 hipError_t launch_copy(const void* src, void* dst, int64_t bytes, hipStream_t s);
 
-// Dense initial fields out[4][ns] (rho, ux, uy, uz per padded slot) sampled trilinearly from a
-// coarse FP32 field (rho_c[cz][cy][cx], u_c[3][cz][cy][cx], voxel centres at fine coordinates
-// (i + 0.5) n / c - 0.5), densities clipped into [rlo, rhi]; padding slots and non-finite samples
-// (counted in *nonfin) get rest.  With flux_x > 0 the velocity of every plane x is scaled so that
-// the flux of u_x over its fluid nodes (kind != 0) is flux_x, or targets[x] when targets (nx
-// device doubles) is given (flux: nx doubles of scratch); speeds are then clipped to umax.  With
-// drho (nx device doubles) every slot of plane x gets drho[x] added to its density, clipped again.
-hipError_t launch_expand_coarse(const float* rho_c, const float* u_c, int cx, int cy, int cz, int64_t nx,
-                                int64_t ny, int64_t nz, int64_t nxp, int64_t nyp, int64_t ns, double umax,
-                                double rlo, double rhi, const uint8_t* kind, double flux_x, const double* targets,
-                                const double* drho, double* flux, double* out, unsigned long long* nonfin,
-                                hipStream_t s);
+// Initial fields out[4][ns] (rho, ux, uy, uz; padded slots) at the nodes of the ntiles tiles, sampled
+// trilinearly from a coarse FP32 field (rho_c[cz][cy][cx], u_c[3][cz][cy][cx], voxel centres at fine
+// coordinates (i + 0.5) n / c - 0.5), densities clipped into [rlo, rhi]; non-finite samples (of all box points,
+// counted in *nonfin) get rest.  With flux_x > 0 the velocity of every plane x is scaled so that the flux of u_x
+// over its nodes is flux_x, or targets[x] when targets (nx device doubles) is given; speeds are then clipped to
+// umax.  With drho (nx device doubles) every node of plane x gets drho[x] added to its density, clipped again.
+// flux (nx doubles) and part are scratch (expand_coarse_doubles in all, with targets and drho); *flag and
+// *nonfin must be zero.
+int64_t expand_coarse_doubles(int64_t nx, int64_t nxp, int ntiles);
+hipError_t launch_expand_coarse(const float* rho_c, const float* u_c, int cx, int cy, int cz, int64_t nx, int64_t ny,
+                                int64_t nz, int64_t nxp, int64_t nyp, int64_t ns, const TileDesc* tdesc, int ntiles,
+                                double umax, double rlo, double rhi, double flux_x, const double* targets,
+                                const double* drho, double* flux, double* part, int* flag, double* out,
+                                unsigned long long* nonfin, hipStream_t s);
 
 // Compact FP32 box fields from the macro planes (macro[4][ns], padded slots): rho[b] and
 // u[c][b] for every box point b = i + nx (j + ny k); points that are not nodes (kind 0) get

@@ -542,24 +542,54 @@ hipError_t launch_expand_coarse(const float* rho_c, const float* u_c, int cx, in
     return hipGetLastError();
 }
 
-// one thread per box point; reads the padded slot of the same point
-__global__ void k_macros_f32(const double* macro, const uint8_t* kind, int64_t nx, int64_t ny, int64_t nbox,
-                             int64_t nxp, int64_t nyp, int64_t ns, float* rho, float* u) {
-    const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nbox) return;
-    const int64_t i = b % nx, r = b / nx;
-    const int64_t n = (r % ny + nyp * (r / ny)) * nxp + i;
-    const bool node = kind[n] != 0;
-    rho[b] = node ? (float)macro[n] : 1.0f;
-    for (int c = 0; c < 3; c++) u[c * nbox + b] = node ? (float)macro[(c + 1) * ns + n] : 0.0f;
+// Compact FP32 fields, four points of a row per thread (VEC: whole quads with 16-byte stores).  Bound by the
+// output's 16 bytes a point: most points are not nodes and read one kind byte.  1024 x 512 x 512: 1.03 ms
+// (4.4 TB/s), 1.30 ms with one point and 64-bit divisions per thread.
+template <bool VEC, class I>
+__global__ __launch_bounds__(256) void k_macros_f32(const double* macro, const uint8_t* kind, int64_t nx, uint32_t ny, int64_t nbox,
+                                                    I nq, I quads, int64_t nxp, int64_t nyp, int64_t ns, float* rho, float* u) {
+    const I q = (I)blockIdx.x * 256 + threadIdx.x;
+    if (q >= quads) return;
+    const I row = q / nq;
+    const int64_t i = 4 * (int64_t)(q - row * nq), r = (int64_t)row;
+    const int64_t n = ((int64_t)((uint32_t)row % ny) + nyp * (int64_t)((uint32_t)row / ny)) * nxp + i, b = r * nx + i;
+    const uint32_t k4 = *reinterpret_cast<const uint32_t*>(kind + n);  // rows are padded: always within the row
+    float v[4][4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const bool node = (k4 >> (8 * e)) & 0xffu;
+        v[0][e] = node ? (float)macro[n + e] : 1.0f;
+#pragma unroll
+        for (int c = 1; c < 4; c++) v[c][e] = node ? (float)macro[c * ns + n + e] : 0.0f;
+    }
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        float* dst = (c == 0 ? rho : u + (c - 1) * nbox) + b;
+        if constexpr (VEC) {
+            typedef float f4 __attribute__((ext_vector_type(4)));
+            __builtin_nontemporal_store(f4{v[c][0], v[c][1], v[c][2], v[c][3]}, reinterpret_cast<f4*>(dst));
+        } else {
+            for (int e = 0; e < 4; e++)
+                if (i + e < nx) dst[e] = v[c][e];
+        }
+    }
 }
 
 hipError_t launch_macros_f32(const double* macro, const uint8_t* kind, int64_t nx, int64_t ny, int64_t nz,
                              int64_t nxp, int64_t nyp, int64_t ns, float* rho, float* u, hipStream_t s) {
     const int64_t nbox = nx * ny * nz;
     if (nbox <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_macros_f32, dim3((unsigned)((nbox + 255) / 256)), dim3(256), 0, s, macro, kind, nx, ny,
-                       nbox, nxp, nyp, ns, rho, u);
+    const int64_t nq = (nx + 3) / 4, quads = nq * ny * nz;
+    const dim3 g((unsigned)((quads + 255) / 256));
+    const bool vec = nx % 4 == 0 && (uintptr_t)rho % 16 == 0 && (uintptr_t)u % 16 == 0;
+    const bool wide = quads > 0xffffff00ll;  // 32-bit quad indices otherwise: their divisions are far cheaper
+#define PV_MACROS(V, I) \
+    hipLaunchKernelGGL((k_macros_f32<V, I>), g, dim3(256), 0, s, macro, kind, nx, (uint32_t)ny, nbox, (I)nq, (I)quads, nxp, nyp, ns, rho, u)
+    if (vec && wide) PV_MACROS(true, int64_t);
+    else if (vec) PV_MACROS(true, uint32_t);
+    else if (wide) PV_MACROS(false, int64_t);
+    else PV_MACROS(false, uint32_t);
+#undef PV_MACROS
     return hipGetLastError();
 }
 

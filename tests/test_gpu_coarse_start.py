@@ -47,3 +47,7 @@ def test_coarse_start(nx, coarse, bad, planes):
     # FP32 interpolation of values up to 1: a few roundings of 2^-24 each
     assert np.abs(r - rf)[nodes].max() < 4e-6 and np.abs(v - uf)[:, nodes].max() < 4e-6
     assert sim.reduce()[3] == 0
+    # the FP32 read-out of the same fields: rows of whole and of partial quads
+    r32, v32 = (t.cpu().numpy() for t in sim.macros_device())
+    assert np.array_equal(r32, np.where(nodes, r, 1.0).astype(np.float32))
+    assert np.array_equal(v32, v.astype(np.float32))

@@ -439,8 +439,16 @@ __global__ __launch_bounds__(256) void k_relayout(const StepParams p) {
 __global__ __launch_bounds__(256) void k_reduce_final(const double* partials, int nparts, double* out4) {
     __shared__ double s[4][256];
     double a[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int i = threadIdx.x; i < nparts; i += 256)
-        for (int k = 0; k < 4; k++) a[k] += partials[4 * (int64_t)i + k];
+    // one block: bound by the latency of its loads, so eight rows are in flight per thread (30,362 rows: 43 -> 20 us)
+#pragma unroll 8
+    for (int i = threadIdx.x; i < nparts; i += 256) {
+        const double2 p = *reinterpret_cast<const double2*>(partials + 4 * (int64_t)i);
+        const double2 q = *reinterpret_cast<const double2*>(partials + 4 * (int64_t)i + 2);
+        a[0] += p.x;
+        a[1] += p.y;
+        a[2] += q.x;
+        a[3] += q.y;
+    }
     for (int k = 0; k < 4; k++) s[k][threadIdx.x] = a[k];
     __syncthreads();
     for (int w = 128; w > 0; w >>= 1) {

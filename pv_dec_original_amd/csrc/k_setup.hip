@@ -187,37 +187,73 @@ __global__ __launch_bounds__(256) void k_tri_prep(const double* tri, int64_t ntr
     prep[6 * ntri + t] = (T[2] + T[5] + T[8]) / 3.0;
 }
 
-// Normal of each listed node: sum over all triangles of unit normal * area / distance^2, then
-// normalised (Subdomain.cpp:343-368).  One thread per node, summing in triangle file order as the
-// reference does; the block's threads stage the per-triangle quantities in LDS, 256 triangles at a
-// time, so each is read from memory once per block instead of once per node.
-__global__ __launch_bounds__(256) void k_normals(const double* prep, int64_t ntri, const double* xyz,
-                                                int64_t n, double* nrm) {
-    constexpr int CH = 256;
-    __shared__ double P[7][CH];
-    const int64_t w = (int64_t)blockIdx.x * 256 + threadIdx.x;
+// Normal of each listed node: sum over all triangles of unit normal * area / distance^2, then normalised
+// (Subdomain.cpp:343-368).  The sums run in triangle file order as the reference's do, one chain per node and
+// component; what a chain adds, the weight area / distance^2 with its FP64 square root and division, is
+// independent of it.  So most threads of a block compute the weights of a chunk of triangles for its NODES nodes
+// into LDS while others, one per (component, node), add the chunk before: the reference's roundings, with the
+// costly part spread over the chip even when there are few nodes (whole set-up of a subdomain with 16823 such
+// nodes and 162664 triangles 31.1 ms with one thread a node, 14.3 this way).  Bound by the FP64
+// rate (about 300 clocks a triangle, wave and SIMD) and, with few nodes, by how evenly the blocks fall on the CUs.
+constexpr int NRM_CH = 64;  // triangles per chunk, 8 consecutive ones per weight thread
+
+template <int NODES>
+constexpr int nrm_threads() { return NODES * NRM_CH / 8 + (3 * NODES + 63) / 64 * 64; }
+
+template <int NODES>
+__global__ __launch_bounds__(nrm_threads<NODES>()) void k_normals(const double* __restrict__ prep, int64_t ntri,
+                                                                const double* __restrict__ xyz, int64_t n,
+                                                                double* __restrict__ nrm) {
+    constexpr int WT = NODES * NRM_CH / 8;  // weight threads: whole waves
+    constexpr int UNR = NODES == 64 ? 16 : 8;  // 64: hides the LDS reads, 106773 nodes 295 ms (8: 322)
+    __shared__ double Wt[2][NRM_CH][NODES];
+    const int t = threadIdx.x, node = t % NODES;
+    const int64_t w = (int64_t)blockIdx.x * NODES + node;
     const bool act = w < n;
-    const double x = act ? xyz[w] : 0.0, y = act ? xyz[n + w] : 0.0, z = act ? xyz[2 * n + w] : 0.0;
-    double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-    for (int64_t t0 = 0; t0 < ntri; t0 += CH) {
-        const int64_t t = t0 + threadIdx.x;
-        __syncthreads();  // the previous chunk is consumed
-        if (t < ntri)
-            for (int c = 0; c < 7; c++) P[c][threadIdx.x] = prep[c * ntri + t];
-        __syncthreads();
-        const int m = (int)(ntri - t0 < CH ? ntri - t0 : CH);
-#pragma unroll 4
-        for (int k = 0; k < m; k++) {
-            const double cX = P[4][k], cY = P[5][k], cZ = P[6][k];
+    const int64_t nch = (ntri + NRM_CH - 1) / NRM_CH;
+    double a = 0.0;
+    if (t < WT) {
+        const double x = act ? xyz[w] : 0.0, y = act ? xyz[n + w] : 0.0, z = act ? xyz[2 * n + w] : 0.0;
+        // NODES = 64: a wave's triangles are the same for all lanes (scalar loads)
+        const int k0 = 8 * (NODES == 64 ? __builtin_amdgcn_readfirstlane(t >> 6) : t / NODES);
+        auto weight = [&](int64_t i) {
+            const double cX = prep[4 * ntri + i], cY = prep[5 * ntri + i], cZ = prep[6 * ntri + i];
             const double distance = sqrt((x - cX) * (x - cX) + (y - cY) * (y - cY) + (z - cZ) * (z - cZ));
-            const double weight = P[3][k] / (distance * distance);
-            a0 += P[0][k] * weight;
-            a1 += P[1][k] * weight;
-            a2 += P[2][k] * weight;
+            return prep[3 * ntri + i] / (distance * distance);
+        };
+        for (int64_t ch = 0; ch <= nch; ch++) {
+            const int64_t t0 = ch * NRM_CH + k0;
+            if (t0 + 8 <= ntri) {
+#pragma unroll
+                for (int k = 0; k < 8; k++) Wt[ch & 1][k0 + k][node] = weight(t0 + k);
+            } else {
+                for (int k = 0; k < 8; k++)
+                    if (t0 + k < ntri) Wt[ch & 1][k0 + k][node] = weight(t0 + k);
+            }
+            __syncthreads();  // chunk ch is there, chunk ch - 1 is consumed
         }
+    } else {
+        const int c = NODES == 64 ? __builtin_amdgcn_readfirstlane((t - WT) >> 6) : (t - WT) / NODES;
+        const double* C = prep + (c < 3 ? c : 2) * ntri;  // threads past the third component repeat it unused
+        for (int64_t ch = 0; ch <= nch; ch++) {
+            if (ch > 0) {
+                const double(*W)[NODES] = Wt[(ch - 1) & 1];
+                const int64_t t0 = (ch - 1) * NRM_CH;
+                if (t0 + NRM_CH <= ntri) {
+#pragma unroll(UNR)
+                    for (int k = 0; k < NRM_CH; k++) a += C[t0 + k] * W[k][node];
+                } else {
+                    for (int64_t i = t0; i < ntri; i++) a += C[i] * W[i - t0][node];
+                }
+            }
+            __syncthreads();
+        }
+        // the three components of a node sit in three threads: gathered in LDS (free after the last barrier)
+        if (c < 3) Wt[0][c][node] = a;
     }
-    if (!act) return;
-    double n0 = a0, n1 = a1, n2 = a2;
+    __syncthreads();
+    if (t >= NODES || !act) return;
+    double n0 = Wt[0][0][t], n1 = Wt[0][1][t], n2 = Wt[0][2][t];
     const double norm = sqrt(n0 * n0 + n1 * n1 + n2 * n2);
     if (norm > 0) {
         n0 /= norm;
@@ -264,7 +300,16 @@ hipError_t launch_tri_prep(const double* tri, int64_t ntri, double* prep, hipStr
 hipError_t launch_normals(const double* prep, int64_t ntri, const double* xyz, int64_t n, double* nrm,
                           hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_normals, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, prep, ntri, xyz, n, nrm);
+    // 64 nodes a block read the triangles by scalar loads, which is 10 % less work a pair; 16 divide few nodes
+    // more evenly over the chip.  The line is four blocks of 64 nodes a CU, where the unevenness (one block in
+    // four at most) has come down to that: 16823 nodes, 162664 triangles 17.8 ms with 64 and 14.3 with 16;
+    // 106773 nodes, 850648 triangles 295 with 64 and 330 with 16 (whole set-up of the subdomain).
+    if (n >= 4 * 256 * 64)
+        hipLaunchKernelGGL(k_normals<64>, dim3((unsigned)((n + 63) / 64)), dim3(nrm_threads<64>()), 0, s, prep,
+                           ntri, xyz, n, nrm);
+    else
+        hipLaunchKernelGGL(k_normals<16>, dim3((unsigned)((n + 15) / 16)), dim3(nrm_threads<16>()), 0, s, prep,
+                           ntri, xyz, n, nrm);
     return hipGetLastError();
 }
 

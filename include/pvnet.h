@@ -58,6 +58,14 @@ typedef struct {
 
 int pvnet_conv_fwd(const pvnet_conv* c, void* stream);
 
+/* The same 3x3x3 convolution on a concatenation that is not laid out: input channels 0 .. cup-1 are `up`, of
+ * shape s/2, upsampled (nearest, as pvnet_up2_fwd), channels cup .. cin-1 are c->x (ldx >= cin - cup).  The
+ * sizes must be even, cup and ldu multiples of 8; bf16 output.  Bit for bit the result on the laid-out input. */
+int pvnet_conv_up_fwd(const pvnet_conv* c, const uint16_t* up, int32_t ldu, int32_t cup, void* stream);
+/* The same convolution with its output in two tensors: channels 0 .. c0-1 to y0, c0 .. cout-1 to c->y
+ * (ldy >= cout - c0); relu_of is indexed by all cout channels; bf16 output, cout and c0 multiples of 8. */
+int pvnet_conv_split_fwd(const pvnet_conv* c, uint16_t* y0, int32_t ldy0, int32_t c0, void* stream);
+
 /* dw[n][k] = sum_m dy[m][n] * x[m + off(tap(k))][ci(k)]  for k < ntaps*cin (row length ntaps*cin)
  * db[n]    = sum_m dy[m][n]                               (if db is not NULL; cout <= 256)
  * ws: FP32 scratch of at least pvnet_wgrad_ws_floats(...) floats for the split-K partials; the
@@ -80,6 +88,8 @@ typedef struct {
 
 int64_t pvnet_wgrad_ws_floats(const pvnet_shape* s, int32_t ntaps, int32_t cin, int32_t cout);
 int pvnet_conv_wgrad(const pvnet_wgrad* g, void* stream);
+/* with the input in two parts, as pvnet_conv_up_fwd */
+int pvnet_conv_up_wgrad(const pvnet_wgrad* g, const uint16_t* up, int32_t ldu, int32_t cup, void* stream);
 
 /* Packs FP32 master weights w32[cout][ntaps*cin] into the bf16 forward layout wt[cout][kpad]
  * and the bf16 input-gradient layout wd[cin][kpad_d] (kpad_d = roundup(ntaps*cout, 32)), whose
@@ -105,6 +115,9 @@ int pvnet_up2_fwd(const pvnet_shape* s, int32_t c, const uint16_t* x, int32_t ld
                   int32_t ldy, void* stream);
 int pvnet_up2_bwd(const pvnet_shape* s, int32_t c, const uint16_t* dy, int32_t lddy, uint16_t* dx,
                   int32_t lddx, void* stream);
+/* followed by the backward of a ReLU whose output is relu_of (shape s/2), in one pass */
+int pvnet_up2_bwd_relu(const pvnet_shape* s, int32_t c, const uint16_t* dy, int32_t lddy, uint16_t* dx,
+                       int32_t lddx, const uint16_t* relu_of, int32_t ldr, void* stream);
 
 /* dx[m][c] = (a[m][c] > 0) ? dx[m][c] : 0, in place (the backward of a ReLU with output a). */
 int pvnet_relu_bwd(int64_t m, int32_t c, const uint16_t* a, int32_t lda, uint16_t* dx, int32_t lddx,

@@ -128,14 +128,18 @@ _vp = C.c_void_p
 _sp = C.POINTER(NetShape)
 PVNET_API = [
     ("pvnet_conv_fwd", C.c_int, [C.POINTER(NetConv), _vp]),
+    ("pvnet_conv_up_fwd", C.c_int, [C.POINTER(NetConv), _vp, C.c_int32, C.c_int32, _vp]),
+    ("pvnet_conv_split_fwd", C.c_int, [C.POINTER(NetConv), _vp, C.c_int32, C.c_int32, _vp]),
     ("pvnet_wgrad_ws_floats", C.c_int64, [_sp, C.c_int32, C.c_int32, C.c_int32]),
     ("pvnet_conv_wgrad", C.c_int, [C.POINTER(NetWgrad), _vp]),
+    ("pvnet_conv_up_wgrad", C.c_int, [C.POINTER(NetWgrad), _vp, C.c_int32, C.c_int32, _vp]),
     ("pvnet_pack_weights", C.c_int, [_vp, C.c_int32, C.c_int32, C.c_int32, _vp, _vp, _vp]),
     ("pvnet_pool2_fwd", C.c_int, [_sp, C.c_int32, _vp, C.c_int32, _vp, C.c_int32, _vp]),
     ("pvnet_pool2_bwd", C.c_int, [_sp, C.c_int32, _vp, C.c_int32, _vp, C.c_int32, C.c_int32, _vp]),
     ("pvnet_pool2_bwd_relu", C.c_int, [_sp, C.c_int32, _vp, C.c_int32, _vp, C.c_int32, _vp, C.c_int32, _vp]),
     ("pvnet_up2_fwd", C.c_int, [_sp, C.c_int32, _vp, C.c_int32, _vp, C.c_int32, _vp]),
     ("pvnet_up2_bwd", C.c_int, [_sp, C.c_int32, _vp, C.c_int32, _vp, C.c_int32, _vp]),
+    ("pvnet_up2_bwd_relu", C.c_int, [_sp, C.c_int32, _vp, C.c_int32, _vp, C.c_int32, _vp, C.c_int32, _vp]),
     ("pvnet_relu_bwd", C.c_int, [C.c_int64, C.c_int32, _vp, C.c_int32, _vp, C.c_int32, _vp]),
     ("pvnet_wall_distance", C.c_int, [_sp, _vp, _vp, _vp]),
     ("pvnet_features", C.c_int, [_sp, _vp, _vp, _vp, _vp, _vp]),

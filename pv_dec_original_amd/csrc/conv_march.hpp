@@ -8,7 +8,11 @@
 //                arrives.  The narrow layers (cin 8, 16, 48): a k-step may span two dz.
 //   k_conv_roll  cin % 32 == 0: every k-step lies within one dz, so plane p is read from LDS once for all
 //                three output planes p+1 (dz = -1), p and p-1 (dz = +1), whose accumulators roll; two slots.
-// Both run the k-steps of k_conv_fwd in the same order (k = tap * cin + ci, 32 per MFMA), so every output
+// The input may come in two parts: channels below `cup` from a tensor of half the size (nearest upsampling), the
+// others from x; a copied unit then picks its source, and the upsampled half is never written out.  The output
+// may go to two tensors in the same way, so that skips and gradients are dense rows for the layers and poolings
+// that read them (a training step on 8 x 96^3: 7.03 -> 5.77 ms, of which the upsampling was 0.30, the poolings
+// 0.43 and a skip written into the middle of 96-byte rows 0.22).  Both run the k-steps of k_conv_fwd in the same order (k = tap * cin + ci, 32 per MFMA), so every output
 // equals that kernel's bit for bit.  The weights are the MFMA's A operand and the voxels its B operand: a
 // lane then holds four consecutive channels of one voxel and writes them with one 8-byte store.
 //
@@ -66,6 +70,7 @@ template <int RT, bool WL, int NP>
 struct MarchBlock {
     const pvnet_conv& a;
     const MarchPlan& p;
+    const NetParts& q;
     uint4* wl;
     int *tab, *soff;
     int lane, g, c16, wv, nu, n0, nw, x0, y0, z0, z1;  // n0: this wave's 16 channels
@@ -76,7 +81,8 @@ struct MarchBlock {
     float bias[4];
     uint2 mk[RT];            // ReLU mask of the plane
 
-    __device__ __forceinline__ MarchBlock(const pvnet_conv& a_, const MarchPlan& p_, uint4* sm, int sp) : a(a_), p(p_) {
+    __device__ __forceinline__ MarchBlock(const pvnet_conv& a_, const MarchPlan& p_, const NetParts& q_, uint4* sm, int sp)
+        : a(a_), p(p_), q(q_) {
         const int t = threadIdx.x;
         lane = t & 63, g = lane >> 4, c16 = lane & 15;
         wv = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -99,7 +105,8 @@ struct MarchBlock {
         z0 = (bid % p.nzs) * p.zseg, z1 = min(a.s.d, z0 + p.zseg);
         box = bid / p.nzs;
 
-        // element offset of every unit within its plane (-1: outside the box).  Two chunks of a voxel lie
+        // element offset of every unit within its plane (-1: outside the box; bit 0: a plane of the half-size
+        // tensor).  Two chunks of a voxel lie
         // side by side: a copy then reads 32 contiguous bytes per voxel, and the 16 + 16 lanes that read a
         // fragment's two chunks together cover every bank once, whatever the tap's shift.
         const int hxy = p.hx * (p.ty + 2);
@@ -108,7 +115,8 @@ struct MarchBlock {
             const int ch = cg * p.g + (r - v * p.g);
             const int hy = v / p.hx, x = x0 - 1 + v - hy * p.hx, y = y0 - 1 + hy;
             const bool in = v < hxy && (unsigned)x < (unsigned)w && (unsigned)y < (unsigned)h;
-            soff[u] = in ? (y * w + x) * a.ldx + ch * 8 : -1;
+            soff[u] = !in ? -1 : 8 * ch < q.cup ? ((y >> 1) * (w >> 1) + (x >> 1)) * q.ldu + ch * 8 + 1
+                                                : (y * w + x) * a.ldx + ch * 8 - q.cup;
         }
         if constexpr (WL) {
             // fragment order: the 64 lanes' operands of (k-step, column tile) are 64 consecutive units
@@ -141,11 +149,13 @@ struct MarchBlock {
     __device__ __forceinline__ void stage_plane(int z, int slot, int first, int of) const {
         const bool zin = (unsigned)z < (unsigned)a.s.d;
         const uint16_t* pb = a.x + (box * a.s.d + (zin ? z : 0)) * ((int64_t)a.s.h * a.s.w) * a.ldx;
+        const uint16_t* pu = q.cup ? q.up + (box * (a.s.d >> 1) + (zin ? z >> 1 : 0)) * ((int64_t)(a.s.h >> 1) * (a.s.w >> 1)) * q.ldu - 1
+                                   : pb;
         for (int u = 64 * first; u < nu; u += 64 * of) {
             const int ul = u + lane;
             if (ul < nu) {
                 const int o = soff[ul];
-                const void* src = (zin && o >= 0) ? (const void*)(pb + o) : (const void*)g_march_zero;
+                const void* src = (zin && o >= 0) ? (const void*)((o & 1 ? pu : pb) + o) : (const void*)g_march_zero;
                 lds_copy16(src, __builtin_amdgcn_readfirstlane(lds0 + 16u * (uint32_t)(slot * p.su + u)));
             }
         }
@@ -185,8 +195,15 @@ struct MarchBlock {
 
     __device__ __forceinline__ void store_plane(int z, const f32x4 (&acc)[RT]) const {
         if (n0 + 4 * g >= a.cout) return;
-        const int64_t mb = (box * a.s.d + z) * ((int64_t)a.s.h * a.s.w);
         const bool relu = a.flags & PVNET_RELU, f32out = a.flags & PVNET_F32OUT;
+        // whether this lane's channels are in the output's first part: opaque, so that the pointer and row length
+        // are not kept in registers through the k-loop
+        int n4 = n0 + 4 * g;
+        asm volatile("" : "+v"(n4));
+        const bool first = n4 < q.c0;
+        const uint32_t ld = first ? q.ldy0 : a.ldy;
+        const int64_t o0 = (box * a.s.d + z) * ((int64_t)a.s.h * a.s.w) * ld + n4 - (first ? 0 : q.c0);
+        char* yb = f32out ? (char*)((float*)a.y + o0) : (char*)((first ? q.y0 : (uint16_t*)a.y) + o0);
 #pragma unroll
         for (int i = 0; i < RT; i++) {
             if (vo[i] < 0) continue;
@@ -197,9 +214,9 @@ struct MarchBlock {
                 if (relu) v[e] = v[e] < 0.f ? 0.f : v[e];
                 if (a.relu_of && !bf_pos((uint16_t)((e < 2 ? mk[i].x : mk[i].y) >> (16 * (e & 1))))) v[e] = 0.f;
             }
-            const int64_t o = (mb + vo[i]) * a.ldy + n0 + 4 * g;
-            if (f32out) *(float4*)((float*)a.y + o) = make_float4(v[0], v[1], v[2], v[3]);
-            else *(uint2*)((uint16_t*)a.y + o) = make_uint2(f2bf_pk(v[0], v[1]), f2bf_pk(v[2], v[3]));
+            const uint64_t o = (uint64_t)(uint32_t)vo[i] * ld;
+            if (f32out) *(float4*)(yb + 4 * o) = make_float4(v[0], v[1], v[2], v[3]);
+            else *(uint2*)(yb + 2 * o) = make_uint2(f2bf_pk(v[0], v[1]), f2bf_pk(v[2], v[3]));
         }
     }
 };
@@ -207,10 +224,10 @@ struct MarchBlock {
 // WM: where the weights are during the k-loop: 0 memory (L2), one step ahead; 1 LDS; 2 registers (NSW
 // k-steps, fixed at compile time)
 template <int RT, int WM, int NSW>
-__global__ __launch_bounds__(256) void k_conv_ring(const pvnet_conv a, const MarchPlan p) {
+__global__ __launch_bounds__(256) void k_conv_ring(const pvnet_conv a, const MarchPlan p, const NetParts q) {
     extern __shared__ uint4 march_sm[];
     const int sp = WM == 2 ? NSW : p.nsteps;
-    MarchBlock<RT, WM == 1, 4> b(a, p, march_sm, sp);
+    MarchBlock<RT, WM == 1, 4> b(a, p, q, march_sm, sp);
     // k-step table per rotation r = z & 3 of the slots: plane z + dz sits in slot (z + dz) & 3
     for (int i = threadIdx.x; i < 4 * 4 * sp; i += 256) {
         const int r = i / (4 * sp), e = i - r * (4 * sp);
@@ -291,10 +308,10 @@ __global__ __launch_bounds__(256) void k_conv_ring(const pvnet_conv a, const Mar
 // only copies planes, so that its copies do not hold up the weight loads of the others (a wave's loads
 // return in order).  WL: weights in LDS, else read from memory (L2) two steps ahead.
 template <int RT, bool WL>
-__global__ __launch_bounds__(512) void k_conv_roll(const pvnet_conv a, const MarchPlan p) {
+__global__ __launch_bounds__(512) void k_conv_roll(const pvnet_conv a, const MarchPlan p, const NetParts q) {
     extern __shared__ uint4 march_sm[];
     const int sp = p.nsteps / 3;  // k-steps of one dz: a multiple of 9
-    MarchBlock<RT, WL, 2> b(a, p, march_sm, sp);
+    MarchBlock<RT, WL, 2> b(a, p, q, march_sm, sp);
     for (int i = threadIdx.x; i < 2 * 4 * sp; i += blockDim.x) {
         const int r = i / (4 * sp), e = i - r * (4 * sp);
         const int k = (e >> 2) * BK + (e & 3) * 8;
@@ -388,7 +405,7 @@ __global__ __launch_bounds__(512) void k_conv_roll(const pvnet_conv a, const Mar
 #undef MARCH_WLOAD
 }
 
-typedef void (*MarchKernel)(const pvnet_conv, const MarchPlan);
+typedef void (*MarchKernel)(const pvnet_conv, const MarchPlan, const NetParts);
 
 template <int RT>
 MarchKernel march_kernel_rt(const MarchPlan& p) {
@@ -533,11 +550,13 @@ inline bool march_plan(const pvnet_conv& c, MarchPlan& p) { return kept_plan<Mar
 
 // The marching kernels take 3x3x3 convolutions whose outputs (and ReLU mask) can be accessed four channels at a
 // time; PVNET_GATHER keeps k_conv_fwd.
-inline bool march_ok(const pvnet_conv& c) {
+inline bool march_ok(const pvnet_conv& c, const NetParts& q) {
     if (c.ntaps != 27 || (c.flags & PVNET_GATHER) || c.cout % 4 || c.ldy % 4) return false;
     if ((uintptr_t)c.y % (c.flags & PVNET_F32OUT ? 16 : 8)) return false;
     if (c.relu_of && (c.ldr % 4 || (uintptr_t)c.relu_of % 8)) return false;
     if ((int64_t)c.s.h * c.s.w * c.ldx >= (int64_t)1 << 31) return false;  // plane offsets are 32-bit
+    if ((int64_t)(c.s.h / 2) * (c.s.w / 2) * q.ldu >= (int64_t)1 << 31) return false;
+    if (q.c0 && (q.ldy0 % 4 || (uintptr_t)q.y0 % 8)) return false;
     // weight rows and the block count are 32-bit too (a block has at least one voxel of every 16 channels)
     return (int64_t)c.cout * c.kpad * 2 < (int64_t)1 << 32 &&
            (int64_t)c.s.nb * c.s.d * c.s.h * c.s.w * ((c.cout + 15) / 16) < (int64_t)1 << 31;

@@ -83,11 +83,19 @@ __device__ __forceinline__ void tap_offset(int ntaps, int tap, int& dz, int& dy,
     }
 }
 
+// Inputs and outputs in two parts.  Input channels 0 .. cup - 1 are `up`, a tensor of half the size in each axis
+// (nearest upsampling), the others x; output channels 0 .. c0 - 1 go to y0, the others to y.  All zero: one part.
+struct NetParts {
+    const uint16_t* up;
+    uint16_t* y0;
+    int32_t ldu, cup, ldy0, c0;
+};
+
 // ---------------------------------------------------------------------------------------------
 // forward / input-gradient convolution: block tile 4*WM voxels x BN channels, 4 waves of WM x BN
 
-template <int BN, int WM>
-__global__ __launch_bounds__(256) void k_conv_fwd(pvnet_conv a, int M, int K) {
+template <int BN, int WM, bool PARTS = false>
+__global__ __launch_bounds__(256) void k_conv_fwd(pvnet_conv a, int M, int K, NetParts pq) {
     constexpr int BM = 4 * WM;
     constexpr int NA = BM / 64;  // A rows loaded per thread and step
     __shared__ __attribute__((aligned(16))) uint16_t As[BM * LP];
@@ -103,11 +111,13 @@ __global__ __launch_bounds__(256) void k_conv_fwd(pvnet_conv a, int M, int K) {
     const int q = t & 3, r = t >> 2, bn = t >> 2;
     uint32_t tmask[NA];
     const uint16_t* rowp[NA];
+    int pz[NA], py[NA], px[NA];  // PARTS: the row's box and plane, y, x
     #pragma unroll
     for (int i = 0; i < NA; i++) {
         const int m = m0 + r + 64 * i;
         const int mm = m < M ? m : 0;
         const int xx = mm % w, tq = mm / w, yy = tq % h, zz = (tq / h) % d;
+        pz[i] = tq / h, py[i] = yy, px[i] = xx;
         uint32_t mk = 0;
         if (m < M) {
             for (int tp = 0; tp < a.ntaps; tp++) {
@@ -134,7 +144,14 @@ __global__ __launch_bounds__(256) void k_conv_fwd(pvnet_conv a, int M, int K) {
         #pragma unroll
         for (int i = 0; i < NA; i++) {
             ra[i] = make_uint4(0, 0, 0, 0);
-            if (kin && ((tmask[i] >> tap) & 1u)) ra[i] = *(const uint4*)(rowp[i] + off);
+            const uint16_t* src = rowp[i] + off;
+            if constexpr (PARTS) {  // sizes are even where cup > 0: halving box * d + z halves both
+                src -= pq.cup;
+                if (ci < pq.cup)
+                    src = pq.up + ((int64_t)((pz[i] + dz) >> 1) * (h >> 1) + ((py[i] + dy) >> 1)) * (w >> 1) * pq.ldu +
+                          (int64_t)((px[i] + dx) >> 1) * pq.ldu + ci;
+            }
+            if (kin && ((tmask[i] >> tap) & 1u)) ra[i] = *(const uint4*)src;
         }
         rb = make_uint4(0, 0, 0, 0);
         if (brow) rb = *(const uint4*)(wp + s * BK);
@@ -183,7 +200,11 @@ __global__ __launch_bounds__(256) void k_conv_fwd(pvnet_conv a, int M, int K) {
                 float v = acc[i][j][e] + b;
                 if (relu) v = v < 0.f ? 0.f : v;
                 if (a.relu_of && !bf_pos(a.relu_of[(int64_t)m * a.ldr + n])) v = 0.f;
-                if (f32out)
+                if (PARTS && n < pq.c0)
+                    pq.y0[(int64_t)m * pq.ldy0 + n] = f2bf(v);
+                else if (PARTS)
+                    ((uint16_t*)a.y)[(int64_t)m * a.ldy + n - pq.c0] = f2bf(v);
+                else if (f32out)
                     ((float*)a.y)[(int64_t)m * a.ldy + n] = v;
                 else
                     ((uint16_t*)a.y)[(int64_t)m * a.ldy + n] = f2bf(v);
@@ -274,8 +295,8 @@ __device__ __forceinline__ void transpose8(const uint4 (&r)[8], uint4 (&o)[8]) {
         }
 }
 
-template <int BN>
-__global__ __launch_bounds__(256) void k_conv_wgrad(pvnet_wgrad a, int M, int K, int mchunk) {
+template <int BN, bool PARTS = false>
+__global__ __launch_bounds__(256) void k_conv_wgrad(pvnet_wgrad a, int M, int K, int mchunk, NetParts pq) {
     constexpr int BMW = 128;  // voxels per LDS fill
     constexpr int PW = BMW + 8;  // LDS row pitch in bf16 (272 bytes)
     __shared__ __attribute__((aligned(16))) uint16_t As[BN * PW];  // dy^T  [n][m]
@@ -309,6 +330,8 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(pvnet_wgrad a, int M, int K,
         const int m0 = mbase + mg * 8;
         if (xrole) {
             int x = m0 % w, tq = m0 / w, y = tq % h, z = (tq / h) % d;
+            const bool up = PARTS && ci < pq.cup;
+            int bz = tq / h - z;  // planes of the boxes before
 #pragma unroll
             for (int i = 0; i < 8; i++) {
                 const int m = m0 + i;
@@ -316,12 +339,15 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(pvnet_wgrad a, int M, int K,
                 const bool in = kin && m < me && (unsigned)z2 < (unsigned)d && (unsigned)y2 < (unsigned)h &&
                                 (unsigned)x2 < (unsigned)w;
                 r[i] = make_uint4(0, 0, 0, 0);
-                if (in) r[i] = *(const uint4*)(a.x + ((int64_t)m + off) * a.ldx + ci);
+                if (in && up)
+                    r[i] = *(const uint4*)(pq.up + (((int64_t)((bz + z2) >> 1) * (h >> 1) + (y2 >> 1)) * (w >> 1) + (x2 >> 1)) * pq.ldu + ci);
+                else if (in)
+                    r[i] = *(const uint4*)(a.x + ((int64_t)m + off) * a.ldx + ci - (PARTS ? pq.cup : 0));
                 if (++x == w) {  // next voxel
                     x = 0;
                     if (++y == h) {
                         y = 0;
-                        if (++z == d) z = 0;
+                        if (++z == d) z = 0, bz += d;
                     }
                 }
             }
@@ -538,7 +564,9 @@ __global__ void k_up2_fwd(pvnet_shape s, int c, const uint16_t* x, int ldx, uint
     *(uint4*)(y + f * ldy + ch) = *(const uint4*)(x + ci * ldx + ch);
 }
 
-__global__ void k_up2_bwd(pvnet_shape s, int c, const uint16_t* dy, int lddy, uint16_t* dx, int lddx) {
+// relu_of (optional) as in k_pool2_bwd
+__global__ void k_up2_bwd(pvnet_shape s, int c, const uint16_t* dy, int lddy, uint16_t* dx, int lddx,
+                          const uint16_t* relu_of, int ldr) {
     Coarse o;
     int ch;
     if (!coarse_of(s, c / 8, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, o, ch)) return;
@@ -552,6 +580,12 @@ __global__ void k_up2_bwd(pvnet_shape s, int c, const uint16_t* dy, int lddy, ui
     uint4 out;
     uint16_t* po = (uint16_t*)&out;
     for (int j = 0; j < 8; j++) po[j] = f2bf(acc[j]);
+    if (relu_of) {
+        const uint4 av = *(const uint4*)(relu_of + coarse_index(s, o) * ldr + ch);
+        const uint16_t* pa = (const uint16_t*)&av;
+        for (int j = 0; j < 8; j++)
+            if (!bf_pos(pa[j])) po[j] = 0;
+    }
     *(uint4*)(dx + coarse_index(s, o) * lddx + ch) = out;
 }
 
@@ -825,32 +859,39 @@ int pool_args(const pvnet_shape* s, int c, const void* a, int lda, const void* b
     return 0;
 }
 
-}  // namespace
+// the gathering kernel: 256-voxel blocks for narrow outputs on large grids; 64-channel tiles only when the grid
+// still has >= 2048 blocks (the K loop is long, so the device needs many blocks in flight)
+template <bool PARTS>
+void conv_gather(const pvnet_conv& c, const NetParts& pq, int64_t M, hipStream_t st) {
+    const int K = c.ntaps * c.cin, mt = blocks_for(M, 128);
+    if (c.cout <= 16 && M >= (int64_t)256 * 2048) {
+        hipLaunchKernelGGL((k_conv_fwd<16, 64, PARTS>), dim3(blocks_for(M, 256), 1), dim3(256), 0, st, c, (int)M, K, pq);
+    } else if (c.cout <= 16) {
+        hipLaunchKernelGGL((k_conv_fwd<16, 32, PARTS>), dim3(mt, 1), dim3(256), 0, st, c, (int)M, K, pq);
+    } else if (c.cout % 64 == 0 && (int64_t)mt * (c.cout / 64) >= 2048) {
+        hipLaunchKernelGGL((k_conv_fwd<64, 32, PARTS>), dim3(mt, c.cout / 64), dim3(256), 0, st, c, (int)M, K, pq);
+    } else {
+        hipLaunchKernelGGL((k_conv_fwd<32, 32, PARTS>), dim3(mt, (c.cout + 31) / 32), dim3(256), 0, st, c, (int)M, K, pq);
+    }
+}
 
-extern "C" {
-
-const char* pvnet_last_error(void) { return g_err.c_str(); }
-
-int pvnet_conv_fwd(const pvnet_conv* c, void* stream) {
-    if (!c || !shape_ok(&c->s)) return fail(1, "pvnet_conv_fwd: bad shape");
-    if (c->ntaps != 1 && c->ntaps != 27) return fail(1, "pvnet_conv_fwd: ntaps must be 1 or 27");
-    if (c->cin <= 0 || c->cin % 8 || c->cout <= 0) return fail(1, "pvnet_conv_fwd: cin must be a positive multiple of 8");
-    if (c->kpad != kpad_of(c->ntaps, c->cin)) return fail(1, "pvnet_conv_fwd: kpad must be roundup(ntaps*cin, 32)");
-    if (c->ldx < c->cin || c->ldx % 8 || c->ldy < c->cout) return fail(1, "pvnet_conv_fwd: bad row lengths");
-    if (!c->x || !c->w || !c->y || !al16(c->x) || !al16(c->w)) return fail(1, "pvnet_conv_fwd: null or misaligned pointer");
-    if (c->relu_of && c->ldr < c->cout) return fail(1, "pvnet_conv_fwd: bad relu_of row length");
+int conv_launch(const pvnet_conv* c, const NetParts& pq, void* stream, const std::string& who) {
+    if (!c || !shape_ok(&c->s)) return fail(1, who + ": bad shape");
+    if (c->ntaps != 1 && c->ntaps != 27) return fail(1, who + ": ntaps must be 1 or 27");
+    if (c->cin <= 0 || c->cin % 8 || c->cout <= 0) return fail(1, who + ": cin must be a positive multiple of 8");
+    if (c->kpad != kpad_of(c->ntaps, c->cin)) return fail(1, who + ": kpad must be roundup(ntaps*cin, 32)");
+    if (c->ldx < c->cin - pq.cup || c->ldx % 8 || c->ldy < c->cout - pq.c0) return fail(1, who + ": bad row lengths");
+    if (!c->x || !c->w || !c->y || !al16(c->x) || !al16(c->w)) return fail(1, who + ": null or misaligned pointer");
+    if (c->relu_of && c->ldr < c->cout) return fail(1, who + ": bad relu_of row length");
     const int64_t M = voxels(c->s);
-    if (M >= (int64_t)1 << 31) return fail(1, "pvnet_conv_fwd: too many voxels");
+    if (M >= (int64_t)1 << 31) return fail(1, who + ": too many voxels");
     hipStream_t st = (hipStream_t)stream;
     const int K = c->ntaps * c->cin;
-    // tiles of the gathering kernel: 256-voxel blocks for narrow outputs on large grids; 64-channel tiles
-    // only when the grid still has >= 2048 blocks (the K loop is long, so the device needs many blocks in
-    // flight)
-    const int mt = blocks_for(M, 128);
+    const bool parts = pq.cup || pq.c0;
     MarchPlan mp;
-    if (march_ok(*c) && march_plan(*c, mp)) {
+    if (march_ok(*c, pq) && march_plan(*c, mp)) {
         const unsigned nblk = (unsigned)mp.ntx * mp.nty * mp.nzs * mp.ng * c->s.nb;
-        hipLaunchKernelGGL(march_kernel(mp), dim3(nblk), dim3(64 * (mp.wx * mp.wn + mp.roll)), mp.lds, st, *c, mp);
+        hipLaunchKernelGGL(march_kernel(mp), dim3(nblk), dim3(64 * (mp.wx * mp.wn + mp.roll)), mp.lds, st, *c, mp, pq);
     } else if (c->ntaps == 1 && K <= BK && c->cout <= 64 && !(c->flags & PVNET_GATHER)) {
         const dim3 gp((unsigned)((M + 64 * PWT - 1) / (64 * PWT)));
         switch ((c->cout + 15) / 16) {
@@ -859,51 +900,51 @@ int pvnet_conv_fwd(const pvnet_conv* c, void* stream) {
             case 3: hipLaunchKernelGGL((k_conv_pw<3>), gp, dim3(256), 0, st, *c, (int)M); break;
             default: hipLaunchKernelGGL((k_conv_pw<4>), gp, dim3(256), 0, st, *c, (int)M); break;
         }
-    } else if (c->cout <= 16 && M >= (int64_t)256 * 2048) {
-        hipLaunchKernelGGL((k_conv_fwd<16, 64>), dim3(blocks_for(M, 256), 1), dim3(256), 0, st, *c, (int)M, K);
-    } else if (c->cout <= 16) {
-        hipLaunchKernelGGL((k_conv_fwd<16, 32>), dim3(mt, 1), dim3(256), 0, st, *c, (int)M, K);
-    } else if (c->cout % 64 == 0 && (int64_t)mt * (c->cout / 64) >= 2048) {
-        hipLaunchKernelGGL((k_conv_fwd<64, 32>), dim3(mt, c->cout / 64), dim3(256), 0, st, *c, (int)M, K);
+    } else if (parts) {
+        conv_gather<true>(*c, pq, M, st);
     } else {
-        hipLaunchKernelGGL((k_conv_fwd<32, 32>), dim3(mt, (c->cout + 31) / 32), dim3(256), 0, st, *c, (int)M, K);
+        conv_gather<false>(*c, pq, M, st);
     }
     NET_LAUNCH();
     return 0;
 }
 
-int64_t pvnet_wgrad_ws_floats(const pvnet_shape* s, int32_t ntaps, int32_t cin, int32_t cout) {
-    if (!shape_ok(s) || cin <= 0 || cout <= 0) return -1;
-    // either kernel's partials fit (the call's flags pick one)
-    return std::max(plan_wgrad(*s, ntaps, cin, cout, 0).ws_total, plan_wgrad(*s, ntaps, cin, cout, PVNET_GATHER).ws_total);
+template <bool PARTS>
+void wgrad_gather(const pvnet_wgrad& a, const NetParts& pq, const WgradPlan& p, int64_t M, hipStream_t st) {
+    const int K = a.ntaps * a.cin;
+    const dim3 grid(p.ktiles, p.ntiles, p.nsplit);
+    if (p.bn == 16)
+        hipLaunchKernelGGL((k_conv_wgrad<16, PARTS>), grid, dim3(256), 0, st, a, (int)M, K, p.mchunk, pq);
+    else if (p.bn == 32)
+        hipLaunchKernelGGL((k_conv_wgrad<32, PARTS>), grid, dim3(256), 0, st, a, (int)M, K, p.mchunk, pq);
+    else
+        hipLaunchKernelGGL((k_conv_wgrad<64, PARTS>), grid, dim3(256), 0, st, a, (int)M, K, p.mchunk, pq);
 }
 
-int pvnet_conv_wgrad(const pvnet_wgrad* a, void* stream) {
-    if (!a || !shape_ok(&a->s)) return fail(1, "pvnet_conv_wgrad: bad shape");
-    if (a->ntaps != 1 && a->ntaps != 27) return fail(1, "pvnet_conv_wgrad: ntaps must be 1 or 27");
+int wgrad_launch(const pvnet_wgrad* a, const NetParts& pq, void* stream, const std::string& who) {
+    if (!a || !shape_ok(&a->s)) return fail(1, who + ": bad shape");
+    if (a->ntaps != 1 && a->ntaps != 27) return fail(1, who + ": ntaps must be 1 or 27");
     if (a->cin <= 0 || a->cin % 8 || a->cout <= 0 || a->cout % 8)
-        return fail(1, "pvnet_conv_wgrad: cin and cout must be positive multiples of 8");
-    if (a->ldx < a->cin || a->ldx % 8 || a->lddy < a->cout || a->lddy % 8) return fail(1, "pvnet_conv_wgrad: bad row lengths");
+        return fail(1, who + ": cin and cout must be positive multiples of 8");
+    if (a->ldx < a->cin - pq.cup || a->ldx % 8 || a->lddy < a->cout || a->lddy % 8) return fail(1, who + ": bad row lengths");
     if (!a->x || !a->dy || !a->ws || !a->dw || !al16(a->x) || !al16(a->dy))
-        return fail(1, "pvnet_conv_wgrad: null or misaligned pointer");
+        return fail(1, who + ": null or misaligned pointer");
     const int64_t M = voxels(a->s);
-    if (M % 32) return fail(1, "pvnet_conv_wgrad: voxel count must be a multiple of 32");
-    if (M >= (int64_t)1 << 31) return fail(1, "pvnet_conv_wgrad: too many voxels");
-    if (a->db && a->cout > 256) return fail(1, "pvnet_conv_wgrad: bias gradient needs cout <= 256");
+    if (M % 32) return fail(1, who + ": voxel count must be a multiple of 32");
+    if (M >= (int64_t)1 << 31) return fail(1, who + ": too many voxels");
+    if (a->db && a->cout > 256) return fail(1, who + ": bias gradient needs cout <= 256");
     hipStream_t st = (hipStream_t)stream;
-    const WgradPlan p = plan_wgrad(a->s, a->ntaps, a->cin, a->cout, a->flags | (wgrad_march_ok(*a) ? 0 : PVNET_GATHER));
+    const WgradPlan p = plan_wgrad(a->s, a->ntaps, a->cin, a->cout, a->flags | (wgrad_march_ok(*a, pq) ? 0 : PVNET_GATHER));
     const int K = a->ntaps * a->cin;
-    dim3 grid(p.ktiles, p.ntiles, p.nsplit);
     const bool fused_db = a->db && p.march;  // the bias sums come with the weights'
     if (p.march) {
-        hipLaunchKernelGGL(wgrad_march_kernel(p.mp), dim3(p.mp.splits * p.mp.ns * p.mp.nf), dim3(256), p.mp.lds, st, *a, p.mp,
+        hipLaunchKernelGGL(wgrad_march_kernel(p.mp), dim3(p.mp.splits * p.mp.ns * p.mp.nf), dim3(256), p.mp.lds, st, *a, p.mp, pq,
                            fused_db ? p.ws_main : (int64_t)-1);
-    } else if (p.bn == 16)
-        hipLaunchKernelGGL(k_conv_wgrad<16>, grid, dim3(256), 0, st, *a, (int)M, K, p.mchunk);
-    else if (p.bn == 32)
-        hipLaunchKernelGGL(k_conv_wgrad<32>, grid, dim3(256), 0, st, *a, (int)M, K, p.mchunk);
-    else
-        hipLaunchKernelGGL(k_conv_wgrad<64>, grid, dim3(256), 0, st, *a, (int)M, K, p.mchunk);
+    } else if (pq.cup) {
+        wgrad_gather<true>(*a, pq, p, M, st);
+    } else {
+        wgrad_gather<false>(*a, pq, p, M, st);
+    }
     NET_LAUNCH();
     const int64_t len = (int64_t)a->cout * K;
     const SumJob jw{a->ws, a->dw, len, (int64_t)K, (int64_t)K, p.nsplit, (int)blocks_for(len, SUM_COLS)};
@@ -923,6 +964,47 @@ int pvnet_conv_wgrad(const pvnet_wgrad* a, void* stream) {
     hipLaunchKernelGGL(k_sum_splits, dim3(jw.blocks + jb.blocks), dim3(256), 0, st, jw, jb);
     NET_LAUNCH();
     return 0;
+}
+
+int up_args(const pvnet_shape* s, int ntaps, int cin, const void* up, int ldu, int cup, const std::string& who) {
+    if (!shape_ok(s) || s->d % 2 || s->h % 2 || s->w % 2) return fail(1, who + ": sizes must be even");
+    if (ntaps != 27 || cup <= 0 || cup % 8 || cup >= cin || ldu < cup || ldu % 8 || !up || !al16(up))
+        return fail(1, who + ": bad upsampled part");
+    return 0;
+}
+
+}  // namespace
+
+extern "C" {
+
+const char* pvnet_last_error(void) { return g_err.c_str(); }
+
+int pvnet_conv_fwd(const pvnet_conv* c, void* stream) { return conv_launch(c, NetParts{}, stream, "pvnet_conv_fwd"); }
+
+int pvnet_conv_up_fwd(const pvnet_conv* c, const uint16_t* up, int32_t ldu, int32_t cup, void* stream) {
+    if (int rc = up_args(c ? &c->s : nullptr, c ? c->ntaps : 0, c ? c->cin : 0, up, ldu, cup, "pvnet_conv_up_fwd")) return rc;
+    if (c->flags & PVNET_F32OUT) return fail(1, "pvnet_conv_up_fwd: bf16 output only");
+    return conv_launch(c, NetParts{up, nullptr, ldu, cup, 0, 0}, stream, "pvnet_conv_up_fwd");
+}
+
+int pvnet_conv_split_fwd(const pvnet_conv* c, uint16_t* y0, int32_t ldy0, int32_t c0, void* stream) {
+    if (!c || c->ntaps != 27 || !y0 || c0 <= 0 || c0 >= c->cout || c0 % 8 || c->cout % 8 || ldy0 < c0)
+        return fail(1, "pvnet_conv_split_fwd: bad argument");
+    if (c->flags & PVNET_F32OUT) return fail(1, "pvnet_conv_split_fwd: bf16 output only");
+    return conv_launch(c, NetParts{nullptr, y0, 0, 0, ldy0, c0}, stream, "pvnet_conv_split_fwd");
+}
+
+int64_t pvnet_wgrad_ws_floats(const pvnet_shape* s, int32_t ntaps, int32_t cin, int32_t cout) {
+    if (!shape_ok(s) || cin <= 0 || cout <= 0) return -1;
+    // either kernel's partials fit (the call's flags pick one)
+    return std::max(plan_wgrad(*s, ntaps, cin, cout, 0).ws_total, plan_wgrad(*s, ntaps, cin, cout, PVNET_GATHER).ws_total);
+}
+
+int pvnet_conv_wgrad(const pvnet_wgrad* a, void* stream) { return wgrad_launch(a, NetParts{}, stream, "pvnet_conv_wgrad"); }
+
+int pvnet_conv_up_wgrad(const pvnet_wgrad* a, const uint16_t* up, int32_t ldu, int32_t cup, void* stream) {
+    if (int rc = up_args(a ? &a->s : nullptr, a ? a->ntaps : 0, a ? a->cin : 0, up, ldu, cup, "pvnet_conv_up_wgrad")) return rc;
+    return wgrad_launch(a, NetParts{up, nullptr, ldu, cup, 0, 0}, stream, "pvnet_conv_up_wgrad");
 }
 
 int pvnet_pack_weights(const float* w32, int32_t ntaps, int32_t cin, int32_t cout, uint16_t* wt, uint16_t* wd,
@@ -980,7 +1062,19 @@ int pvnet_up2_bwd(const pvnet_shape* s, int32_t c, const uint16_t* dy, int32_t l
                   void* stream) {
     if (int rc = pool_args(s, c, dy, lddy, dx, lddx, "pvnet_up2_bwd")) return rc;
     const int64_t n = voxels(*s) / 8 * (c / 8);
-    hipLaunchKernelGGL(k_up2_bwd, dim3(blocks_for(n, 256)), dim3(256), 0, (hipStream_t)stream, *s, c, dy, lddy, dx, lddx);
+    hipLaunchKernelGGL(k_up2_bwd, dim3(blocks_for(n, 256)), dim3(256), 0, (hipStream_t)stream, *s, c, dy, lddy, dx, lddx,
+                       (const uint16_t*)nullptr, 0);
+    NET_LAUNCH();
+    return 0;
+}
+
+int pvnet_up2_bwd_relu(const pvnet_shape* s, int32_t c, const uint16_t* dy, int32_t lddy, uint16_t* dx, int32_t lddx,
+                       const uint16_t* relu_of, int32_t ldr, void* stream) {
+    if (int rc = pool_args(s, c, dy, lddy, dx, lddx, "pvnet_up2_bwd_relu")) return rc;
+    if (!relu_of || !al16(relu_of) || ldr < c || ldr % 8) return fail(1, "pvnet_up2_bwd_relu: bad relu_of");
+    const int64_t n = voxels(*s) / 8 * (c / 8);
+    hipLaunchKernelGGL(k_up2_bwd, dim3(blocks_for(n, 256)), dim3(256), 0, (hipStream_t)stream, *s, c, dy, lddy, dx, lddx,
+                       relu_of, ldr);
     NET_LAUNCH();
     return 0;
 }

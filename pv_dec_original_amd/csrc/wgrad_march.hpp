@@ -40,7 +40,8 @@ __device__ __forceinline__ uint2 tr_read(const char* lds) {
 }
 
 template <int CF>
-__global__ __launch_bounds__(256, 3) void k_wgrad_march(const pvnet_wgrad a, const WgradMarch p, const int64_t dboff) {
+__global__ __launch_bounds__(256, 3) void k_wgrad_march(const pvnet_wgrad a, const WgradMarch p, const NetParts q,
+                                                        const int64_t dboff) {
     extern __shared__ uint4 wm_sm[];
     const int t = threadIdx.x, lane = t & 63, g = lane >> 4, c16 = lane & 15;
     const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -86,36 +87,38 @@ __global__ __launch_bounds__(256, 3) void k_wgrad_march(const pvnet_wgrad a, con
         const int64_t box = r / p.nty;
         const int z0 = zq * p.zseg, z1 = min(d, z0 + p.zseg);
         __syncthreads();  // the previous run is done with the LDS
-        // element offset of every unit within its plane (-1: zero)
+        // element offset of every unit within its plane (-1: zero; bit 0: x's half-size part, as in conv_march)
         for (int i = t; i < nuS; i += 256) {
             const int v = i >> 1, ch = s0 + 8 * (i & 1);
             const int hy = v / p.hx, x = x0 - 1 + v - hy * p.hx, y = y0 - 1 + hy;
             soS[i] = (unsigned)x < (unsigned)w && (unsigned)y < (unsigned)h && ch < a.cout ? (y * w + x) * a.lddy + ch : -1;
         }
         for (int i = t; i < nuF; i += 256) {
-            const int cp = i / (2 * sl32), q = i - cp * 2 * sl32, v = q >> 1, ch = f0 + 16 * cp + 8 * (q & 1);
-            const int yy = v / p.tx;
-            soF[i] = v < vox && ch < a.cin ? ((y0 + yy) * w + x0 + v - yy * p.tx) * a.ldx + ch : -1;
+            const int cp = i / (2 * sl32), k = i - cp * 2 * sl32, v = k >> 1, ch = f0 + 16 * cp + 8 * (k & 1);
+            const int yy = v / p.tx, y = y0 + yy, x = x0 + v - yy * p.tx;
+            soF[i] = v >= vox || ch >= a.cin ? -1 : ch < q.cup ? ((y >> 1) * (w >> 1) + (x >> 1)) * q.ldu + ch + 1
+                                                               : (y * w + x) * a.ldx + ch - q.cup;
         }
         __syncthreads();
-        auto stage = [&](const uint16_t* base, int ld, int z, const int* so, int nu, uint32_t lds) {
+        auto stage = [&](const uint16_t* base, int ld, int z, const int* so, int nu, uint32_t lds, bool parts) {
             const bool zin = (unsigned)z < (unsigned)d;
             const uint16_t* pb = base + (box * d + (zin ? z : 0)) * ((int64_t)h * w) * ld;
+            const uint16_t* pu = parts && q.cup ? q.up + (box * (d >> 1) + (z >> 1)) * ((int64_t)(h >> 1) * (w >> 1)) * q.ldu - 1 : pb;
             for (int i = 64 * wv; i < nu; i += 256)
                 if (i + lane < nu) {
                     const int o = so[i + lane];
-                    lds_copy16(zin && o >= 0 ? (const void*)(pb + o) : (const void*)g_march_zero,
+                    lds_copy16(zin && o >= 0 ? (const void*)((o & 1 ? pu : pb) + o) : (const void*)g_march_zero,
                                __builtin_amdgcn_readfirstlane(lds + 16u * (uint32_t)i));
                 }
         };
-        for (int z = z0 - 1; z <= z0 + 1; z++) stage(a.dy, a.lddy, z, soS, nuS, ldsS + 16u * (uint32_t)((z & 3) * p.su));
-        stage(a.x, a.ldx, z0, soF, nuF, ldsF + 16u * (uint32_t)((z0 & 1) * p.fu));
+        for (int z = z0 - 1; z <= z0 + 1; z++) stage(a.dy, a.lddy, z, soS, nuS, ldsS + 16u * (uint32_t)((z & 3) * p.su), false);
+        stage(a.x, a.ldx, z0, soF, nuF, ldsF + 16u * (uint32_t)((z0 & 1) * p.fu), true);
         march_wait();
         march_barrier();
         for (int z = z0; z < z1; z++) {
             if (z + 1 < z1) {
-                stage(a.dy, a.lddy, z + 2, soS, nuS, ldsS + 16u * (uint32_t)(((z + 2) & 3) * p.su));
-                stage(a.x, a.ldx, z + 1, soF, nuF, ldsF + 16u * (uint32_t)(((z + 1) & 1) * p.fu));
+                stage(a.dy, a.lddy, z + 2, soS, nuS, ldsS + 16u * (uint32_t)(((z + 2) & 3) * p.su), false);
+                stage(a.x, a.ldx, z + 1, soF, nuF, ldsF + 16u * (uint32_t)(((z + 1) & 1) * p.fu), true);
             }
             int toff[7];  // byte offset of each shift from a voxel's own unit, wave-uniform
 #pragma unroll
@@ -186,7 +189,7 @@ __global__ __launch_bounds__(256, 3) void k_wgrad_march(const pvnet_wgrad a, con
             if (s0 + 4 * g + e < a.cout) a.ws[dboff + (int64_t)split * a.cout + s0 + 4 * g + e] = accb[e];
 }
 
-typedef void (*WgradKernel)(const pvnet_wgrad, const WgradMarch, const int64_t);
+typedef void (*WgradKernel)(const pvnet_wgrad, const WgradMarch, const NetParts, const int64_t);
 
 inline WgradKernel wgrad_march_kernel(const WgradMarch& p) {
     return p.cf == 1 ? k_wgrad_march<1> : p.cf == 2 ? k_wgrad_march<2> : k_wgrad_march<3>;
@@ -245,6 +248,6 @@ inline bool wgrad_march_plan(const pvnet_shape& s, int cin, int cout, WgradMarch
 
 // What one call needs beyond a plan: plane offsets fit 32 bits (as in conv_march, PVNET_GATHER and pointwise
 // layers stay on k_conv_wgrad)
-inline bool wgrad_march_ok(const pvnet_wgrad& a) {
-    return (int64_t)a.s.h * a.s.w * std::max(a.ldx, a.lddy) < (int64_t)1 << 31;
+inline bool wgrad_march_ok(const pvnet_wgrad& a, const NetParts& q) {
+    return (int64_t)a.s.h * a.s.w * std::max(std::max(a.ldx, a.lddy), q.ldu) < (int64_t)1 << 31;
 }

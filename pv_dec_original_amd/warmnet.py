@@ -190,9 +190,9 @@ class UNet:
              "dist": torch.zeros(M[0], dtype=torch.float32, device=dev),
              "dY": bf(M[0], OUT_CH)}
         for k in range(L - 1):
-            ccat = lv[k + 1] + lv[k]
             b[f"A{k}"], b[f"dA{k}"] = bf(M[k], lv[k]), bf(M[k], lv[k])
-            b[f"CAT{k}"], b[f"dCAT{k}"] = bf(M[k], ccat), bf(M[k], ccat)
+            # skip and its gradient; the upsampled half of the concatenation exists only as its gradient
+            b[f"S{k}"], b[f"dS{k}"], b[f"dUP{k}"] = bf(M[k], lv[k]), bf(M[k], lv[k]), bf(M[k], lv[k + 1])
             b[f"DA{k}"], b[f"dDA{k}"] = bf(M[k], lv[k]), bf(M[k], lv[k])
             b[f"DEC{k}"], b[f"dDEC{k}"] = bf(M[k], lv[k]), bf(M[k], lv[k])
             b[f"P{k + 1}"], b[f"dP{k + 1}"] = bf(M[k + 1], lv[k]), bf(M[k + 1], lv[k])
@@ -217,24 +217,33 @@ class UNet:
             return L - 1
         return int(n[1:-1])
 
-    def _conv(self, lay, s, x, ldx, y, ldy, relu=None, f32=False, bias=True, xoff=0, yoff=0):
+    def _conv(self, lay, s, x, ldx, y, ldy, relu=None, f32=False, bias=True, up=None):
         flags = (N.NET_RELU if (lay.relu if relu is None else relu) else 0) | (N.NET_F32OUT if f32 else 0)
-        c = N.NetConv(s, lay.ntaps, lay.cin, lay.cout, lay.kpad, _ptr(x, xoff), ldx, flags,
+        c = N.NetConv(s, lay.ntaps, lay.cin, lay.cout, lay.kpad, _ptr(x), ldx, flags,
                       _ptr(self.wt[lay.name]), _ptr(self.p, lay.boff) if bias else None,
-                      _ptr(y, yoff), ldy, 0, None)
-        N.net_check(N.net().pvnet_conv_fwd(C.byref(c), self._st()))
+                      _ptr(y), ldy, 0, None)
+        if up is None:
+            N.net_check(N.net().pvnet_conv_fwd(C.byref(c), self._st()))
+        else:  # channels in front of x's: (half-size tensor, channels)
+            N.net_check(N.net().pvnet_conv_up_fwd(C.byref(c), _ptr(up[0]), up[1], up[1], self._st()))
 
-    def _dgrad(self, lay, s, dy, lddy, dx, lddx, relu_of=None, ldr=0, dyoff=0, roff=0):
-        c = N.NetConv(s, lay.ntaps, lay.cout, lay.cin, lay.kpad_d, _ptr(dy, dyoff), lddy, 0,
+    def _dgrad(self, lay, s, dy, lddy, dx, lddx, relu_of=None, ldr=0, first=None):
+        c = N.NetConv(s, lay.ntaps, lay.cout, lay.cin, lay.kpad_d, _ptr(dy), lddy, 0,
                       _ptr(self.wd[lay.name]), None, _ptr(dx), lddx, ldr,
-                      _ptr(relu_of, roff) if relu_of is not None else None)
-        N.net_check(N.net().pvnet_conv_fwd(C.byref(c), self._st()))
+                      _ptr(relu_of) if relu_of is not None else None)
+        if first is None:
+            N.net_check(N.net().pvnet_conv_fwd(C.byref(c), self._st()))
+        else:  # the first channels go to a tensor of their own: (tensor, channels)
+            N.net_check(N.net().pvnet_conv_split_fwd(C.byref(c), _ptr(first[0]), first[1], first[1], self._st()))
 
-    def _wgrad(self, lay, s, x, ldx, dy, lddy, xoff=0, dyoff=0):
+    def _wgrad(self, lay, s, x, ldx, dy, lddy, up=None):
         b = self._bufs
-        g = N.NetWgrad(s, lay.ntaps, lay.cin, lay.cout, _ptr(x, xoff), ldx, lddy, _ptr(dy, dyoff),
+        g = N.NetWgrad(s, lay.ntaps, lay.cin, lay.cout, _ptr(x), ldx, lddy, _ptr(dy),
                        _ptr(b["ws"]), _ptr(self.g, lay.offset), _ptr(self.g, lay.boff))
-        N.net_check(N.net().pvnet_conv_wgrad(C.byref(g), self._st()))
+        if up is None:
+            N.net_check(N.net().pvnet_conv_wgrad(C.byref(g), self._st()))
+        else:
+            N.net_check(N.net().pvnet_conv_up_wgrad(C.byref(g), _ptr(up[0]), up[1], up[1], self._st()))
 
     # -- forward / backward -----------------------------------------------------------------
 
@@ -253,19 +262,16 @@ class UNet:
                                       self._st()))
         x, ldx = b["X0"], IN_CH
         for k in range(L - 1):
-            ccat = lv[k + 1] + lv[k]
             self._conv(by[f"e{k}a"], S[k], x, ldx, b[f"A{k}"], lv[k])
-            self._conv(by[f"e{k}b"], S[k], b[f"A{k}"], lv[k], b[f"CAT{k}"], ccat, yoff=lv[k + 1])
-            N.net_check(NL.pvnet_pool2_fwd(C.byref(S[k]), lv[k], _ptr(b[f"CAT{k}"], lv[k + 1]), ccat,
+            self._conv(by[f"e{k}b"], S[k], b[f"A{k}"], lv[k], b[f"S{k}"], lv[k])
+            N.net_check(NL.pvnet_pool2_fwd(C.byref(S[k]), lv[k], _ptr(b[f"S{k}"]), lv[k],
                                            _ptr(b[f"P{k + 1}"]), lv[k], self._st()))
             x, ldx = b[f"P{k + 1}"], lv[k]
         self._conv(by["bta"], S[L - 1], x, ldx, b["BA"], lv[L - 1])
         self._conv(by["btb"], S[L - 1], b["BA"], lv[L - 1], b[f"DEC{L - 1}"], lv[L - 1])
         for k in range(L - 2, -1, -1):
-            ccat = lv[k + 1] + lv[k]
-            N.net_check(NL.pvnet_up2_fwd(C.byref(S[k]), lv[k + 1], _ptr(b[f"DEC{k + 1}"]), lv[k + 1],
-                                         _ptr(b[f"CAT{k}"]), ccat, self._st()))
-            self._conv(by[f"d{k}a"], S[k], b[f"CAT{k}"], ccat, b[f"DA{k}"], lv[k])
+            self._conv(by[f"d{k}a"], S[k], b[f"S{k}"], lv[k], b[f"DA{k}"], lv[k],
+                       up=(b[f"DEC{k + 1}"], lv[k + 1]))
             self._conv(by[f"d{k}b"], S[k], b[f"DA{k}"], lv[k], b[f"DEC{k}"], lv[k])
         self._conv(by["head"], S[0], b["DEC0"], lv[0], b["Y"], OUT_CH, f32=True)
         return b["Y"]
@@ -293,16 +299,14 @@ class UNet:
         self._wgrad(head, S[0], b["DEC0"], lv[0], b["dY"], OUT_CH)
         self._dgrad(head, S[0], b["dY"], OUT_CH, b["dDEC0"], lv[0], relu_of=b["DEC0"], ldr=lv[0])
         for k in range(L - 1):
-            ccat = lv[k + 1] + lv[k]
             la, lb = by[f"d{k}a"], by[f"d{k}b"]
             self._wgrad(lb, S[k], b[f"DA{k}"], lv[k], b[f"dDEC{k}"], lv[k])
             self._dgrad(lb, S[k], b[f"dDEC{k}"], lv[k], b[f"dDA{k}"], lv[k], relu_of=b[f"DA{k}"], ldr=lv[k])
-            self._wgrad(la, S[k], b[f"CAT{k}"], ccat, b[f"dDA{k}"], lv[k])
-            self._dgrad(la, S[k], b[f"dDA{k}"], lv[k], b[f"dCAT{k}"], ccat)
-            N.net_check(NL.pvnet_up2_bwd(C.byref(S[k]), lv[k + 1], _ptr(b[f"dCAT{k}"]), ccat,
-                                         _ptr(b[f"dDEC{k + 1}"]), lv[k + 1], self._st()))
-            N.net_check(NL.pvnet_relu_bwd(b["M"][k + 1], lv[k + 1], _ptr(b[f"DEC{k + 1}"]), lv[k + 1],
-                                          _ptr(b[f"dDEC{k + 1}"]), lv[k + 1], self._st()))
+            self._wgrad(la, S[k], b[f"S{k}"], lv[k], b[f"dDA{k}"], lv[k], up=(b[f"DEC{k + 1}"], lv[k + 1]))
+            self._dgrad(la, S[k], b[f"dDA{k}"], lv[k], b[f"dS{k}"], lv[k], first=(b[f"dUP{k}"], lv[k + 1]))
+            N.net_check(NL.pvnet_up2_bwd_relu(C.byref(S[k]), lv[k + 1], _ptr(b[f"dUP{k}"]), lv[k + 1],
+                                              _ptr(b[f"dDEC{k + 1}"]), lv[k + 1], _ptr(b[f"DEC{k + 1}"]),
+                                              lv[k + 1], self._st()))
         ta, tb = by["bta"], by["btb"]
         top = L - 1
         self._wgrad(tb, S[top], b["BA"], lv[top], b[f"dDEC{top}"], lv[top])
@@ -311,14 +315,11 @@ class UNet:
         self._wgrad(ta, S[top], xin, lv[top - 1], b["dBA"], lv[top])
         self._dgrad(ta, S[top], b["dBA"], lv[top], b[f"dP{top}"], lv[top - 1])
         for k in range(L - 2, -1, -1):
-            ccat = lv[k + 1] + lv[k]
             ea, eb = by[f"e{k}a"], by[f"e{k}b"]
             N.net_check(NL.pvnet_pool2_bwd_relu(C.byref(S[k]), lv[k], _ptr(b[f"dP{k + 1}"]), lv[k],
-                                                _ptr(b[f"dCAT{k}"], lv[k + 1]), ccat, _ptr(b[f"CAT{k}"], lv[k + 1]),
-                                                ccat, self._st()))
-            self._wgrad(eb, S[k], b[f"A{k}"], lv[k], b[f"dCAT{k}"], ccat, dyoff=lv[k + 1])
-            self._dgrad(eb, S[k], b[f"dCAT{k}"], ccat, b[f"dA{k}"], lv[k], relu_of=b[f"A{k}"], ldr=lv[k],
-                        dyoff=lv[k + 1])
+                                                _ptr(b[f"dS{k}"]), lv[k], _ptr(b[f"S{k}"]), lv[k], self._st()))
+            self._wgrad(eb, S[k], b[f"A{k}"], lv[k], b[f"dS{k}"], lv[k])
+            self._dgrad(eb, S[k], b[f"dS{k}"], lv[k], b[f"dA{k}"], lv[k], relu_of=b[f"A{k}"], ldr=lv[k])
             xk, ldk = (b["X0"], IN_CH) if k == 0 else (b[f"P{k}"], lv[k - 1])
             self._wgrad(ea, S[k], xk, ldk, b[f"dA{k}"], lv[k])
             if k > 0:

@@ -314,6 +314,9 @@ int pvlbm_iteration(pvlbm_handle h, int64_t* it);
  * the populations after iteration n-1 (Simulation.cpp:52-105).  Dense box arrays; u holds three
  * planes.  Solid points get 0.  Either pointer may be NULL. */
 int pvlbm_get_macros(pvlbm_handle h, double* rho, double* u);
+/* The same for the nodes alone: points that are not nodes are left as they are (arrays that are zero
+ * already, or a field of the same handle to be brought up to date, need no second pass). */
+int pvlbm_fill_macros(pvlbm_handle h, double* rho, double* u);
 
 /* The same fields as FP32 into caller-owned device memory on this handle's device: rho[nbox],
  * u[3][nbox] (dense box order); points that are not nodes get rho = 1, u = 0, so the arrays can

@@ -112,6 +112,7 @@ PVLBM_API = [
     ("pvlbm_step_timed", C.c_int, [C.c_void_p, C.c_int, _d, _d]),
     ("pvlbm_iteration", C.c_int, [C.c_void_p, _i64]),
     ("pvlbm_get_macros", C.c_int, [C.c_void_p, _d, _d]),
+    ("pvlbm_fill_macros", C.c_int, [C.c_void_p, _d, _d]),
     ("pvlbm_get_macros_device", C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p]),
     ("pvlbm_get_wss", C.c_int, [C.c_void_p, _d]),
     ("pvlbm_get_normals", C.c_int, [C.c_void_p, _d]),

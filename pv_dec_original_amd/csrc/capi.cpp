@@ -98,6 +98,8 @@ double nudge(double v, double lo, double hi) {
 // The simulation handle
 // =============================================================================================
 
+constexpr int32_t GATHER_TILES = 512;  // tiles of one group of a read-out: at most 1 MB of node values
+
 struct pvlbm_sim {
     std::string err;
     hipStream_t stream = nullptr;
@@ -131,6 +133,11 @@ struct pvlbm_sim {
     double* d_macro = nullptr;
     double* d_partials = nullptr;
     double* d_red = nullptr;
+    // node values on their way to the host, in two halves of GATHER_TILES tiles each: device, pinned host and the
+    // events of the copies, allocated by the first read-out; position of each group's first node, and their number
+    double *d_gather = nullptr, *h_gather = nullptr;
+    hipEvent_t ev_gather[2] = {nullptr, nullptr};
+    std::vector<int32_t> gather_first;
     double* d_expand = nullptr;  // scratch of a start from a coarse field, allocated by the first one
     unsigned long long* d_gate = nullptr;
     // host copy of the triangles (link fractions), boundary slots (padded node, closure)
@@ -189,8 +196,11 @@ struct pvlbm_sim {
     ~pvlbm_sim() {
         if (stream) (void)hipStreamSynchronize(stream);
         void* ptrs[] = {d_bq, d_kind, d_aux, d_tdesc, d_pop[0], d_pop[1], d_bmask, d_bclose, d_bprof, d_brho,
-                        d_M, d_nrm, d_wss, d_tau3, d_acc, d_macro, d_partials, d_red, d_expand, d_gate};
+                        d_M, d_nrm, d_wss, d_tau3, d_acc, d_macro, d_partials, d_red, d_expand, d_gather, d_gate};
         for (void* p : ptrs) dfree(p);
+        if (h_gather) (void)hipHostFree(h_gather);
+        for (hipEvent_t e : ev_gather)
+            if (e) (void)hipEventDestroy(e);
         if (ev0) (void)hipEventDestroy(ev0);
         if (ev1) (void)hipEventDestroy(ev1);
         if (stream) (void)hipStreamDestroy(stream);
@@ -252,6 +262,44 @@ struct pvlbm_sim {
     double* ensure_expand() {
         if (!d_expand) d_expand = dalloc<double>((size_t)expand_coarse_doubles(nx, nxp, ntiles));
         return d_expand;
+    }
+
+    void ensure_gather() {
+        if (!d_gather) d_gather = dalloc<double>((size_t)2 * GATHER_TILES * 64 * 4);
+        if (!h_gather) HIPCHK(hipHostMalloc((void**)&h_gather, sizeof(double) * 2 * GATHER_TILES * 64 * 4, hipHostMallocDefault));
+        for (hipEvent_t& e : ev_gather)
+            if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    }
+
+    // Density and velocity of the nodes into dense box arrays; other points are left alone.  Groups of tiles are
+    // gathered on the device and copied while the group before is put in place, so the host reads and writes the
+    // nodes and not the box (a vessel of 96^3 points, 250 steps and this: 3.9 ms, 14.3 with the padded planes
+    // copied whole into a fresh buffer).  One megabyte a group: long enough a copy for the link, and still in the host's cache when read.
+    void fill_macros(double* rho, double* u) {
+        const int32_t groups = (ntiles + GATHER_TILES - 1) / GATHER_TILES;
+        if (groups == 0) return;
+        ensure_gather();
+        const int64_t nbox = nx * ny * nz, half = (int64_t)GATHER_TILES * 64 * 4;
+        auto start = [&](int32_t gi) {
+            const int32_t t0 = gi * GATHER_TILES, cnt = gather_first[gi + 1] - gather_first[gi];
+            double* d = d_gather + (gi & 1) * half;
+            HIPCHK(launch_macros_nodes(d_macro, ns, d_tdesc, t0, std::min(GATHER_TILES, ntiles - t0), d, stream));
+            HIPCHK(hipMemcpyAsync(h_gather + (gi & 1) * half, d, sizeof(double) * 4 * cnt, hipMemcpyDeviceToHost, stream));
+            HIPCHK(hipEventRecord(ev_gather[gi & 1], stream));
+        };
+        start(0);
+        for (int32_t gi = 0; gi < groups; gi++) {
+            HIPCHK(hipEventSynchronize(ev_gather[gi & 1]));
+            if (gi + 1 < groups) start(gi + 1);
+            const double* v = h_gather + (gi & 1) * half;
+            const int64_t* box = lists[PVLBM_LIST_FLUID].data() + gather_first[gi];
+            const int32_t cnt = gather_first[gi + 1] - gather_first[gi];
+            for (int32_t i = 0; i < cnt; i++) {
+                const int64_t b = box[i];
+                if (rho) rho[b] = v[4 * i];
+                if (u) u[b] = v[4 * i + 1], u[nbox + b] = v[4 * i + 2], u[2 * nbox + b] = v[4 * i + 3];
+            }
+        }
     }
 
     // Brings the state into the layout of the scheme in use (values only move: fields unchanged).
@@ -772,18 +820,20 @@ extern "C" int pvlbm_create(const uint8_t* fluid, const pvlbm_grid* grid, double
         // tile descriptors: lane masks and first side-table slots (slots follow node order)
         std::vector<TileDesc> tdesc(tiles.size());
         {
-            int32_t bs = 0, wsl = 0;
+            int32_t bs = 0, wsl = 0, nodes = 0;
             for (size_t ti = 0; ti < tiles.size(); ti++) {
                 TileDesc& D = tdesc[ti];
                 D.tile = tiles[ti];
                 D.bslot = bs;
                 D.wslot = wsl;
-                D.pad = 0;
+                if (ti % GATHER_TILES == 0) S->gather_first.push_back(nodes);
+                D.first = nodes;
                 D.node = D.ntw = D.bnd = 0;
                 for (int l = 0; l < 64; l++) {
                     const uint8_t kd = kind[(size_t)tiles[ti] * 64 + l];
                     if (kd == K_SOLID) continue;
                     D.node |= 1ull << l;
+                    nodes++;
                     if (kd == K_NTW) {
                         D.ntw |= 1ull << l;
                         wsl++;
@@ -793,6 +843,7 @@ extern "C" int pvlbm_create(const uint8_t* fluid, const pvlbm_grid* grid, double
                     }
                 }
             }
+            S->gather_first.push_back(nodes);
             if (bs != S->nb || wsl != (int32_t)wnode.size()) fail(PVLBM_EINVAL, "internal: slot order mismatch");
             // cache footprint of one lattice: the 128-byte lines of a plane that hold a node, x Q
             const int per = (int)(128 / S->store_bytes());
@@ -1339,21 +1390,16 @@ extern "C" int pvlbm_iteration(pvlbm_handle h, int64_t* it) {
 extern "C" int pvlbm_get_macros(pvlbm_handle h, double* rho, double* u) {
     if (!h) return PVLBM_EINVAL;
     return guarded(h, [&] {
-        std::vector<double> m((size_t)(4 * h->ns));
-        HIPCHK(hipMemcpyAsync(m.data(), h->d_macro, sizeof(double) * m.size(), hipMemcpyDeviceToHost, h->stream));
-        HIPCHK(hipStreamSynchronize(h->stream));
-        std::vector<uint8_t> k((size_t)h->nsp);
-        HIPCHK(hipMemcpy(k.data(), h->d_kind, (size_t)h->nsp, hipMemcpyDeviceToHost));
         const int64_t nbox = h->nx * h->ny * h->nz;
-        for (int64_t r = 0; r < h->ny * h->nz; r++)
-            for (int64_t i = 0; i < h->nx; i++) {
-                const int64_t n = h->prow(r) * h->nxp + i, b = r * h->nx + i;
-                const bool node = k[n] != K_SOLID;
-                if (rho) rho[b] = node ? m[n] : 0.0;
-                if (u)
-                    for (int c = 0; c < 3; c++) u[c * nbox + b] = node ? m[(c + 1) * h->ns + n] : 0.0;
-            }
+        if (rho) std::memset(rho, 0, sizeof(double) * nbox);
+        if (u) std::memset(u, 0, sizeof(double) * 3 * nbox);
+        h->fill_macros(rho, u);
     });
+}
+
+extern "C" int pvlbm_fill_macros(pvlbm_handle h, double* rho, double* u) {
+    if (!h) return PVLBM_EINVAL;
+    return guarded(h, [&] { h->fill_macros(rho, u); });
 }
 
 extern "C" int pvlbm_get_macros_device(pvlbm_handle h, float* rho, float* u) {

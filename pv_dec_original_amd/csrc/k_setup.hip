@@ -638,6 +638,28 @@ hipError_t launch_macros_f32(const double* macro, const uint8_t* kind, int64_t n
     return hipGetLastError();
 }
 
+// One wave per tile.  Bound by the four loads of eight bytes a node; what counts is what is not moved: the planes
+// are the padded box, most of it without nodes.
+__global__ __launch_bounds__(256) void k_macros_nodes(const double* macro, int64_t ns, const TileDesc* tdesc, int32_t t0,
+                                                      int32_t nt, double* out) {
+    const int32_t t = (int32_t)blockIdx.x * 4 + (int32_t)(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (t >= nt) return;
+    const TileDesc& D = tdesc[t0 + t];
+    if (!((D.node >> lane) & 1)) return;
+    const int64_t n = (int64_t)D.tile * 64 + lane;
+    const int64_t i = D.first - tdesc[t0].first + __popcll(D.node & ((1ull << lane) - 1));
+    dvec2* o = reinterpret_cast<dvec2*>(out + 4 * i);
+    o[0] = dvec2{macro[n], macro[ns + n]};
+    o[1] = dvec2{macro[2 * ns + n], macro[3 * ns + n]};
+}
+
+hipError_t launch_macros_nodes(const double* macro, int64_t ns, const TileDesc* tdesc, int32_t t0, int32_t nt,
+                               double* out, hipStream_t s) {
+    if (nt <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_macros_nodes, dim3((unsigned)((nt + 3) / 4)), dim3(256), 0, s, macro, ns, tdesc, t0, nt, out);
+    return hipGetLastError();
+}
+
 // one thread per output point of a separable index grid
 __global__ void k_sample_kinds(const uint8_t* kind, int64_t nxp, int64_t nyp, const int32_t* ix, int nx,
                                const int32_t* iy, int ny, const int32_t* iz, int nz, uint8_t* out) {

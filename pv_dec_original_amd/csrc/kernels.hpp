@@ -33,7 +33,7 @@ struct alignas(16) TileDesc {
     int32_t tile;
     int32_t bslot;   // first boundary-table slot of the tile
     int32_t wslot;   // first next-to-wall-table slot of the tile
-    int32_t pad;
+    int32_t first;   // nodes in the tiles before: position of the tile's first node in node order
     uint64_t node;
     uint64_t ntw;
     uint64_t bnd;
@@ -154,6 +154,11 @@ hipError_t launch_expand_coarse(const float* rho_c, const float* u_c, int cx, in
 // rho = 1, u = 0.
 hipError_t launch_macros_f32(const double* macro, const uint8_t* kind, int64_t nx, int64_t ny, int64_t nz,
                              int64_t nxp, int64_t nyp, int64_t ns, float* rho, float* u, hipStream_t s);
+
+// The macro planes of the nodes of tiles t0 .. t0 + nt - 1 as FP64 records {rho, u0, u1, u2} in node
+// order: out[4 i] is the i-th of them (32-byte aligned, at most 64 nt records).
+hipError_t launch_macros_nodes(const double* macro, int64_t ns, const TileDesc* tdesc, int32_t t0, int32_t nt,
+                               double* out, hipStream_t s);
 
 // out[(k ny + j) nx + i] = kind of box point (ix[i], iy[j], iz[k]) (padded layout nxp x nyp);
 // the indices must lie in the box (device arrays).

@@ -341,7 +341,7 @@ class Simulation:
         sd = self.SubDomain_
         rho = np.zeros((sd.nz, sd.ny, sd.nx))
         u = np.zeros((3, sd.nz, sd.ny, sd.nx))
-        self._chk(N.lib().pvlbm_get_macros(self.handle, N.dptr(rho), N.dptr(u)))
+        self._chk(N.lib().pvlbm_fill_macros(self.handle, N.dptr(rho), N.dptr(u)))
         return rho, u
 
     def macros_device(self):

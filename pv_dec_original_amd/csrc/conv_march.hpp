@@ -41,13 +41,6 @@ struct MarchPlan {
 
 __device__ uint4 g_march_zero[4];  // source of the units outside the box
 
-// two floats to bf16, the first in the low half: the conversion instruction rounds as f2bf does (equal on
-// all 2^32 inputs, NaN included)
-__device__ __forceinline__ uint32_t f2bf_pk(float lo, float hi) {
-    const __bf16 v[2] = {(__bf16)lo, (__bf16)hi};
-    return *reinterpret_cast<const uint32_t*>(v);
-}
-
 // 16 bytes per lane from src to LDS byte address lds + 16 * lane.  Written as one asm statement because the
 // compiler would wait for the copy before the next LDS read; march_wait() is the wait, before the barrier
 // that hands the slot over.  No register waits for it (m0 is put back); the nop is the hazard between
@@ -548,12 +541,16 @@ bool kept_plan(const MarchKey& key, Plan& p, Search search) {
 
 inline bool march_plan(const pvnet_conv& c, MarchPlan& p) { return kept_plan<MarchPlan>(MarchKey{c.s, c.cin, c.cout}, p, march_search); }
 
+// outputs (and ReLU mask) that can be accessed four channels at a time
+inline bool rows_by_four(const pvnet_conv& c) {
+    if (c.cout % 4 || c.ldy % 4 || (uintptr_t)c.y % (c.flags & PVNET_F32OUT ? 16 : 8)) return false;
+    return !c.relu_of || (c.ldr % 4 == 0 && (uintptr_t)c.relu_of % 8 == 0);
+}
+
 // The marching kernels take 3x3x3 convolutions whose outputs (and ReLU mask) can be accessed four channels at a
 // time; PVNET_GATHER keeps k_conv_fwd.
 inline bool march_ok(const pvnet_conv& c, const NetParts& q) {
-    if (c.ntaps != 27 || (c.flags & PVNET_GATHER) || c.cout % 4 || c.ldy % 4) return false;
-    if ((uintptr_t)c.y % (c.flags & PVNET_F32OUT ? 16 : 8)) return false;
-    if (c.relu_of && (c.ldr % 4 || (uintptr_t)c.relu_of % 8)) return false;
+    if (c.ntaps != 27 || (c.flags & PVNET_GATHER) || !rows_by_four(c)) return false;
     if ((int64_t)c.s.h * c.s.w * c.ldx >= (int64_t)1 << 31) return false;  // plane offsets are 32-bit
     if ((int64_t)(c.s.h / 2) * (c.s.w / 2) * q.ldu >= (int64_t)1 << 31) return false;
     if (q.c0 && (q.ldy0 % 4 || (uintptr_t)q.y0 % 8)) return false;

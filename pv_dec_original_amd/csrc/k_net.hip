@@ -60,6 +60,13 @@ __device__ __forceinline__ uint16_t f2bf(float f) {
     return (uint16_t)(u >> 16);
 }
 
+// two floats to bf16, the first in the low half: the conversion instruction rounds as f2bf does (equal on
+// all 2^32 inputs, NaN included)
+__device__ __forceinline__ uint32_t f2bf_pk(float lo, float hi) {
+    const __bf16 v[2] = {(__bf16)lo, (__bf16)hi};
+    return *reinterpret_cast<const uint32_t*>(v);
+}
+
 // bf16 bit pattern strictly greater than zero (NaN is not)
 __device__ __forceinline__ bool bf_pos(uint16_t b) { return (b & 0x8000u) == 0 && b != 0 && b <= 0x7f80u; }
 
@@ -217,52 +224,76 @@ __global__ __launch_bounds__(256) void k_conv_fwd(pvnet_conv a, int M, int K, Ne
 // voxels and feeds the matrix core straight from global memory, with no LDS and no barrier.  Lane
 // (c16, g) holds the input channels 8g .. 8g+7 of voxel c16 of a tile (zero beyond cin) and the
 // weight row 16 j + c16 at the same k-values: the operands k_conv_fwd stages for the same
-// convolution, so the outputs are the same bit for bit.
+// convolution, so the outputs are the same bit for bit.  The weights are the MFMA's A operand, so that a lane holds
+// four consecutive channels of one voxel and, where rows allow (vec), reads its mask and writes them at once.  Bound by memory: 8 x 96^3 voxels 16 -> 8 in FP32 and 8 -> 16 with a
+// mask 156 us for both (6.4 TB/s of rows), 276 with one channel of four voxels a lane.
 constexpr int PWT = 4;
 
 template <int NJ>
-__global__ __launch_bounds__(256) void k_conv_pw(pvnet_conv a, int M) {
+__global__ __launch_bounds__(256) void k_conv_pw(pvnet_conv a, int M, bool vec) {
     const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
     const int64_t tile0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * PWT;
-    bf16x8 bfr[NJ];
-    float bias[NJ];
+    bf16x8 wf[NJ];
+    float bias[NJ][4];
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
         const int n = 16 * j + c16;
         uint4 v = make_uint4(0, 0, 0, 0);
         if (n < a.cout) v = *(const uint4*)(a.w + (int64_t)n * a.kpad + g * 8);
-        bfr[j] = *reinterpret_cast<const bf16x8*>(&v);
-        bias[j] = (n < a.cout && a.bias) ? a.bias[n] : 0.f;
+        wf[j] = *reinterpret_cast<const bf16x8*>(&v);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int c = 16 * j + 4 * g + e;
+            bias[j][e] = (c < a.cout && a.bias) ? a.bias[c] : 0.f;
+        }
     }
     uint4 ra[PWT];
+    uint2 mk[PWT][NJ];
 #pragma unroll
     for (int i = 0; i < PWT; i++) {
         const int64_t m = (tile0 + i) * 16 + c16;
         ra[i] = make_uint4(0, 0, 0, 0);
         if (m < M && g * 8 < a.cin) ra[i] = *(const uint4*)(a.x + m * a.ldx + g * 8);
+        if (vec && a.relu_of) {
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+                if (m < M && 16 * j + 4 * g < a.cout) mk[i][j] = *(const uint2*)(a.relu_of + m * a.ldr + 16 * j + 4 * g);
+        }
     }
     const bool relu = a.flags & PVNET_RELU, f32out = a.flags & PVNET_F32OUT;
 #pragma unroll
-    for (int i = 0; i < PWT; i++)
+    for (int i = 0; i < PWT; i++) {
+        const int64_t m = (tile0 + i) * 16 + c16;
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
-            const f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(&ra[i]), bfr[j],
+            const f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], *reinterpret_cast<const bf16x8*>(&ra[i]),
                                                                       f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-            const int n = 16 * j + c16;
-            if (n >= a.cout) continue;
+            const int n = 16 * j + 4 * g;
+            if (m >= M || n >= a.cout) continue;
+            float v[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const int64_t m = (tile0 + i) * 16 + g * 4 + e;  // MFMA row 4 g + e
-                if (m >= M) continue;
-                float v = acc[e] + bias[j];
-                if (relu) v = v < 0.f ? 0.f : v;
-                if (a.relu_of && !bf_pos(a.relu_of[m * a.ldr + n])) v = 0.f;
-                if (f32out)
-                    ((float*)a.y)[m * a.ldy + n] = v;
-                else
-                    ((uint16_t*)a.y)[m * a.ldy + n] = f2bf(v);
+                v[e] = acc[e] + bias[j][e];
+                if (relu) v[e] = v[e] < 0.f ? 0.f : v[e];
+            }
+            if (vec) {
+                if (a.relu_of)
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (!bf_pos((uint16_t)((e < 2 ? mk[i][j].x : mk[i][j].y) >> (16 * (e & 1))))) v[e] = 0.f;
+                if (f32out) *(float4*)((float*)a.y + m * a.ldy + n) = make_float4(v[0], v[1], v[2], v[3]);
+                else *(uint2*)((uint16_t*)a.y + m * a.ldy + n) = make_uint2(f2bf_pk(v[0], v[1]), f2bf_pk(v[2], v[3]));
+                continue;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                if (n + e >= a.cout) continue;
+                if (a.relu_of && !bf_pos(a.relu_of[m * a.ldr + n + e])) v[e] = 0.f;
+                if (f32out) ((float*)a.y)[m * a.ldy + n + e] = v[e];
+                else ((uint16_t*)a.y)[m * a.ldy + n + e] = f2bf(v[e]);
             }
         }
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -823,6 +854,7 @@ struct WgradPlan {
     int ktiles, ntiles, bn, nsplit, mchunk, cblk, cchunk;
     int64_t ws_main, ws_total;
     bool march;  // k_wgrad_march
+    bool pw;     // k_wgrad_pw, chunks per block in mchunk
     WgradMarch mp;
 };
 
@@ -847,10 +879,17 @@ WgradPlan plan_wgrad(const pvnet_shape& s, int ntaps, int cin, int cout, int fla
         p.nsplit = p.mp.splits;
         p.ws_main = (int64_t)p.nsplit * cout * K;
     }
+    p.pw = ntaps == 1 && cin <= 32 && cout <= 16 && !(flags & PVNET_GATHER);
+    if (p.pw) {
+        const int64_t chunks = (M + WPW_VOX - 1) / WPW_VOX;
+        p.mchunk = 4 * (int)((chunks + 4 * WPW_BLOCKS - 1) / (4 * WPW_BLOCKS));  // whole rounds of the four waves
+        p.nsplit = (int)((chunks + p.mchunk - 1) / p.mchunk);
+        p.ws_main = (int64_t)p.nsplit * cout * K;
+    }
     p.cchunk = (int)std::max<int64_t>(256, ((M + 1023) / 1024 + 255) & ~(int64_t)255);  // ~1024 blocks
     p.cblk = (int)((M + p.cchunk - 1) / p.cchunk);
     // the bias rows: one per column-sum block, or one per split when the marching kernel sums them
-    p.ws_total = p.ws_main + (int64_t)std::max(p.cblk, p.march ? p.nsplit : 0) * cout;
+    p.ws_total = p.ws_main + (int64_t)std::max(p.cblk, p.march || p.pw ? p.nsplit : 0) * cout;
     return p;
 }
 
@@ -899,11 +938,12 @@ int conv_launch(const pvnet_conv* c, const NetParts& pq, void* stream, const std
         hipLaunchKernelGGL(march_kernel(mp), dim3(nblk), dim3(64 * (mp.wx * mp.wn + mp.roll)), mp.lds, st, *c, mp, pq);
     } else if (c->ntaps == 1 && K <= BK && c->cout <= 64 && !(c->flags & PVNET_GATHER)) {
         const dim3 gp((unsigned)((M + 64 * PWT - 1) / (64 * PWT)));
+        const bool vec = rows_by_four(*c);
         switch ((c->cout + 15) / 16) {
-            case 1: hipLaunchKernelGGL((k_conv_pw<1>), gp, dim3(256), 0, st, *c, (int)M); break;
-            case 2: hipLaunchKernelGGL((k_conv_pw<2>), gp, dim3(256), 0, st, *c, (int)M); break;
-            case 3: hipLaunchKernelGGL((k_conv_pw<3>), gp, dim3(256), 0, st, *c, (int)M); break;
-            default: hipLaunchKernelGGL((k_conv_pw<4>), gp, dim3(256), 0, st, *c, (int)M); break;
+            case 1: hipLaunchKernelGGL((k_conv_pw<1>), gp, dim3(256), 0, st, *c, (int)M, vec); break;
+            case 2: hipLaunchKernelGGL((k_conv_pw<2>), gp, dim3(256), 0, st, *c, (int)M, vec); break;
+            case 3: hipLaunchKernelGGL((k_conv_pw<3>), gp, dim3(256), 0, st, *c, (int)M, vec); break;
+            default: hipLaunchKernelGGL((k_conv_pw<4>), gp, dim3(256), 0, st, *c, (int)M, vec); break;
         }
     } else if (parts) {
         conv_gather<true>(*c, pq, M, st);
@@ -941,9 +981,12 @@ int wgrad_launch(const pvnet_wgrad* a, const NetParts& pq, void* stream, const s
     hipStream_t st = (hipStream_t)stream;
     const WgradPlan p = plan_wgrad(a->s, a->ntaps, a->cin, a->cout, a->flags | (wgrad_march_ok(*a, pq) ? 0 : PVNET_GATHER));
     const int K = a->ntaps * a->cin;
-    const bool fused_db = a->db && p.march;  // the bias sums come with the weights'
+    const bool fused_db = a->db && (p.march || p.pw);  // the bias sums come with the weights'
     if (p.march) {
         hipLaunchKernelGGL(wgrad_march_kernel(p.mp), dim3(p.mp.splits * p.mp.ns * p.mp.nf), dim3(256), p.mp.lds, st, *a, p.mp, pq,
+                           fused_db ? p.ws_main : (int64_t)-1);
+    } else if (p.pw) {
+        hipLaunchKernelGGL(wgrad_pw_kernel(a->cin, a->cout), dim3(p.nsplit), dim3(256), 0, st, *a, (int)M, p.mchunk,
                            fused_db ? p.ws_main : (int64_t)-1);
     } else if (pq.cup) {
         wgrad_gather<true>(*a, pq, p, M, st);

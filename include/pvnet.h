@@ -97,6 +97,15 @@ int pvnet_conv_up_wgrad(const pvnet_wgrad* g, const uint16_t* up, int32_t ldu, i
  * wd[ci][tap'*cout + co] = w32[co][(ntaps-1-tap')*cin + ci]. */
 int pvnet_pack_weights(const float* w32, int32_t ntaps, int32_t cin, int32_t cout, uint16_t* wt,
                        uint16_t* wd, void* stream);
+/* the same for n layers, in one launch for up to 32 */
+typedef struct {
+    const float* w32;
+    uint16_t* wt;
+    uint16_t* wd;
+    int32_t ntaps, cin, cout;
+    int32_t reserved; /* 0 */
+} pvnet_pack;
+int pvnet_pack_layers(const pvnet_pack* layers, int32_t n, void* stream);
 
 /* 2x2x2 average pooling: y (shape s/2) from x (shape s); backward adds dy/8 to each child of
  * dx (accumulate = 1) or overwrites it (accumulate = 0).  All three sizes of s must be even. */

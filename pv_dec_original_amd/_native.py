@@ -69,6 +69,12 @@ class NetWgrad(C.Structure):
                 ("ws", C.c_void_p), ("dw", C.c_void_p), ("db", C.c_void_p), ("flags", C.c_int32)]
 
 
+class NetPack(C.Structure):
+    """pvnet_pack (master weights of one layer and their two bf16 layouts)."""
+    _fields_ = [("w32", C.c_void_p), ("wt", C.c_void_p), ("wd", C.c_void_p), ("ntaps", C.c_int32),
+                ("cin", C.c_int32), ("cout", C.c_int32), ("reserved", C.c_int32)]
+
+
 NET_RELU, NET_F32OUT, NET_GATHER = 1, 2, 4
 
 _lib = None
@@ -135,6 +141,7 @@ PVNET_API = [
     ("pvnet_conv_wgrad", C.c_int, [C.POINTER(NetWgrad), _vp]),
     ("pvnet_conv_up_wgrad", C.c_int, [C.POINTER(NetWgrad), _vp, C.c_int32, C.c_int32, _vp]),
     ("pvnet_pack_weights", C.c_int, [_vp, C.c_int32, C.c_int32, C.c_int32, _vp, _vp, _vp]),
+    ("pvnet_pack_layers", C.c_int, [C.POINTER(NetPack), C.c_int32, _vp]),
     ("pvnet_pool2_fwd", C.c_int, [_sp, C.c_int32, _vp, C.c_int32, _vp, C.c_int32, _vp]),
     ("pvnet_pool2_bwd", C.c_int, [_sp, C.c_int32, _vp, C.c_int32, _vp, C.c_int32, C.c_int32, _vp]),
     ("pvnet_pool2_bwd_relu", C.c_int, [_sp, C.c_int32, _vp, C.c_int32, _vp, C.c_int32, _vp, C.c_int32, _vp]),

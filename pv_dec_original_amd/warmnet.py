@@ -160,10 +160,11 @@ class UNet:
         return C.c_void_p(self.torch.cuda.current_stream().cuda_stream)
 
     def pack(self):
-        L = N.net()
-        for lay in self.spec.layers:
-            N.net_check(L.pvnet_pack_weights(_ptr(self.p, lay.offset), lay.ntaps, lay.cin, lay.cout,
-                                              _ptr(self.wt[lay.name]), _ptr(self.wd[lay.name]), self._st()))
+        layers = self.spec.layers
+        jobs = (N.NetPack * len(layers))(*[
+            N.NetPack(_ptr(self.p, lay.offset), _ptr(self.wt[lay.name]), _ptr(self.wd[lay.name]), lay.ntaps, lay.cin,
+                      lay.cout, 0) for lay in layers])
+        N.net_check(N.net().pvnet_pack_layers(jobs, len(layers), self._st()))
 
     def params_numpy(self):
         return self.p.detach().cpu().numpy().copy()

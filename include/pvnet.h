@@ -156,6 +156,11 @@ int64_t pvnet_loss_ws_doubles(int64_t m);
 int pvnet_mse_loss(int64_t m, int32_t nc, const float* y, int32_t ldy, const uint16_t* t,
                    const uint8_t* code, const float* wc, uint16_t* dy, int32_t lddy, double* part,
                    double* loss, void* stream);
+/* the same with wc in host memory (nc <= 8, read before the call returns): no copy to the device, which
+ * would wait for the stream */
+int pvnet_mse_loss_host_weights(int64_t m, int32_t nc, const float* y, int32_t ldy, const uint16_t* t,
+                                const uint8_t* code, const float* wc, uint16_t* dy, int32_t lddy,
+                                double* part, double* loss, void* stream);
 
 /* Adam (Kingma & Ba 2015) on n FP32 parameters, step t >= 1, bias-corrected:
  *   m = b1 m + (1-b1) g;  v = b2 v + (1-b2) g^2;  p -= lr * (m/(1-b1^t)) / (sqrt(v/(1-b2^t)) + eps) */

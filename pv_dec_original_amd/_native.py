@@ -154,6 +154,8 @@ PVNET_API = [
     ("pvnet_loss_ws_doubles", C.c_int64, [C.c_int64]),
     ("pvnet_mse_loss", C.c_int, [C.c_int64, C.c_int32, _vp, C.c_int32, _vp, _vp, _vp, _vp, C.c_int32,
                                  _vp, _vp, _vp]),
+    ("pvnet_mse_loss_host_weights", C.c_int, [C.c_int64, C.c_int32, _vp, C.c_int32, _vp, _vp, _vp, _vp, C.c_int32,
+                                 _vp, _vp, _vp]),
     ("pvnet_adam", C.c_int, [C.c_int64, _vp, _vp, _vp, _vp, C.c_float, C.c_float, C.c_float,
                              C.c_float, C.c_int32, _vp]),
     ("pvnet_last_error", C.c_char_p, []),

@@ -737,9 +737,17 @@ __global__ void k_features(pvnet_shape s, const uint8_t* code, const float* prm,
 
 constexpr int LOSS_BLOCK = 256;
 
+// channel weights: in device memory, or (p null) with the launch
+constexpr int LOSS_NC = 8;
+struct LossWeights {
+    const float* p;
+    float w[LOSS_NC];
+    __device__ __forceinline__ float operator[](int k) const { return p ? p[k] : w[k]; }
+};
+
 __global__ __launch_bounds__(LOSS_BLOCK) void k_loss_partial(int64_t M, int nc, const float* y, int ldy,
                                                              const uint16_t* t, const uint8_t* code,
-                                                             const float* wc, double* part) {
+                                                             const LossWeights wc, double* part) {
     __shared__ double ss[LOSS_BLOCK], sc[LOSS_BLOCK];
     const int64_t i = (int64_t)blockIdx.x * LOSS_BLOCK + threadIdx.x;
     double e = 0.0, c = 0.0;
@@ -791,7 +799,7 @@ __global__ __launch_bounds__(LOSS_BLOCK) void k_loss_final(int nblk, int nc, con
 }
 
 __global__ void k_loss_grad(int64_t M, int nc, const float* y, int ldy, const uint16_t* t, const uint8_t* code,
-                            const float* wc, const double* loss, uint16_t* dy, int lddy) {
+                            const LossWeights wc, const double* loss, uint16_t* dy, int lddy) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= M) return;
     const double cnt = loss[1];
@@ -1048,6 +1056,22 @@ int up_args(const pvnet_shape* s, int ntaps, int cin, const void* up, int ldu, i
     return 0;
 }
 
+int loss_launch(int64_t m, int32_t nc, const float* y, int32_t ldy, const uint16_t* t, const uint8_t* code,
+                const LossWeights& wc, uint16_t* dy, int32_t lddy, double* part, double* loss, void* stream,
+                const std::string& who) {
+    if (m <= 0 || nc <= 0 || ldy < nc || lddy < nc || !y || !t || !code || !dy || !part || !loss)
+        return fail(1, who + ": bad argument");
+    hipStream_t st = (hipStream_t)stream;
+    const int nblk = blocks_for(m, LOSS_BLOCK);
+    hipLaunchKernelGGL(k_loss_partial, dim3(nblk), dim3(LOSS_BLOCK), 0, st, m, nc, y, ldy, t, code, wc, part);
+    NET_LAUNCH();
+    hipLaunchKernelGGL(k_loss_final, dim3(1), dim3(LOSS_BLOCK), 0, st, nblk, nc, part, loss);
+    NET_LAUNCH();
+    hipLaunchKernelGGL(k_loss_grad, dim3(blocks_for(m, 256)), dim3(256), 0, st, m, nc, y, ldy, t, code, wc, loss, dy, lddy);
+    NET_LAUNCH();
+    return 0;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1214,17 +1238,17 @@ int64_t pvnet_loss_ws_doubles(int64_t m) { return m > 0 ? 2 * ((m + LOSS_BLOCK -
 
 int pvnet_mse_loss(int64_t m, int32_t nc, const float* y, int32_t ldy, const uint16_t* t, const uint8_t* code,
                    const float* wc, uint16_t* dy, int32_t lddy, double* part, double* loss, void* stream) {
-    if (m <= 0 || nc <= 0 || ldy < nc || lddy < nc || !y || !t || !code || !wc || !dy || !part || !loss)
-        return fail(1, "pvnet_mse_loss: bad argument");
-    hipStream_t st = (hipStream_t)stream;
-    const int nblk = blocks_for(m, LOSS_BLOCK);
-    hipLaunchKernelGGL(k_loss_partial, dim3(nblk), dim3(LOSS_BLOCK), 0, st, m, nc, y, ldy, t, code, wc, part);
-    NET_LAUNCH();
-    hipLaunchKernelGGL(k_loss_final, dim3(1), dim3(LOSS_BLOCK), 0, st, nblk, nc, part, loss);
-    NET_LAUNCH();
-    hipLaunchKernelGGL(k_loss_grad, dim3(blocks_for(m, 256)), dim3(256), 0, st, m, nc, y, ldy, t, code, wc, loss, dy, lddy);
-    NET_LAUNCH();
-    return 0;
+    if (!wc) return fail(1, "pvnet_mse_loss: bad argument");
+    return loss_launch(m, nc, y, ldy, t, code, LossWeights{wc, {}}, dy, lddy, part, loss, stream, "pvnet_mse_loss");
+}
+
+int pvnet_mse_loss_host_weights(int64_t m, int32_t nc, const float* y, int32_t ldy, const uint16_t* t,
+                                const uint8_t* code, const float* wc, uint16_t* dy, int32_t lddy, double* part,
+                                double* loss, void* stream) {
+    if (!wc || nc <= 0 || nc > LOSS_NC) return fail(1, "pvnet_mse_loss_host_weights: bad argument");
+    LossWeights w{};
+    for (int k = 0; k < nc; k++) w.w[k] = wc[k];
+    return loss_launch(m, nc, y, ldy, t, code, w, dy, lddy, part, loss, stream, "pvnet_mse_loss_host_weights");
 }
 
 int pvnet_adam(int64_t n, float* p, const float* g, float* m, float* v, float lr, float b1, float b2, float eps,

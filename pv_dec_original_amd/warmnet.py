@@ -281,12 +281,13 @@ class UNet:
         """Masked MSE of the last forward output against target (bf16 device tensor (M, 4));
         leaves dL/dY in the dY buffer and returns the device tensor [loss, n_fluid]."""
         b = self._bufs
-        wc = self.torch.tensor(weights, dtype=self.torch.float32, device="cuda")
+        if len(weights) < N_TARGET:
+            raise ValueError(f"need {N_TARGET} channel weights, got {len(weights)}")
+        wc = (C.c_float * N_TARGET)(*[float(w) for w in weights[:N_TARGET]])
         M = b["M"][0]
-        N.net_check(N.net().pvnet_mse_loss(M, N_TARGET, _ptr(b["Y"]), OUT_CH, _ptr(target), _ptr(code),
-                                           _ptr(wc), _ptr(b["dY"]), OUT_CH, _ptr(b["lpart"]),
-                                           _ptr(b["loss"]), self._st()))
-        self._wc = wc  # keep alive until the stream has used it
+        N.net_check(N.net().pvnet_mse_loss_host_weights(M, N_TARGET, _ptr(b["Y"]), OUT_CH, _ptr(target), _ptr(code),
+                                                        C.cast(wc, C.c_void_p), _ptr(b["dY"]), OUT_CH,
+                                                        _ptr(b["lpart"]), _ptr(b["loss"]), self._st()))
         return b["loss"]
 
     def backward(self):

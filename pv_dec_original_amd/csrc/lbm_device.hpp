@@ -82,11 +82,41 @@ __device__ __forceinline__ void moments(const R (&f)[27], R& rho, R (&u)[3]) {
 }
 
 // ---- equilibrium of one direction, Simulation.cpp:186-196 ----
+//   w rho (1 + 3 du + 4.5 du du - 1.5 u.u),  du = ux cx + uy cy + uz cz
+// Directions come in opposite pairs whose du differ in sign alone, exactly, so 3 du and 4.5 du du are written in the
+// pair's canonical sign (first non-zero component positive) and shared by the compiler; terms with a zero component
+// are left out: each adds a signed zero, which changes no later value.  What the left-out products do keep is that an
+// infinite velocity makes every direction not a number: `one` carries that.  The 16-bit steps are bound by vector
+// instructions: 968,846 nodes, D3Q19, FP16, all in cache, with WSS in every step 34.5 -> 31.6 us a step (19.0 M
+// vector instructions of 4 clocks before: 31 us of the chip).
+template <int Q, int D>
+struct Dir {
+    static constexpr int x = Lat<Q>::cx[D], y = Lat<Q>::cy[D], z = Lat<Q>::cz[D];
+    static constexpr bool rest = x == 0 && y == 0 && z == 0;
+    static constexpr bool neg = x < 0 || (x == 0 && (y < 0 || (y == 0 && z < 0)));
+    static constexpr int s = neg ? -1 : 1;
+    static constexpr int px = s * x, py = s * y, pz = s * z;  // the pair's canonical direction
+};
+
+template <int C, bool FIRST, class R>
+__device__ __forceinline__ R add_term(R a, R v) {
+    if constexpr (C == 0) return a;
+    else if constexpr (FIRST) return v;
+    else if constexpr (C > 0) return a + v;
+    else return a - v;
+}
+
 template <int Q, int D, class R>
 __device__ __forceinline__ R feq_dir(R rho, const R (&u)[3]) {
-    R du = u[0] * R(Lat<Q>::cx[D]) + u[1] * R(Lat<Q>::cy[D]) + u[2] * R(Lat<Q>::cz[D]);
-    R u_sqr = u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
-    return R(Lat<Q>::w[D]) * rho * (R(1.0) + R(3.0) * du + R(4.5) * du * du - R(1.5) * u_sqr);
+    using C = Dir<Q, D>;
+    const R u_sqr = u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
+    const R one = R(1.0) + (u[0] * R(0.0) + u[1] * R(0.0) + u[2] * R(0.0));
+    if constexpr (C::rest) return R(Lat<Q>::w[D]) * rho * (one - R(1.5) * u_sqr);
+    R du = add_term<C::px, true>(R(0.0), u[0]);
+    du = add_term<C::py, C::px == 0>(du, u[1]);
+    du = add_term<C::pz, C::px == 0 && C::py == 0>(du, u[2]);
+    const R t = R(3.0) * du, q = R(4.5) * du * du;
+    return R(Lat<Q>::w[D]) * rho * ((C::neg ? one - t : one + t) + q - R(1.5) * u_sqr);
 }
 
 template <int Q, class R, int D = 0>
@@ -223,10 +253,11 @@ __device__ __forceinline__ void wall_rule(R (&m)[Q], uint32_t nmiss) {
 // non-equilibrium population of direction A in component I, with the loop's operation order.
 // Terms with a zero velocity component are left out: for a finite normal each is a signed zero,
 // and adding a signed zero to these sums, which start at +0 and so never hold -0, leaves them
-// unchanged, so the weight rounds exactly as the full loop's.
+// unchanged, so the weight rounds exactly as the full loop's.  Opposite directions have the same weight (every sign
+// cancels, exactly): it is written in the pair's canonical sign, so that the compiler computes it once.
 template <int Q, class R, int I, int A>
 __device__ __forceinline__ R wss_weight(const R (&n)[3]) {
-    constexpr int c0 = Lat<Q>::cx[A], c1 = Lat<Q>::cy[A], c2 = Lat<Q>::cz[A];
+    constexpr int c0 = Dir<Q, A>::px, c1 = Dir<Q, A>::py, c2 = Dir<Q, A>::pz;
     constexpr int ci = (I == 0) ? c0 : (I == 1) ? c1 : c2;
     R sum_k = R(0.0);
     if constexpr (c0 != 0) sum_k += R(c0) * n[0] * n[I];

@@ -345,10 +345,12 @@ __device__ __forceinline__ bool node_update(const StepParams& p, int blk, double
             const R C = R(p.C);
             const R t0 = C * s0, t1 = C * s1, t2 = C * s2;
             const R W = sqrt(t0 * t0 + t1 * t1 + t2 * t2);
-            p.wss[ws] = (double)W;
-            p.tau3[ws] = (double)t0;
-            p.tau3[ms + ws] = (double)t1;
-            p.tau3[2 * ms + ws] = (double)t2;
+            if (p.flags & F_WSS_OUT) {  // 32 of the 152 bytes a next-to-wall node moves for its WSS
+                p.wss[ws] = (double)W;
+                p.tau3[ws] = (double)t0;
+                p.tau3[ms + ws] = (double)t1;
+                p.tau3[2 * ms + ws] = (double)t2;
+            }
             p.acc[ws] = pacc[0] + (double)t0;
             p.acc[ms + ws] = pacc[1] + (double)t1;
             p.acc[2 * ms + ws] = pacc[2] + (double)t2;

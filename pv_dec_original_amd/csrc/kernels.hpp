@@ -12,6 +12,7 @@ enum StepFlags : int {
     F_WSS = 1,     // evaluate WSS and its accumulators on next-to-wall nodes
     F_MACRO = 2,   // write rho/u of this launch's collision to the macro planes
     F_REDUCE = 4,  // write FP64 block partial sums (mass, inlet/outlet flux, non-finite count)
+    F_WSS_OUT = 16,  // with F_WSS: also write WSS and its vector (they are those of the last such launch of a call)
     F_INIT = 8,    // no gather/closure: start from f = w or f = f_eq(init_rho, init_u)
 };
 

@@ -327,7 +327,7 @@ __device__ __forceinline__ void transpose8(const uint4 (&r)[8], uint4 (&o)[8]) {
 }
 
 template <int BN, bool PARTS = false>
-__global__ __launch_bounds__(256) void k_conv_wgrad(pvnet_wgrad a, int M, int K, int mchunk, NetParts pq) {
+__global__ __launch_bounds__(256) void k_conv_wgrad(pvnet_wgrad a, int M, int K, int mchunk, NetParts pq, int64_t dboff) {
     constexpr int BMW = 128;  // voxels per LDS fill
     constexpr int PW = BMW + 8;  // LDS row pitch in bf16 (272 bytes)
     __shared__ __attribute__((aligned(16))) uint16_t As[BN * PW];  // dy^T  [n][m]
@@ -353,8 +353,14 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(pvnet_wgrad a, int M, int K,
     const int64_t off = ((int64_t)dz * h + dy) * w + dx;
     const bool dcol = drole && n0 + nc * 8 < a.cout;
 
-    f32x4 acc[BN / 16];
-    for (int j = 0; j < BN / 16; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 acc[BN / 16], accb[BN / 16];
+    for (int j = 0; j < BN / 16; j++) acc[j] = accb[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // the bias gradient: dy against ones, in one wave of the blocks of the first k-values (a launch of column sums
+    // before, 3.7 us: 4000 x 80 -> 32 pointwise, all three passes 32.1 -> 29.1 us)
+    const bool dob = dboff >= 0 && blockIdx.x == 0 && __builtin_amdgcn_readfirstlane(wv) == 0;
+    bf16x8 ones;
+#pragma unroll
+    for (int e = 0; e < 8; e++) ones[e] = (__bf16)1.0f;
 
     uint4 r[8];
     auto load = [&](int mbase) {
@@ -411,10 +417,17 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(pvnet_wgrad a, int M, int K,
             for (int j = 0; j < BN / 16; j++) {
                 const bf16x8 ad = *(const bf16x8*)(As + (j * 16 + c16) * PW + kk * 32 + g * 8);
                 acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ad, bx, acc[j], 0, 0, 0);
+                if (dob) accb[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ad, ones, accb[j], 0, 0, 0);
             }
         }
         __syncthreads();
     }
+    if (dob && c16 == 0)  // every column holds the sum of its row's channel
+        for (int j = 0; j < BN / 16; j++)
+            for (int e = 0; e < 4; e++) {
+                const int n = n0 + j * 16 + g * 4 + e;
+                if (n < a.cout) a.ws[dboff + (int64_t)split * a.cout + n] = accb[j][e];
+            }
 
     const int kk = k0 + wv * 16 + c16;
     if (kk >= K) return;
@@ -425,36 +438,11 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(pvnet_wgrad a, int M, int K,
         }
 }
 
-// column sums of dy over a chunk of voxels per block: part[blk][n].  Thread t sums the 8-channel
-// group t % g over the rows r = t / g, t / g + R, ... (g = cout / 8, R = 256 / g); the R partial
-// rows are then added in ascending order.
-__global__ __launch_bounds__(256) void k_colsum(const uint16_t* dy, int ld, int cout, int M, int mchunk,
-                                                float* part) {
-    __shared__ float sp[256 * 8];
-    const int g = cout / 8, R = 256 / g;
-    const int t = threadIdx.x, c8 = t % g, rg = t / g;
-    const int mb = blockIdx.x * mchunk, me = min(M, mb + mchunk);
-    float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (rg < R)
-        for (int m = mb + rg; m < me; m += R) {
-            const uint4 v = *(const uint4*)(dy + (int64_t)m * ld + c8 * 8);
-            const uint16_t* pv = (const uint16_t*)&v;
-            for (int j = 0; j < 8; j++) acc[j] += bf2f(pv[j]);
-        }
-    for (int j = 0; j < 8; j++) sp[t * 8 + j] = acc[j];
-    __syncthreads();
-    if (t < cout) {
-        const int cg = t / 8, j = t % 8;
-        float s = 0.f;
-        for (int r = 0; r < R; r++) s += sp[(r * g + cg) * 8 + j];
-        part[(int64_t)blockIdx.x * cout + t] = s;
-    }
-}
-
 // dst[i] = sum_s src[s * len + i] in a fixed order: a block takes 16 columns, its 16 row groups
 // sum the rows rg, rg + 16, ... in ascending order, and the 16 partials are added in ascending rg.  Bound
 // by the latency of a row group's loads where the splits are many and the columns few: eight of them are in
-// flight (768 splits of 6912 columns 16.9 us with one, 8.5 with eight; the order of the sum is the same)
+// flight (768 splits of 6912 columns 16.9 us with one, 8.5 with eight; the order of the sum is the same).  The
+// partials are summed in 64 bits: the rounding left is that of the partials' own chains and of the result.
 constexpr int SUM_COLS = 16;
 
 // One reduction of split partials: dst[(i / rowlen) ldd + i % rowlen] = sum_s src[s len + i].
@@ -469,7 +457,7 @@ struct SumJob {
 // Two reductions in one launch (the weight and bias gradients of a layer): blocks below
 // a.blocks take job a, the others job b, each summing exactly as alone.
 __global__ __launch_bounds__(256) void k_sum_splits(const SumJob a, const SumJob b) {
-    __shared__ float sp[16][SUM_COLS + 1];
+    __shared__ double sp[16][SUM_COLS + 1];
     const bool second = (int)blockIdx.x >= a.blocks;
     const float* src = second ? b.src : a.src;
     float* dst = second ? b.dst : a.dst;
@@ -478,17 +466,17 @@ __global__ __launch_bounds__(256) void k_sum_splits(const SumJob a, const SumJob
     const int blk = second ? (int)blockIdx.x - a.blocks : (int)blockIdx.x;
     const int t = threadIdx.x, col = t % SUM_COLS, rg = t / SUM_COLS;
     const int64_t i = (int64_t)blk * SUM_COLS + col;
-    float s = 0.f;
+    double s = 0.0;
     if (i < len) {
 #pragma unroll 8
-        for (int p = rg; p < nsplit; p += 16) s += src[(int64_t)p * len + i];
+        for (int p = rg; p < nsplit; p += 16) s += (double)src[(int64_t)p * len + i];
     }
     sp[rg][col] = s;
     __syncthreads();
     if (t < SUM_COLS && i < len) {
-        float acc = 0.f;
+        double acc = 0.0;
         for (int r = 0; r < 16; r++) acc += sp[r][t];
-        dst[(i / rowlen) * ldd + i % rowlen] = acc;
+        dst[(i / rowlen) * ldd + i % rowlen] = (float)acc;
     }
 }
 
@@ -886,7 +874,7 @@ bool al16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 int kpad_of(int ntaps, int c) { return (ntaps * c + BK - 1) / BK * BK; }
 
 struct WgradPlan {
-    int ktiles, ntiles, bn, nsplit, mchunk, cblk, cchunk;
+    int ktiles, ntiles, bn, nsplit, mchunk;
     int64_t ws_main, ws_total;
     bool march;  // k_wgrad_march
     bool pw;     // k_wgrad_pw, chunks per block in mchunk
@@ -921,10 +909,7 @@ WgradPlan plan_wgrad(const pvnet_shape& s, int ntaps, int cin, int cout, int fla
         p.nsplit = (int)((chunks + p.mchunk - 1) / p.mchunk);
         p.ws_main = (int64_t)p.nsplit * cout * K;
     }
-    p.cchunk = (int)std::max<int64_t>(256, ((M + 1023) / 1024 + 255) & ~(int64_t)255);  // ~1024 blocks
-    p.cblk = (int)((M + p.cchunk - 1) / p.cchunk);
-    // the bias rows: one per column-sum block, or one per split when the marching kernel sums them
-    p.ws_total = p.ws_main + (int64_t)std::max(p.cblk, p.march || p.pw ? p.nsplit : 0) * cout;
+    p.ws_total = p.ws_main + (int64_t)p.nsplit * cout;  // and the bias rows
     return p;
 }
 
@@ -954,16 +939,16 @@ void conv_gather(const pvnet_conv& c, const NetParts& pq, int64_t M, hipStream_t
     }
 }
 
-int conv_launch(const pvnet_conv* c, const NetParts& pq, void* stream, const std::string& who) {
-    if (!c || !shape_ok(&c->s)) return fail(1, who + ": bad shape");
-    if (c->ntaps != 1 && c->ntaps != 27) return fail(1, who + ": ntaps must be 1 or 27");
-    if (c->cin <= 0 || c->cin % 8 || c->cout <= 0) return fail(1, who + ": cin must be a positive multiple of 8");
-    if (c->kpad != kpad_of(c->ntaps, c->cin)) return fail(1, who + ": kpad must be roundup(ntaps*cin, 32)");
-    if (c->ldx < c->cin - pq.cup || c->ldx % 8 || c->ldy < c->cout - pq.c0) return fail(1, who + ": bad row lengths");
-    if (!c->x || !c->w || !c->y || !al16(c->x) || !al16(c->w)) return fail(1, who + ": null or misaligned pointer");
-    if (c->relu_of && c->ldr < c->cout) return fail(1, who + ": bad relu_of row length");
+int conv_launch(const pvnet_conv* c, const NetParts& pq, void* stream, const char* who) {
+    if (!c || !shape_ok(&c->s)) return fail(1, std::string(who) + ": bad shape");
+    if (c->ntaps != 1 && c->ntaps != 27) return fail(1, std::string(who) + ": ntaps must be 1 or 27");
+    if (c->cin <= 0 || c->cin % 8 || c->cout <= 0) return fail(1, std::string(who) + ": cin must be a positive multiple of 8");
+    if (c->kpad != kpad_of(c->ntaps, c->cin)) return fail(1, std::string(who) + ": kpad must be roundup(ntaps*cin, 32)");
+    if (c->ldx < c->cin - pq.cup || c->ldx % 8 || c->ldy < c->cout - pq.c0) return fail(1, std::string(who) + ": bad row lengths");
+    if (!c->x || !c->w || !c->y || !al16(c->x) || !al16(c->w)) return fail(1, std::string(who) + ": null or misaligned pointer");
+    if (c->relu_of && c->ldr < c->cout) return fail(1, std::string(who) + ": bad relu_of row length");
     const int64_t M = voxels(c->s);
-    if (M >= (int64_t)1 << 31) return fail(1, who + ": too many voxels");
+    if (M >= (int64_t)1 << 31) return fail(1, std::string(who) + ": too many voxels");
     hipStream_t st = (hipStream_t)stream;
     const int K = c->ntaps * c->cin;
     const bool parts = pq.cup || pq.c0;
@@ -990,77 +975,67 @@ int conv_launch(const pvnet_conv* c, const NetParts& pq, void* stream, const std
 }
 
 template <bool PARTS>
-void wgrad_gather(const pvnet_wgrad& a, const NetParts& pq, const WgradPlan& p, int64_t M, hipStream_t st) {
+void wgrad_gather(const pvnet_wgrad& a, const NetParts& pq, const WgradPlan& p, int64_t M, int64_t dboff, hipStream_t st) {
     const int K = a.ntaps * a.cin;
     const dim3 grid(p.ktiles, p.ntiles, p.nsplit);
     if (p.bn == 16)
-        hipLaunchKernelGGL((k_conv_wgrad<16, PARTS>), grid, dim3(256), 0, st, a, (int)M, K, p.mchunk, pq);
+        hipLaunchKernelGGL((k_conv_wgrad<16, PARTS>), grid, dim3(256), 0, st, a, (int)M, K, p.mchunk, pq, dboff);
     else if (p.bn == 32)
-        hipLaunchKernelGGL((k_conv_wgrad<32, PARTS>), grid, dim3(256), 0, st, a, (int)M, K, p.mchunk, pq);
+        hipLaunchKernelGGL((k_conv_wgrad<32, PARTS>), grid, dim3(256), 0, st, a, (int)M, K, p.mchunk, pq, dboff);
     else
-        hipLaunchKernelGGL((k_conv_wgrad<64, PARTS>), grid, dim3(256), 0, st, a, (int)M, K, p.mchunk, pq);
+        hipLaunchKernelGGL((k_conv_wgrad<64, PARTS>), grid, dim3(256), 0, st, a, (int)M, K, p.mchunk, pq, dboff);
 }
 
-int wgrad_launch(const pvnet_wgrad* a, const NetParts& pq, void* stream, const std::string& who) {
-    if (!a || !shape_ok(&a->s)) return fail(1, who + ": bad shape");
-    if (a->ntaps != 1 && a->ntaps != 27) return fail(1, who + ": ntaps must be 1 or 27");
+int wgrad_launch(const pvnet_wgrad* a, const NetParts& pq, void* stream, const char* who) {
+    if (!a || !shape_ok(&a->s)) return fail(1, std::string(who) + ": bad shape");
+    if (a->ntaps != 1 && a->ntaps != 27) return fail(1, std::string(who) + ": ntaps must be 1 or 27");
     if (a->cin <= 0 || a->cin % 8 || a->cout <= 0 || a->cout % 8)
-        return fail(1, who + ": cin and cout must be positive multiples of 8");
-    if (a->ldx < a->cin - pq.cup || a->ldx % 8 || a->lddy < a->cout || a->lddy % 8) return fail(1, who + ": bad row lengths");
+        return fail(1, std::string(who) + ": cin and cout must be positive multiples of 8");
+    if (a->ldx < a->cin - pq.cup || a->ldx % 8 || a->lddy < a->cout || a->lddy % 8) return fail(1, std::string(who) + ": bad row lengths");
     if (!a->x || !a->dy || !a->ws || !a->dw || !al16(a->x) || !al16(a->dy))
-        return fail(1, who + ": null or misaligned pointer");
+        return fail(1, std::string(who) + ": null or misaligned pointer");
     const int64_t M = voxels(a->s);
-    if (M % 32) return fail(1, who + ": voxel count must be a multiple of 32");
-    if (M >= (int64_t)1 << 31) return fail(1, who + ": too many voxels");
-    if (a->db && a->cout > 256) return fail(1, who + ": bias gradient needs cout <= 256");
+    if (M % 32) return fail(1, std::string(who) + ": voxel count must be a multiple of 32");
+    if (M >= (int64_t)1 << 31) return fail(1, std::string(who) + ": too many voxels");
+    if (a->db && a->cout > 256) return fail(1, std::string(who) + ": bias gradient needs cout <= 256");
     hipStream_t st = (hipStream_t)stream;
     const WgradPlan p = plan_wgrad(a->s, a->ntaps, a->cin, a->cout, a->flags | (wgrad_march_ok(*a, pq) ? 0 : PVNET_GATHER));
     const int K = a->ntaps * a->cin;
-    const bool fused_db = a->db && (p.march || p.pw);  // the bias sums come with the weights'
+    const int64_t dboff = a->db ? p.ws_main : -1;  // the bias sums come with the weights'
     if (p.march) {
         hipLaunchKernelGGL(wgrad_march_kernel(p.mp), dim3(p.mp.splits * p.mp.ns * p.mp.nf), dim3(256), p.mp.lds, st, *a, p.mp, pq,
-                           fused_db ? p.ws_main : (int64_t)-1);
+                           dboff);
     } else if (p.pw) {
-        hipLaunchKernelGGL(wgrad_pw_kernel(a->cin, a->cout), dim3(p.nsplit), dim3(256), 0, st, *a, (int)M, p.mchunk,
-                           fused_db ? p.ws_main : (int64_t)-1);
+        hipLaunchKernelGGL(wgrad_pw_kernel(a->cin, a->cout), dim3(p.nsplit), dim3(256), 0, st, *a, (int)M, p.mchunk, dboff);
     } else if (pq.cup) {
-        wgrad_gather<true>(*a, pq, p, M, st);
+        wgrad_gather<true>(*a, pq, p, M, dboff, st);
     } else {
-        wgrad_gather<false>(*a, pq, p, M, st);
+        wgrad_gather<false>(*a, pq, p, M, dboff, st);
     }
     NET_LAUNCH();
     const int64_t len = (int64_t)a->cout * K;
     const SumJob jw{a->ws, a->dw, len, (int64_t)K, (int64_t)K, p.nsplit, (int)blocks_for(len, SUM_COLS)};
     SumJob jb{nullptr, nullptr, 0, 1, 1, 0, 0};
-    if (fused_db) {
+    if (a->db)
         jb = SumJob{a->ws + p.ws_main, a->db, (int64_t)a->cout, (int64_t)a->cout, (int64_t)a->cout, p.nsplit,
                     (int)blocks_for(a->cout, SUM_COLS)};
-    } else if (a->db) {
-        // the bias column sums read only dy: they run before the split sums, whose launch then
-        // reduces the weight and the bias partials together
-        float* part = a->ws + p.ws_main;
-        hipLaunchKernelGGL(k_colsum, dim3(p.cblk), dim3(256), 0, st, a->dy, a->lddy, a->cout, (int)M, p.cchunk, part);
-        NET_LAUNCH();
-        jb = SumJob{part, a->db, (int64_t)a->cout, (int64_t)a->cout, (int64_t)a->cout, p.cblk,
-                    (int)blocks_for(a->cout, SUM_COLS)};
-    }
     hipLaunchKernelGGL(k_sum_splits, dim3(jw.blocks + jb.blocks), dim3(256), 0, st, jw, jb);
     NET_LAUNCH();
     return 0;
 }
 
-int up_args(const pvnet_shape* s, int ntaps, int cin, const void* up, int ldu, int cup, const std::string& who) {
-    if (!shape_ok(s) || s->d % 2 || s->h % 2 || s->w % 2) return fail(1, who + ": sizes must be even");
+int up_args(const pvnet_shape* s, int ntaps, int cin, const void* up, int ldu, int cup, const char* who) {
+    if (!shape_ok(s) || s->d % 2 || s->h % 2 || s->w % 2) return fail(1, std::string(who) + ": sizes must be even");
     if (ntaps != 27 || cup <= 0 || cup % 8 || cup >= cin || ldu < cup || ldu % 8 || !up || !al16(up))
-        return fail(1, who + ": bad upsampled part");
+        return fail(1, std::string(who) + ": bad upsampled part");
     return 0;
 }
 
 int loss_launch(int64_t m, int32_t nc, const float* y, int32_t ldy, const uint16_t* t, const uint8_t* code,
                 const LossWeights& wc, uint16_t* dy, int32_t lddy, double* part, double* loss, void* stream,
-                const std::string& who) {
+                const char* who) {
     if (m <= 0 || nc <= 0 || ldy < nc || lddy < nc || !y || !t || !code || !dy || !part || !loss)
-        return fail(1, who + ": bad argument");
+        return fail(1, std::string(who) + ": bad argument");
     hipStream_t st = (hipStream_t)stream;
     const int nblk = blocks_for(m, LOSS_BLOCK);
     hipLaunchKernelGGL(k_loss_partial, dim3(nblk), dim3(LOSS_BLOCK), 0, st, m, nc, y, ldy, t, code, wc, part);

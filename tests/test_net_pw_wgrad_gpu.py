@@ -46,3 +46,17 @@ def test_pointwise_wgrad_sums(case):
     ref = gd.t().contiguous() @ xd
     assert float((got[0][0] - ref).norm() / ref.norm()) < 1e-5
     assert float((got[0][1] - gd.sum(0)).norm() / gd.sum(0).norm()) < 1e-5
+
+
+WIDE = [
+    # the tiled kernel, whose bias sums ride on its first blocks: each tile height, several k-tiles, part chunks
+    ((1, 1, 4, 8), 40, 8, 40, 0, 8, 0),
+    ((2, 3, 4, 4), 8, 24, 8, 0, 32, 8),
+    ((1, 8, 32, 43), 72, 64, 80, 8, 64, 0),
+    ((3, 8, 37, 32), 224, 136, 224, 0, 136, 0),
+]
+
+
+@pytest.mark.parametrize("case", WIDE, ids=[f"t{i}" for i in range(len(WIDE))])
+def test_wide_pointwise_wgrad_sums(case):
+    test_pointwise_wgrad_sums(case)

@@ -137,7 +137,7 @@ struct pvlbm_sim {
     // events of the copies, allocated by the first read-out; position of each group's first node, and their number
     double *d_gather = nullptr, *h_gather = nullptr;
     hipEvent_t ev_gather[2] = {nullptr, nullptr};
-    std::vector<int32_t> gather_first;
+    std::vector<int64_t> gather_first;
     double* d_expand = nullptr;  // scratch of a start from a coarse field, allocated by the first one
     unsigned long long* d_gate = nullptr;
     // host copy of the triangles (link fractions), boundary slots (padded node, closure)
@@ -281,7 +281,7 @@ struct pvlbm_sim {
         ensure_gather();
         const int64_t nbox = nx * ny * nz, half = (int64_t)GATHER_TILES * 64 * 4;
         auto start = [&](int32_t gi) {
-            const int32_t t0 = gi * GATHER_TILES, cnt = gather_first[gi + 1] - gather_first[gi];
+            const int32_t t0 = gi * GATHER_TILES, cnt = (int32_t)(gather_first[gi + 1] - gather_first[gi]);
             double* d = d_gather + (gi & 1) * half;
             HIPCHK(launch_macros_nodes(d_macro, ns, d_tdesc, t0, std::min(GATHER_TILES, ntiles - t0), d, stream));
             HIPCHK(hipMemcpyAsync(h_gather + (gi & 1) * half, d, sizeof(double) * 4 * cnt, hipMemcpyDeviceToHost, stream));
@@ -293,7 +293,7 @@ struct pvlbm_sim {
             if (gi + 1 < groups) start(gi + 1);
             const double* v = h_gather + (gi & 1) * half;
             const int64_t* box = lists[PVLBM_LIST_FLUID].data() + gather_first[gi];
-            const int32_t cnt = gather_first[gi + 1] - gather_first[gi];
+            const int32_t cnt = (int32_t)(gather_first[gi + 1] - gather_first[gi]);
             for (int32_t i = 0; i < cnt; i++) {
                 const int64_t b = box[i];
                 if (rho) rho[b] = v[4 * i];
@@ -820,14 +820,15 @@ extern "C" int pvlbm_create(const uint8_t* fluid, const pvlbm_grid* grid, double
         // tile descriptors: lane masks and first side-table slots (slots follow node order)
         std::vector<TileDesc> tdesc(tiles.size());
         {
-            int32_t bs = 0, wsl = 0, nodes = 0;
+            int32_t bs = 0, wsl = 0;
+            int64_t nodes = 0;
             for (size_t ti = 0; ti < tiles.size(); ti++) {
                 TileDesc& D = tdesc[ti];
                 D.tile = tiles[ti];
                 D.bslot = bs;
                 D.wslot = wsl;
                 if (ti % GATHER_TILES == 0) S->gather_first.push_back(nodes);
-                D.first = nodes;
+                D.first = (uint32_t)nodes;
                 D.node = D.ntw = D.bnd = 0;
                 for (int l = 0; l < 64; l++) {
                     const uint8_t kd = kind[(size_t)tiles[ti] * 64 + l];

@@ -647,7 +647,7 @@ __global__ __launch_bounds__(256) void k_macros_nodes(const double* macro, int64
     const TileDesc& D = tdesc[t0 + t];
     if (!((D.node >> lane) & 1)) return;
     const int64_t n = (int64_t)D.tile * 64 + lane;
-    const int64_t i = D.first - tdesc[t0].first + __popcll(D.node & ((1ull << lane) - 1));
+    const int64_t i = (D.first - tdesc[t0].first) + (uint32_t)__popcll(D.node & ((1ull << lane) - 1));
     dvec2* o = reinterpret_cast<dvec2*>(out + 4 * i);
     o[0] = dvec2{macro[n], macro[ns + n]};
     o[1] = dvec2{macro[2 * ns + n], macro[3 * ns + n]};

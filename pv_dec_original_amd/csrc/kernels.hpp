@@ -34,7 +34,7 @@ struct alignas(16) TileDesc {
     int32_t tile;
     int32_t bslot;   // first boundary-table slot of the tile
     int32_t wslot;   // first next-to-wall-table slot of the tile
-    int32_t first;   // nodes in the tiles before: position of the tile's first node in node order
+    uint32_t first;  // nodes in the tiles before, modulo 2^32: differences place a tile's nodes within its group
     uint64_t node;
     uint64_t ntw;
     uint64_t bnd;

@@ -587,21 +587,22 @@ hipError_t launch_expand_coarse(const float* rho_c, const float* u_c, int cx, in
     return hipGetLastError();
 }
 
-// Compact FP32 fields, four points of a row per thread (VEC: whole quads with 16-byte stores).  Bound by the
+// Compact FP32 fields, PT consecutive points of a row per thread (VEC: four, with 16-byte stores).  Bound by the
 // output's 16 bytes a point: most points are not nodes and read one kind byte.  1024 x 512 x 512: 1.03 ms
 // (4.4 TB/s), 1.30 ms with one point and 64-bit divisions per thread.
-template <bool VEC, class I>
+template <bool VEC, int PT, class I>
 __global__ __launch_bounds__(256) void k_macros_f32(const double* macro, const uint8_t* kind, int64_t nx, uint32_t ny, int64_t nbox,
                                                     I nq, I quads, int64_t nxp, int64_t nyp, int64_t ns, float* rho, float* u) {
     const I q = (I)blockIdx.x * 256 + threadIdx.x;
     if (q >= quads) return;
     const I row = q / nq;
-    const int64_t i = 4 * (int64_t)(q - row * nq), r = (int64_t)row;
+    const int64_t i = PT * (int64_t)(q - row * nq), r = (int64_t)row;
     const int64_t n = ((int64_t)((uint32_t)row % ny) + nyp * (int64_t)((uint32_t)row / ny)) * nxp + i, b = r * nx + i;
-    const uint32_t k4 = *reinterpret_cast<const uint32_t*>(kind + n);  // rows are padded: always within the row
-    float v[4][4];
+    // rows are padded: four kinds are always within the row
+    const uint32_t k4 = PT == 4 ? *reinterpret_cast<const uint32_t*>(kind + n) : kind[n];
+    float v[4][PT];
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
+    for (int e = 0; e < PT; e++) {
         const bool node = (k4 >> (8 * e)) & 0xffu;
         v[0][e] = node ? (float)macro[n + e] : 1.0f;
 #pragma unroll
@@ -614,7 +615,7 @@ __global__ __launch_bounds__(256) void k_macros_f32(const double* macro, const u
             typedef float f4 __attribute__((ext_vector_type(4)));
             __builtin_nontemporal_store(f4{v[c][0], v[c][1], v[c][2], v[c][3]}, reinterpret_cast<f4*>(dst));
         } else {
-            for (int e = 0; e < 4; e++)
+            for (int e = 0; e < PT; e++)
                 if (i + e < nx) dst[e] = v[c][e];
         }
     }
@@ -624,16 +625,21 @@ hipError_t launch_macros_f32(const double* macro, const uint8_t* kind, int64_t n
                              int64_t nxp, int64_t nyp, int64_t ns, float* rho, float* u, hipStream_t s) {
     const int64_t nbox = nx * ny * nz;
     if (nbox <= 0) return hipSuccess;
-    const int64_t nq = (nx + 3) / 4, quads = nq * ny * nz;
-    const dim3 g((unsigned)((quads + 255) / 256));
     const bool vec = nx % 4 == 0 && (uintptr_t)rho % 16 == 0 && (uintptr_t)u % 16 == 0;
+    // rows that are not whole aligned quads: one point per thread, so that the lanes' 4-byte stores lie side by side
+    // (871 x 435 x 435: 0.85 ms; with four points a thread 100 steps and this took 10.17 ms, now 9.75); beyond
+    // 32-bit indices four, to stay within a launch
+    const bool one = !vec && nbox <= 0xffffff00ll;
+    const int64_t nq = one ? nx : (nx + 3) / 4, quads = nq * ny * nz;
+    const dim3 g((unsigned)((quads + 255) / 256));
     const bool wide = quads > 0xffffff00ll;  // 32-bit quad indices otherwise: their divisions are far cheaper
-#define PV_MACROS(V, I) \
-    hipLaunchKernelGGL((k_macros_f32<V, I>), g, dim3(256), 0, s, macro, kind, nx, (uint32_t)ny, nbox, (I)nq, (I)quads, nxp, nyp, ns, rho, u)
-    if (vec && wide) PV_MACROS(true, int64_t);
-    else if (vec) PV_MACROS(true, uint32_t);
-    else if (wide) PV_MACROS(false, int64_t);
-    else PV_MACROS(false, uint32_t);
+#define PV_MACROS(V, PT, I) \
+    hipLaunchKernelGGL((k_macros_f32<V, PT, I>), g, dim3(256), 0, s, macro, kind, nx, (uint32_t)ny, nbox, (I)nq, (I)quads, nxp, nyp, ns, rho, u)
+    if (vec && wide) PV_MACROS(true, 4, int64_t);
+    else if (vec) PV_MACROS(true, 4, uint32_t);
+    else if (one) PV_MACROS(false, 1, uint32_t);
+    else if (wide) PV_MACROS(false, 4, int64_t);
+    else PV_MACROS(false, 4, uint32_t);
 #undef PV_MACROS
     return hipGetLastError();
 }

@@ -353,14 +353,14 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(pvnet_wgrad a, int M, int K,
     const int64_t off = ((int64_t)dz * h + dy) * w + dx;
     const bool dcol = drole && n0 + nc * 8 < a.cout;
 
-    f32x4 acc[BN / 16], accb[BN / 16];
-    for (int j = 0; j < BN / 16; j++) acc[j] = accb[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // the bias gradient: dy against ones, in one wave of the blocks of the first k-values (a launch of column sums
-    // before, 3.7 us: 4000 x 80 -> 32 pointwise, all three passes 32.1 -> 29.1 us)
-    const bool dob = dboff >= 0 && blockIdx.x == 0 && __builtin_amdgcn_readfirstlane(wv) == 0;
-    bf16x8 ones;
-#pragma unroll
-    for (int e = 0; e < 8; e++) ones[e] = (__bf16)1.0f;
+    f32x4 acc[BN / 16];
+    for (int j = 0; j < BN / 16; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // the bias gradient: dy against ones, in the blocks of the first k-values, wave j taking the 16 channels j (a launch
+    // of column sums before, 3.7 us: 4000 x 80 -> 32 pointwise, all three passes 32.1 -> 29.1 us).  One accumulator a
+    // wave, and the ones made where they are used: with all four accumulators in one wave the kernel had 162 registers
+    // instead of 104 (8 x 24^3, 27 taps, 64 -> 64: 139 us, 108 so; 224 -> 64: 426 and 332).
+    const int bj = dboff >= 0 && blockIdx.x == 0 ? __builtin_amdgcn_readfirstlane(wv) : -1;
+    f32x4 accb = f32x4{0.f, 0.f, 0.f, 0.f};
 
     uint4 r[8];
     auto load = [&](int mbase) {
@@ -417,17 +417,20 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(pvnet_wgrad a, int M, int K,
             for (int j = 0; j < BN / 16; j++) {
                 const bf16x8 ad = *(const bf16x8*)(As + (j * 16 + c16) * PW + kk * 32 + g * 8);
                 acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ad, bx, acc[j], 0, 0, 0);
-                if (dob) accb[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ad, ones, accb[j], 0, 0, 0);
+                if (j == bj) {
+                    uint4 ones = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
+                    asm volatile("" : "+v"(ones.x), "+v"(ones.y), "+v"(ones.z), "+v"(ones.w));  // not kept through the loop
+                    accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ad, *reinterpret_cast<const bf16x8*>(&ones), accb, 0, 0, 0);
+                }
             }
         }
         __syncthreads();
     }
-    if (dob && c16 == 0)  // every column holds the sum of its row's channel
-        for (int j = 0; j < BN / 16; j++)
-            for (int e = 0; e < 4; e++) {
-                const int n = n0 + j * 16 + g * 4 + e;
-                if (n < a.cout) a.ws[dboff + (int64_t)split * a.cout + n] = accb[j][e];
-            }
+    if (bj >= 0 && bj < BN / 16 && c16 == 0)  // every column holds the sum of its row's channel
+        for (int e = 0; e < 4; e++) {
+            const int n = n0 + bj * 16 + g * 4 + e;
+            if (n < a.cout) a.ws[dboff + (int64_t)split * a.cout + n] = accb[e];
+        }
 
     const int kk = k0 + wv * 16 + c16;
     if (kk >= K) return;

@@ -335,7 +335,8 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(pvnet_wgrad a, int M, int K,
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     const int g = lane >> 4, c16 = lane & 15;
     const int k0 = blockIdx.x * 64, n0 = blockIdx.y * BN, split = blockIdx.z;
-    const int mb = split * mchunk, me = min(M, mb + mchunk);
+    // voxel numbers are unsigned: those of a fill's end may lie beyond 2^31
+    const uint32_t mb = (uint32_t)split * (uint32_t)mchunk, me = min((uint32_t)M, mb + (uint32_t)mchunk);
     const int d = a.s.d, h = a.s.h, w = a.s.w;
 
     // roles: x blocks (t < 128): voxel group mg, k chunk kc; dy blocks (128 <= t < 128 + 2 BN)
@@ -363,15 +364,16 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(pvnet_wgrad a, int M, int K,
     f32x4 accb = f32x4{0.f, 0.f, 0.f, 0.f};
 
     uint4 r[8];
-    auto load = [&](int mbase) {
-        const int m0 = mbase + mg * 8;
+    auto load = [&](uint32_t mbase) {
+        const uint32_t m0 = mbase + mg * 8;
         if (xrole) {
-            int x = m0 % w, tq = m0 / w, y = tq % h, z = (tq / h) % d;
+            const uint32_t tq = m0 / (uint32_t)w;
+            int x = m0 % (uint32_t)w, y = tq % (uint32_t)h, z = (tq / (uint32_t)h) % (uint32_t)d;
             const bool up = PARTS && ci < pq.cup;
-            int bz = tq / h - z;  // planes of the boxes before
+            int bz = (int)(tq / (uint32_t)h) - z;  // planes of the boxes before
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                const int m = m0 + i;
+                const uint32_t m = m0 + i;
                 const int z2 = z + dz, y2 = y + dy, x2 = x + dx;
                 const bool in = kin && m < me && (unsigned)z2 < (unsigned)d && (unsigned)y2 < (unsigned)h &&
                                 (unsigned)x2 < (unsigned)w;
@@ -391,7 +393,7 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(pvnet_wgrad a, int M, int K,
         } else {
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                const int m = m0 + i;
+                const uint32_t m = m0 + i;
                 r[i] = make_uint4(0, 0, 0, 0);
                 if (dcol && m < me) r[i] = *(const uint4*)(a.dy + (int64_t)m * a.lddy + n0 + nc * 8);
             }
@@ -399,7 +401,7 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(pvnet_wgrad a, int M, int K,
     };
 
     if (mb < me) load(mb);
-    for (int mbase = mb; mbase < me; mbase += BMW) {
+    for (uint32_t mbase = mb; mbase < me; mbase += BMW) {
         if (xrole || drole) {
             uint4 o[8];
             transpose8(r, o);

@@ -270,8 +270,8 @@ __global__ __launch_bounds__(256) void k_wgrad_pw(const pvnet_wgrad a, const int
     const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint4*)&sm[wv][0][0];
-    // chunks wv, wv + 4, .. of the block's run
-    const int c0 = blockIdx.x * per, c1 = min((M + WPW_VOX - 1) / WPW_VOX, c0 + per);
+    // chunks wv, wv + 4, .. of the block's run (M + WPW_VOX may not fit 32 bits)
+    const int c0 = blockIdx.x * per, c1 = min((M - 1) / WPW_VOX + 1, c0 + per);
     auto stage = [&](int c, int buf) {
 #pragma unroll
         for (int i = 0; i < UN / 64; i++) {

@@ -24,21 +24,6 @@
 // 160->160 96 -> 46; 1 x 24 x 24 x 48 64->64 40 -> 24; 3 x 20 x 18 x 28 160->64 96 -> 40.
 #pragma once
 
-
-// one tile plan; LDS quantities in 16-byte units (8 channels of one voxel)
-struct MarchPlan {
-    int32_t tx, ty, ntx, nty;  // tile and tiles per plane
-    int32_t zseg, nzs;         // output planes per block, runs per box
-    int32_t hx, hp;            // halo row pitch, halo units of one channel chunk
-    int32_t su;                // units of one plane slot
-    int32_t nsteps, ng;        // k-steps, channel groups
-    int32_t K;
-    int32_t g;                 // channel chunks interleaved per voxel in LDS (2, or 1 for odd cin / 8)
-    int32_t roll, rt, wm;      // kernel and template arguments
-    int32_t wx, wn;            // compute waves over voxels and over channel tiles (ring: 4, 1)
-    int32_t lds;               // bytes
-};
-
 __device__ uint4 g_march_zero[4];  // source of the units outside the box
 
 // 16 bytes per lane from src to LDS byte address lds + 16 * lane.  Written as one asm statement because the
@@ -429,114 +414,6 @@ inline MarchKernel march_kernel(const MarchPlan& p) {
         case 6: return march_kernel_rt<6>(p);
         default: return nullptr;
     }
-}
-
-// The plan of a convolution: every tile, run length, wave split and place of the weights that fits is priced
-// and the cheapest is taken.  The price is the time of a block that is either alone on its CU (a chain of
-// k-steps and planes with their latencies) or one of cc that share the CU's matrix cores (m: 16 clocks an MFMA
-// and SIMD), its LDS (l), its L1 (l1: weights read from memory) and the way to memory (io), times the rounds
-// of blocks the device needs.  The constants, in clocks, were fitted to 56,000 timed plans of 49 layers (cin
-// 8-224, cout 8-224, 2,048 to 7.1 M voxels, whole and ragged): over those the plan taken is 7% (mean) and at
-// most 35% (a 6 us layer) slower than the best one timed.
-struct MarchKey {
-    pvnet_shape s;
-    int32_t cin, cout;
-    bool operator==(const MarchKey& o) const {
-        return s.nb == o.s.nb && s.d == o.s.d && s.h == o.s.h && s.w == o.s.w && cin == o.cin && cout == o.cout;
-    }
-};
-
-inline bool march_search(const MarchKey& c, MarchPlan& best) {
-    const int steps = (27 * c.cin + BK - 1) / BK, ct = (c.cout + 15) / 16, cch = c.cin / 8;
-    const int w = c.s.w, h = c.s.h, d = c.s.d;
-    double best_cost = 0;
-    auto axis = [](int n, const int* cut, int ncut, const int* fix, int nfix, int* out) {
-        int k = 0;
-        auto add = [&](int v) {
-            if (v < 1 || v > n) return;
-            for (int i = 0; i < k; i++) if (out[i] == v) return;
-            out[k++] = v;
-        };
-        for (int i = 0; i < ncut; i++) add((n + cut[i] - 1) / cut[i]);
-        for (int i = 0; i < nfix; i++) add(fix[i]);
-        return k;
-    };
-    static const int cut[] = {1, 2, 3, 4, 5, 6, 8, 12, 16, 24}, fixx[] = {8, 12, 16, 24}, fixy[] = {4, 6, 8, 12, 16};
-    int xs[16], ys[16], zs[16];
-    const int nx = axis(w, cut, 8, fixx, 4, xs), ny = axis(h, cut, 8, fixy, 5, ys), nz = axis(d, cut, 10, fixy, 0, zs);
-    for (int roll = 0; roll < 2; roll++) {
-        if (roll ? c.cin % BK != 0 : c.cin > 128) continue;  // a ring of more channels leaves tiles too small
-        const int np = roll ? 2 : 4, sp = roll ? steps / 3 : steps;
-        for (int ix = 0; ix < nx; ix++)
-            for (int iy = 0; iy < ny; iy++) {
-                const int tx = xs[ix], ty = ys[iy], vox = tx * ty;
-                if (vox > 384 || (vox < 48 && vox < w * h)) continue;
-                const int hp = (tx + 2) * (ty + 2), nu = cch * hp, su = (nu + 63) / 64 * 64;
-                if (16 * np * su > 160 * 1024) continue;
-                const double tiles = (double)((w + tx - 1) / tx) * ((h + ty - 1) / ty) * c.s.nb;
-                for (int wx = roll ? 1 : 4; wx <= (roll ? 4 : 4); wx++) {
-                    int rt = (vox + 16 * wx - 1) / (16 * wx);
-                    if (rt > (roll ? 5 : 6)) continue;
-                    if (!roll && rt == 5) rt = 6;
-                    if (vox < 48 ? false : vox < 16 * wx * rt * 0.6) continue;
-                    for (int wn = 1; wn <= (roll ? 5 : 1) && wn <= ct; wn++) {
-                        const int W = wx * wn;
-                        if (roll && (W < 2 || W > 5)) continue;
-                        for (int wm = 0; wm < (roll ? 2 : 3); wm++) {
-                            if (wm == 2 && steps != 7 && steps != 14 && steps != 21 && !(steps == 41 && rt <= 4)) continue;
-                            const int lds = 16 * (np * su + (wm == 1 ? 64 * wn * steps : 0)) + 4 * (np * 4 * sp + nu);
-                            if (lds > 160 * 1024) continue;
-                            const int vg = std::min(256, ((roll ? 20 * rt + 108 : 18 * rt + 60 + (wm == 2 ? 4 * steps : 16)) + 7) / 8 * 8);
-                            const int wt = W + roll;
-                            const double cc = std::max(1, std::min({160 * 1024 / lds, 4 * (512 / vg) / wt, 8}));
-                            for (int iz = 0; iz < nz; iz++) {
-                                const int nzs = (d + zs[iz] - 1) / zs[iz];
-                                const double za = (double)d / nzs, pl = za + 2;
-                                const double B = tiles * nzs * ((ct + wn - 1) / wn);
-                                const double nst = roll ? sp * pl : steps * za, mf = steps * za * rt;
-                                const double xr = nst * rt, wr = wm == 2 ? 0 : roll ? sp * (3 * za + 2) : steps * za;
-                                const double fill = wm == 1 ? 250.0 * steps * wn : 0.0;
-                                const double m = 4 * mf * W, l = 1.25 * (xr + (wm == 1 ? wr : 0)) * W, l1 = wm == 0 ? 25 * wr * W : 0.0,
-                                             io = 0.164 * pl * nu + 0.113 * vox * za * wn * 16;
-                                const double thr = (0.585 * std::max({m, l, l1, io}) + 0.337 * (m + l + l1 + io) + 0.5 * fill) *
-                                                   (1 + 0.43 / (cc * W));
-                                const double step = 32 + (wm == 0 ? 51 : 0) + 16 * mf / nst * std::max(1.0, W / 4.0);
-                                const double lat = 1730 + fill + nst * step + pl * (80 + 2.1 * nu / (roll ? 1 : 4));
-                                const double cost = B <= 256 * cc ? std::max(lat, thr * std::ceil(B / 256))
-                                                                  : std::max(lat, thr * cc) * std::ceil(B / (256 * cc));
-                                if (best_cost == 0 || cost < best_cost) {
-                                    best_cost = cost;
-                                    best = MarchPlan{tx, ty, (w + tx - 1) / tx, (h + ty - 1) / ty, zs[iz], nzs, tx + 2, hp, su, steps,
-                                                     (ct + wn - 1) / wn, 27 * c.cin, cch % 2 ? 1 : 2, roll, rt, wm, wx, wn, lds};
-                                }
-                            }
-                        }
-                    }
-                }
-            }
-    }
-    return best_cost > 0;
-}
-
-// The plan of a shape, kept per thread for the shapes used last (a plan is a pure function of its key).
-template <class Plan, class Search>
-bool kept_plan(const MarchKey& key, Plan& p, Search search) {
-    struct Slot {
-        MarchKey key;
-        Plan plan;
-        int ok;  // 0 empty, 1 plan, 2 no plan fits
-    };
-    constexpr int SLOTS = 128;
-    thread_local Slot slots[SLOTS];
-    uint32_t hsh = 2166136261u;
-    for (int32_t v : {key.s.nb, key.s.d, key.s.h, key.s.w, key.cin, key.cout}) hsh = (hsh ^ (uint32_t)v) * 16777619u;
-    Slot& sl = slots[(hsh ^ (hsh >> 15)) % SLOTS];
-    if (!sl.ok || !(sl.key == key)) {
-        sl.key = key;
-        sl.ok = search(key, sl.plan) ? 1 : 2;
-    }
-    p = sl.plan;
-    return sl.ok == 1;
 }
 
 inline bool march_plan(const pvnet_conv& c, MarchPlan& p) { return kept_plan<MarchPlan>(MarchKey{c.s, c.cin, c.cout}, p, march_search); }

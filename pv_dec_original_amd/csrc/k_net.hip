@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "../../include/pvnet.h"
+#include "march_plans.hpp"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -47,7 +48,6 @@ int fail(int code, const std::string& msg) {
         if (e_ != hipSuccess) return fail(2, std::string("launch: ") + hipGetErrorString(e_)); \
     } while (0)
 
-constexpr int BK = 32;  // k-values per MFMA step
 constexpr int LP = 40;  // LDS row pitch in bf16 (32 + 8 padding: 80-byte rows)
 
 __device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }

@@ -1,0 +1,213 @@
+// march_plans.hpp — how the marching convolutions and weight gradients divide a layer: plans from the sizes alone.
+//
+// Host code without device parts: what conv_march.hpp and wgrad_march.hpp launch, and what a test can ask for on any
+// machine.
+#pragma once
+
+#include <algorithm>
+#include <cmath>
+#include <cstdint>
+
+#include "../../include/pvnet.h"
+
+namespace {
+
+constexpr int BK = 32;  // k-values per MFMA step
+
+// one tile plan; LDS quantities in 16-byte units (8 channels of one voxel)
+struct MarchPlan {
+    int32_t tx, ty, ntx, nty;  // tile and tiles per plane
+    int32_t zseg, nzs;         // output planes per block, runs per box
+    int32_t hx, hp;            // halo row pitch, halo units of one channel chunk
+    int32_t su;                // units of one plane slot
+    int32_t nsteps, ng;        // k-steps, channel groups
+    int32_t K;
+    int32_t g;                 // channel chunks interleaved per voxel in LDS (2, or 1 for odd cin / 8)
+    int32_t roll, rt, wm;      // kernel and template arguments
+    int32_t wx, wn;            // compute waves over voxels and over channel tiles (ring: 4, 1)
+    int32_t lds;               // bytes
+};
+
+// the shape a plan is for
+struct MarchKey {
+    pvnet_shape s;
+    int32_t cin, cout;
+    bool operator==(const MarchKey& o) const {
+        return s.nb == o.s.nb && s.d == o.s.d && s.h == o.s.h && s.w == o.s.w && cin == o.cin && cout == o.cout;
+    }
+};
+
+// The plan of a convolution: every tile, run length, wave split and place of the weights that fits is priced
+// and the cheapest is taken.  The price is the time of a block that is either alone on its CU (a chain of
+// k-steps and planes with their latencies) or one of cc that share the CU's matrix cores (m: 16 clocks an MFMA
+// and SIMD), its LDS (l), its L1 (l1: weights read from memory) and the way to memory (io), times the rounds
+// of blocks the device needs.  The constants, in clocks, were fitted to 56,000 timed plans of 49 layers (cin
+// 8-224, cout 8-224, 2,048 to 7.1 M voxels, whole and ragged): over those the plan taken is 7% (mean) and at
+// most 35% (a 6 us layer) slower than the best one timed.
+inline bool march_search(const MarchKey& c, MarchPlan& best) {
+    const int steps = (27 * c.cin + BK - 1) / BK, ct = (c.cout + 15) / 16, cch = c.cin / 8;
+    const int w = c.s.w, h = c.s.h, d = c.s.d;
+    double best_cost = 0;
+    auto axis = [](int n, const int* cut, int ncut, const int* fix, int nfix, int* out) {
+        int k = 0;
+        auto add = [&](int v) {
+            if (v < 1 || v > n) return;
+            for (int i = 0; i < k; i++) if (out[i] == v) return;
+            out[k++] = v;
+        };
+        for (int i = 0; i < ncut; i++) add((n + cut[i] - 1) / cut[i]);
+        for (int i = 0; i < nfix; i++) add(fix[i]);
+        return k;
+    };
+    static const int cut[] = {1, 2, 3, 4, 5, 6, 8, 12, 16, 24}, fixx[] = {8, 12, 16, 24}, fixy[] = {4, 6, 8, 12, 16};
+    int xs[16], ys[16], zs[16];
+    const int nx = axis(w, cut, 8, fixx, 4, xs), ny = axis(h, cut, 8, fixy, 5, ys), nz = axis(d, cut, 10, fixy, 0, zs);
+    for (int roll = 0; roll < 2; roll++) {
+        if (roll ? c.cin % BK != 0 : c.cin > 128) continue;  // a ring of more channels leaves tiles too small
+        const int np = roll ? 2 : 4, sp = roll ? steps / 3 : steps;
+        for (int ix = 0; ix < nx; ix++)
+            for (int iy = 0; iy < ny; iy++) {
+                const int tx = xs[ix], ty = ys[iy], vox = tx * ty;
+                if (vox > 384 || (vox < 48 && vox < w * h)) continue;
+                const int hp = (tx + 2) * (ty + 2), nu = cch * hp, su = (nu + 63) / 64 * 64;
+                if (16 * np * su > 160 * 1024) continue;
+                const double tiles = (double)((w + tx - 1) / tx) * ((h + ty - 1) / ty) * c.s.nb;
+                for (int wx = roll ? 1 : 4; wx <= (roll ? 4 : 4); wx++) {
+                    int rt = (vox + 16 * wx - 1) / (16 * wx);
+                    if (rt > (roll ? 5 : 6)) continue;
+                    if (!roll && rt == 5) rt = 6;
+                    if (vox < 48 ? false : vox < 16 * wx * rt * 0.6) continue;
+                    for (int wn = 1; wn <= (roll ? 5 : 1) && wn <= ct; wn++) {
+                        const int W = wx * wn;
+                        if (roll && (W < 2 || W > 5)) continue;
+                        for (int wm = 0; wm < (roll ? 2 : 3); wm++) {
+                            if (wm == 2 && steps != 7 && steps != 14 && steps != 21 && !(steps == 41 && rt <= 4)) continue;
+                            const int lds = 16 * (np * su + (wm == 1 ? 64 * wn * steps : 0)) + 4 * (np * 4 * sp + nu);
+                            if (lds > 160 * 1024) continue;
+                            const int vg = std::min(256, ((roll ? 20 * rt + 108 : 18 * rt + 60 + (wm == 2 ? 4 * steps : 16)) + 7) / 8 * 8);
+                            const int wt = W + roll;
+                            const double cc = std::max(1, std::min({160 * 1024 / lds, 4 * (512 / vg) / wt, 8}));
+                            for (int iz = 0; iz < nz; iz++) {
+                                const int nzs = (d + zs[iz] - 1) / zs[iz];
+                                const double za = (double)d / nzs, pl = za + 2;
+                                const double B = tiles * nzs * ((ct + wn - 1) / wn);
+                                const double nst = roll ? sp * pl : steps * za, mf = steps * za * rt;
+                                const double xr = nst * rt, wr = wm == 2 ? 0 : roll ? sp * (3 * za + 2) : steps * za;
+                                const double fill = wm == 1 ? 250.0 * steps * wn : 0.0;
+                                const double m = 4 * mf * W, l = 1.25 * (xr + (wm == 1 ? wr : 0)) * W, l1 = wm == 0 ? 25 * wr * W : 0.0,
+                                             io = 0.164 * pl * nu + 0.113 * vox * za * wn * 16;
+                                const double thr = (0.585 * std::max({m, l, l1, io}) + 0.337 * (m + l + l1 + io) + 0.5 * fill) *
+                                                   (1 + 0.43 / (cc * W));
+                                const double step = 32 + (wm == 0 ? 51 : 0) + 16 * mf / nst * std::max(1.0, W / 4.0);
+                                const double lat = 1730 + fill + nst * step + pl * (80 + 2.1 * nu / (roll ? 1 : 4));
+                                const double cost = B <= 256 * cc ? std::max(lat, thr * std::ceil(B / 256))
+                                                                  : std::max(lat, thr * cc) * std::ceil(B / (256 * cc));
+                                if (best_cost == 0 || cost < best_cost) {
+                                    best_cost = cost;
+                                    best = MarchPlan{tx, ty, (w + tx - 1) / tx, (h + ty - 1) / ty, zs[iz], nzs, tx + 2, hp, su, steps,
+                                                     (ct + wn - 1) / wn, 27 * c.cin, cch % 2 ? 1 : 2, roll, rt, wm, wx, wn, lds};
+                                }
+                            }
+                        }
+                    }
+                }
+            }
+    }
+    return best_cost > 0;
+}
+
+// the plan of a weight gradient
+struct WgradMarch {
+    int32_t tx, ty, ntx, nty;   // tile (divides the plane) and tiles per plane
+    int32_t zseg, nzs;          // planes per run, runs per box
+    int32_t hx, hp, gr;         // halo row pitch and size; 32-voxel groups of a tile
+    int32_t su, fu;             // LDS units (16 bytes) of one dy and one x plane
+    int32_t cf, ns, nf;         // 16-channel tiles of x per block; blocks over the channels of dy and x
+    int32_t units, per, splits; // runs in all, runs per block, blocks over the voxels
+    int32_t lds;
+};
+
+// The plan of a weight gradient, from the sizes alone (the scratch size a caller asks for and the launch agree on
+// any device).  Tiles divide the plane, so that no operand needs masking inside a plane.  Every tile, run length
+// and CF that fits is priced as conv_march prices its plans: a block alone on its CU against the share of the
+// matrix cores, LDS and copies when cc blocks share it, plus the split partials' traffic; constants in clocks,
+// fitted to 22,000 timed plans of 18 layers.  The plan taken is 4% (mean) and at most 29% slower than the best
+// one timed over those.
+inline bool wgrad_march_search(const pvnet_shape& s, int cin, int cout, WgradMarch& best) {
+    constexpr int WANT = 768;  // blocks: three per CU
+    double best_cost = 0;
+    static const int cuts[] = {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32, 48};
+    const int ft = (cin + 15) / 16, st = (cout + 15) / 16;
+    for (int tx = 1; tx <= 256 && tx <= s.w; tx++) {
+        if (s.w % tx) continue;
+        for (int ty = 1; ty <= 64 && ty <= s.h; ty++) {
+            const int vox = tx * ty, gr = (vox + 31) / 32, hp = (tx + 2) * (ty + 2);
+            if (s.h % ty || vox > 512 || (vox < 32 && vox < s.w * s.h && tx < s.w)) continue;
+            for (int cf = 1; cf <= 3 && cf <= ft; cf++) {
+                const int su = (2 * hp + 63) / 64 * 64, fu = (2 * cf * gr * 32 + 63) / 64 * 64;
+                const int lds = 16 * (4 * su + 2 * fu) + 4 * (gr * 32 + 2 * hp + 2 * cf * gr * 32);
+                if (lds > 160 * 1024) continue;
+                const int nf = (ft + cf - 1) / cf;
+                const double c = std::max(1, std::min(160 * 1024 / lds, cf == 3 ? 3 : cf == 2 ? 4 : 6));
+                for (int cut : cuts) {
+                    if (cut > s.d) break;
+                    const int zseg = (s.d + cut - 1) / cut, nzs = (s.d + zseg - 1) / zseg;
+                    const int64_t units = (int64_t)s.nb * (s.w / tx) * (s.h / ty) * nzs;
+                    const int want = (int)std::max<int64_t>(1, std::min<int64_t>(units, WANT / (nf * st)));
+                    const int per = (int)((units + want - 1) / want), splits = (int)((units + per - 1) / per);
+                    const double B = (double)splits * nf * st, za = (double)s.d / nzs;
+                    const double lat = per * (4400 + 6.9 * hp + 830 * (za + 2) + za * gr * (500 + 168.0 * cf));
+                    const double thr = per * za * (gr * std::max(112.0 * cf, 32.6 * (7 + cf)) + 0.81 * (hp + cf * gr * 32));
+                    const double cc = std::min(c, std::ceil(B / 256));
+                    const double cost = (std::max(lat, thr * cc) + 0.36 * (lat + thr * cc)) * std::ceil(B / (256 * c)) +
+                                        0.2 * splits * cout * cin;
+                    if (best_cost == 0 || cost < best_cost) {
+                        best_cost = cost;
+                        best = WgradMarch{tx, ty, s.w / tx, s.h / ty, zseg, nzs, tx + 2, hp, gr, su, fu, cf, st, nf, (int)units, per, splits, lds};
+                    }
+                }
+            }
+        }
+    }
+    return best_cost > 0;
+}
+
+// The plan of a shape, a pure function of its key, searched once per thread and kept with the others the thread has
+// used.  A key sits in the first free slot from its hash on, so that no shape drives out another; a table that is three
+// quarters full starts over.  (A network's training step asks for 41 plans; a search takes 10 to 90 us.)
+template <class Plan, class Search>
+bool kept_plan(const MarchKey& key, Plan& p, Search search) {
+    struct Slot {
+        MarchKey key;
+        Plan plan;
+        int ok;  // 0 empty, 1 plan, 2 no plan
+    };
+    constexpr int SLOTS = 512, FULL = SLOTS / 4 * 3;
+    thread_local Slot slots[SLOTS];
+    thread_local int used = 0;
+    uint32_t hsh = 2166136261u;
+    for (int32_t v : {key.s.nb, key.s.d, key.s.h, key.s.w, key.cin, key.cout}) hsh = (hsh ^ (uint32_t)v) * 16777619u;
+    const uint32_t home = (hsh ^ (hsh >> 15)) % SLOTS;
+    uint32_t i = home;
+    while (slots[i].ok && !(slots[i].key == key)) i = (i + 1) % SLOTS;
+    if (!slots[i].ok) {
+        if (used == FULL) {
+            for (Slot& s : slots) s.ok = 0;
+            used = 0;
+            i = home;
+        }
+        slots[i].key = key;
+        slots[i].ok = search(key, slots[i].plan) ? 1 : 2;
+        used++;
+    }
+    p = slots[i].plan;
+    return slots[i].ok == 1;
+}
+
+inline bool wgrad_march_plan(const pvnet_shape& s, int cin, int cout, WgradMarch& p) {
+    return kept_plan<WgradMarch>(MarchKey{s, cin, cout}, p, [](const MarchKey& k, WgradMarch& q) {
+        return (int64_t)k.s.nb * k.s.d * k.s.h * k.s.w < (int64_t)1 << 31 && wgrad_march_search(k.s, k.cin, k.cout, q);
+    });
+}
+
+}  // namespace

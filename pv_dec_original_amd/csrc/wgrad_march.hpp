@@ -20,16 +20,6 @@
 // 8 x 24^3 224->64 339 -> 127, 64->64 115 -> 55; 8 x 12^3 160->160 111 -> 62; 3 x 20 x 18 x 28 64->160 92 -> 50.
 #pragma once
 
-struct WgradMarch {
-    int32_t tx, ty, ntx, nty;   // tile (divides the plane) and tiles per plane
-    int32_t zseg, nzs;          // planes per run, runs per box
-    int32_t hx, hp, gr;         // halo row pitch and size; 32-voxel groups of a tile
-    int32_t su, fu;             // LDS units (16 bytes) of one dy and one x plane
-    int32_t cf, ns, nf;         // 16-channel tiles of x per block; blocks over the channels of dy and x
-    int32_t units, per, splits; // runs in all, runs per block, blocks over the voxels
-    int32_t lds;
-};
-
 typedef short tr4 __attribute__((ext_vector_type(4)));
 
 // 4 voxels (rows of 16 channels, 32 bytes apart) x this lane's channel: lane 16 q + c of the wave addresses
@@ -193,57 +183,6 @@ typedef void (*WgradKernel)(const pvnet_wgrad, const WgradMarch, const NetParts,
 
 inline WgradKernel wgrad_march_kernel(const WgradMarch& p) {
     return p.cf == 1 ? k_wgrad_march<1> : p.cf == 2 ? k_wgrad_march<2> : k_wgrad_march<3>;
-}
-
-// The plan of a weight gradient, from the sizes alone (the scratch size a caller asks for and the launch agree on
-// any device).  Tiles divide the plane, so that no operand needs masking inside a plane.  Every tile, run length
-// and CF that fits is priced as conv_march prices its plans: a block alone on its CU against the share of the
-// matrix cores, LDS and copies when cc blocks share it, plus the split partials' traffic; constants in clocks,
-// fitted to 22,000 timed plans of 18 layers.  The plan taken is 4% (mean) and at most 29% slower than the best
-// one timed over those.
-inline bool wgrad_march_search(const pvnet_shape& s, int cin, int cout, WgradMarch& best) {
-    constexpr int WANT = 768;  // blocks: three per CU
-    double best_cost = 0;
-    static const int cuts[] = {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32, 48};
-    const int ft = (cin + 15) / 16, st = (cout + 15) / 16;
-    for (int tx = 1; tx <= 256 && tx <= s.w; tx++) {
-        if (s.w % tx) continue;
-        for (int ty = 1; ty <= 64 && ty <= s.h; ty++) {
-            const int vox = tx * ty, gr = (vox + 31) / 32, hp = (tx + 2) * (ty + 2);
-            if (s.h % ty || vox > 512 || (vox < 32 && vox < s.w * s.h && tx < s.w)) continue;
-            for (int cf = 1; cf <= 3 && cf <= ft; cf++) {
-                const int su = (2 * hp + 63) / 64 * 64, fu = (2 * cf * gr * 32 + 63) / 64 * 64;
-                const int lds = 16 * (4 * su + 2 * fu) + 4 * (gr * 32 + 2 * hp + 2 * cf * gr * 32);
-                if (lds > 160 * 1024) continue;
-                const int nf = (ft + cf - 1) / cf;
-                const double c = std::max(1, std::min(160 * 1024 / lds, cf == 3 ? 3 : cf == 2 ? 4 : 6));
-                for (int cut : cuts) {
-                    if (cut > s.d) break;
-                    const int zseg = (s.d + cut - 1) / cut, nzs = (s.d + zseg - 1) / zseg;
-                    const int64_t units = (int64_t)s.nb * (s.w / tx) * (s.h / ty) * nzs;
-                    const int want = (int)std::max<int64_t>(1, std::min<int64_t>(units, WANT / (nf * st)));
-                    const int per = (int)((units + want - 1) / want), splits = (int)((units + per - 1) / per);
-                    const double B = (double)splits * nf * st, za = (double)s.d / nzs;
-                    const double lat = per * (4400 + 6.9 * hp + 830 * (za + 2) + za * gr * (500 + 168.0 * cf));
-                    const double thr = per * za * (gr * std::max(112.0 * cf, 32.6 * (7 + cf)) + 0.81 * (hp + cf * gr * 32));
-                    const double cc = std::min(c, std::ceil(B / 256));
-                    const double cost = (std::max(lat, thr * cc) + 0.36 * (lat + thr * cc)) * std::ceil(B / (256 * c)) +
-                                        0.2 * splits * cout * cin;
-                    if (best_cost == 0 || cost < best_cost) {
-                        best_cost = cost;
-                        best = WgradMarch{tx, ty, s.w / tx, s.h / ty, zseg, nzs, tx + 2, hp, gr, su, fu, cf, st, nf, (int)units, per, splits, lds};
-                    }
-                }
-            }
-        }
-    }
-    return best_cost > 0;
-}
-
-inline bool wgrad_march_plan(const pvnet_shape& s, int cin, int cout, WgradMarch& p) {
-    return kept_plan<WgradMarch>(MarchKey{s, cin, cout}, p, [](const MarchKey& k, WgradMarch& q) {
-        return (int64_t)k.s.nb * k.s.d * k.s.h * k.s.w < (int64_t)1 << 31 && wgrad_march_search(k.s, k.cin, k.cout, q);
-    });
 }
 
 // What one call needs beyond a plan: plane offsets fit 32 bits (as in conv_march, PVNET_GATHER and pointwise

@@ -1,0 +1,46 @@
+"""The planner of the marching kernels on the host: plans are searched once and kept."""
+import random
+
+import pytest
+
+from pv_dec_original_amd.warmnet import UNetSpec
+from tests import plan_probe as P
+
+
+def _unet_keys(shape, levels=(16, 32, 64, 160)):
+    """(shape, cin, cout) of every 3x3x3 convolution of a training step: forward and input gradient."""
+    nb, d, h, w = shape
+    keys = []
+    for lay in UNetSpec(levels).layers:
+        if lay.ntaps == 27:
+            k = len(levels) - 1 if lay.name.startswith("bt") else int(lay.name[1:-1])
+            s = (nb, d >> k, h >> k, w >> k)
+            keys += [(s, lay.cin, lay.cout), (s, lay.cout, lay.cin)]
+    return keys
+
+
+def test_steady_calls_do_not_search():
+    r = random.Random(1)
+    shapes = [(8, 96, 96, 96), (1, 96, 96, 192)]
+    shapes += [(r.choice([1, 2, 4, 8]),) + tuple(8 * r.randint(2, 14) for _ in range(3)) for _ in range(12)]
+    for shape in shapes:
+        keys = _unet_keys(shape)
+        for k in keys:
+            assert P.kept(*k)[1]
+        n = P.kept(*keys[0])[0]
+        for k in keys:
+            assert P.kept(*k) == (n, True), (shape, k)
+
+
+def test_table_starts_over_when_full():
+    n0 = None
+    for i in range(1200):
+        n, same = P.kept((1, 4, 4 + i % 40, 4 + i // 40), 16, 16)
+        assert same
+        n0 = n if n0 is None else n0
+    assert n - n0 >= 1199  # each shape was new
+
+
+@pytest.mark.parametrize("key", [((0x7fff, 1, 1, 1), 8, 8), ((1, 1, 1, 4096), 8, 8), ((1, 512, 1, 1), 128, 256)])
+def test_odd_shapes_plan_or_not(key):
+    assert P.kept(*key)[1]

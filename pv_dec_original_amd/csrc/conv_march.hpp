@@ -416,8 +416,6 @@ inline MarchKernel march_kernel(const MarchPlan& p) {
     }
 }
 
-inline bool march_plan(const pvnet_conv& c, MarchPlan& p) { return kept_plan<MarchPlan>(MarchKey{c.s, c.cin, c.cout}, p, march_search); }
-
 // outputs (and ReLU mask) that can be accessed four channels at a time
 inline bool rows_by_four(const pvnet_conv& c) {
     if (c.cout % 4 || c.ldy % 4 || (uintptr_t)c.y % (c.flags & PVNET_F32OUT ? 16 : 8)) return false;

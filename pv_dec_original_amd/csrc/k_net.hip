@@ -958,7 +958,7 @@ int conv_launch(const pvnet_conv* c, const NetParts& pq, void* stream, const cha
     const int K = c->ntaps * c->cin;
     const bool parts = pq.cup || pq.c0;
     MarchPlan mp;
-    if (march_ok(*c, pq) && march_plan(*c, mp)) {
+    if (march_ok(*c, pq) && march_plan(c->s, c->cin, c->cout, mp)) {
         const unsigned nblk = (unsigned)mp.ntx * mp.nty * mp.nzs * mp.ng * c->s.nb;
         hipLaunchKernelGGL(march_kernel(mp), dim3(nblk), dim3(64 * (mp.wx * mp.wn + mp.roll)), mp.lds, st, *c, mp, pq);
     } else if (c->ntaps == 1 && K <= BK && c->cout <= 64 && !(c->flags & PVNET_GATHER)) {

@@ -37,17 +37,51 @@ struct MarchKey {
     }
 };
 
-// The plan of a convolution: every tile, run length, wave split and place of the weights that fits is priced
-// and the cheapest is taken.  The price is the time of a block that is either alone on its CU (a chain of
-// k-steps and planes with their latencies) or one of cc that share the CU's matrix cores (m: 16 clocks an MFMA
-// and SIMD), its LDS (l), its L1 (l1: weights read from memory) and the way to memory (io), times the rounds
-// of blocks the device needs.  The constants, in clocks, were fitted to 56,000 timed plans of 49 layers (cin
-// 8-224, cout 8-224, 2,048 to 7.1 M voxels, whole and ragged): over those the plan taken is 7% (mean) and at
-// most 35% (a 6 us layer) slower than the best one timed.
-inline bool march_search(const MarchKey& c, MarchPlan& best) {
+// What a block of the marching kernels costs.  cu: clocks of its CU, the larger part of what it asks of the matrix
+// cores, the LDS, the L1 (weights read from memory) and the way to memory plus a share of the others; alone: clocks it
+// takes by itself, a chain of k-steps and planes with their latencies.  A CU that holds c blocks needs c cu and one
+// alone, of which the longer hides part of the other; blocks beyond what the device holds come in further rounds.
+// The constants (clocks, launch in us) were fitted to 53,000 timed plans of 1,550 layers (cin 8-224, cout 8-224, 32 to
+// 4 M voxels, whole and ragged, boxes of one voxel to 200 a side): rms error 11 % (ring) and 15 % (roll); over 260
+// other layers the plan taken is 3.5 % (mean) and at most 41 % slower than the best one timed.  A plan's price decides
+// how long a call takes, never what it computes.
+struct MarchPrice {
+    double launch;
+    double mma, lds, l1, in, out;         // per MFMA, fragment read from LDS, weight fragment from L1, unit in, channel out
+    double share, few;                    // of the smaller parts; waves too few to keep the CU busy
+    double weights[3];                    // per k-step: weights read at the start (by where they are: memory, LDS, registers)
+    double start, step[3], mstep;         // alone: the start, a k-step, its MFMAs
+    double plane, unit;                   // a plane and its units
+    double hide;                          // of the shorter of the two
+};
+constexpr MarchPrice RING_PRICE{2.78, 0.0, 5.31, 26.2, 0.372, 0.188, 0.477, 1.05, {0, 77.7, 79.8}, 784, {20.7, 0, 0}, 0.383, 642, 1.99, 2.2};
+constexpr MarchPrice ROLL_PRICE{2.06, 0.715, 2.59, 36.1, 0.173, 0.656, 0.9, 0.0, {0, 133, 0}, 968, {0, 0, 0}, 0.644, 1490, 2.93, 0.68};
+
+// registers of a thread, as the compiler reports them (an old figure here costs time only)
+inline int march_vgprs(int roll, int rt, int wm, int steps) {
+    static const int ring[] = {0, 44, 60, 78, 100, 0, 138}, held[] = {0, 38, 46, 57, 72, 0, 102}, rolled[] = {0, 116, 149, 182, 218, 256};
+    return roll ? std::min(256, rolled[rt] + 15 * wm) : wm == 2 ? held[rt] + 4 * steps : ring[rt];
+}
+
+// blocks a CU holds at once: 160 KB of LDS in pieces of 1,280 bytes, 512 registers a SIMD lane
+inline int blocks_per_cu(int lds, int vgprs, int waves) {
+    constexpr int LDS = 160 * 1024, PIECE = 1280;
+    return std::max(1, std::min(LDS / ((lds + PIECE - 1) / PIECE * PIECE), 4 * (512 / ((vgprs + 7) / 8 * 8)) / waves));
+}
+
+// us of `blocks` blocks of which a CU holds cc, on 256 CUs
+inline double rounds_us(double blocks, int cc, double cu, double alone, double hide) {
+    const double rounds = std::ceil(blocks / (256.0 * cc)), rest = std::ceil((blocks - (rounds - 1) * 256 * cc) / 256);
+    auto one = [&](double c) { return std::max(alone, cu * c) + hide * std::min(alone, cu * c); };
+    return ((rounds - 1) * one(cc) + one(rest)) / 2400;
+}
+
+// The plan of a convolution: every tile, run length, wave split and place of the weights that fits is priced and the
+// cheapest is taken; us: its price.
+inline bool march_search(const MarchKey& c, MarchPlan& best, double& us) {
     const int steps = (27 * c.cin + BK - 1) / BK, ct = (c.cout + 15) / 16, cch = c.cin / 8;
     const int w = c.s.w, h = c.s.h, d = c.s.d;
-    double best_cost = 0;
+    us = 0;
     auto axis = [](int n, const int* cut, int ncut, const int* fix, int nfix, int* out) {
         int k = 0;
         auto add = [&](int v) {
@@ -84,26 +118,24 @@ inline bool march_search(const MarchKey& c, MarchPlan& best) {
                             if (wm == 2 && steps != 7 && steps != 14 && steps != 21 && !(steps == 41 && rt <= 4)) continue;
                             const int lds = 16 * (np * su + (wm == 1 ? 64 * wn * steps : 0)) + 4 * (np * 4 * sp + nu);
                             if (lds > 160 * 1024) continue;
-                            const int vg = std::min(256, ((roll ? 20 * rt + 108 : 18 * rt + 60 + (wm == 2 ? 4 * steps : 16)) + 7) / 8 * 8);
-                            const int wt = W + roll;
-                            const double cc = std::max(1, std::min({160 * 1024 / lds, 4 * (512 / vg) / wt, 8}));
+                            const int cc = std::min(16, blocks_per_cu(lds, march_vgprs(roll, rt, wm, steps), W + roll));
+                            const MarchPrice& P = roll ? ROLL_PRICE : RING_PRICE;
+                            const double wfill = P.weights[wm] * steps * (wm == 1 ? wn : 1);
                             for (int iz = 0; iz < nz; iz++) {
                                 const int nzs = (d + zs[iz] - 1) / zs[iz];
                                 const double za = (double)d / nzs, pl = za + 2;
                                 const double B = tiles * nzs * ((ct + wn - 1) / wn);
                                 const double nst = roll ? sp * pl : steps * za, mf = steps * za * rt;
                                 const double xr = nst * rt, wr = wm == 2 ? 0 : roll ? sp * (3 * za + 2) : steps * za;
-                                const double fill = wm == 1 ? 250.0 * steps * wn : 0.0;
-                                const double m = 4 * mf * W, l = 1.25 * (xr + (wm == 1 ? wr : 0)) * W, l1 = wm == 0 ? 25 * wr * W : 0.0,
-                                             io = 0.164 * pl * nu + 0.113 * vox * za * wn * 16;
-                                const double thr = (0.585 * std::max({m, l, l1, io}) + 0.337 * (m + l + l1 + io) + 0.5 * fill) *
-                                                   (1 + 0.43 / (cc * W));
-                                const double step = 32 + (wm == 0 ? 51 : 0) + 16 * mf / nst * std::max(1.0, W / 4.0);
-                                const double lat = 1730 + fill + nst * step + pl * (80 + 2.1 * nu / (roll ? 1 : 4));
-                                const double cost = B <= 256 * cc ? std::max(lat, thr * std::ceil(B / 256))
-                                                                  : std::max(lat, thr * cc) * std::ceil(B / (256 * cc));
-                                if (best_cost == 0 || cost < best_cost) {
-                                    best_cost = cost;
+                                const double m = P.mma * mf * W, l = P.lds * (xr + (wm == 1 ? wr : 0)) * W,
+                                             l1 = wm == 0 ? P.l1 * wr * W : 0.0, io = P.in * pl * nu + P.out * vox * za * wn * 16;
+                                const double top = std::max({m, l, l1, io});
+                                const double cu = (top + P.share * (m + l + l1 + io - top)) * (1 + P.few / (cc * W)) + 0.5 * wfill;
+                                const double step = P.step[wm] + P.mstep * 16 * mf / nst * std::max(1.0, W / 4.0);
+                                const double alone = P.start + wfill + nst * step + pl * (P.plane + P.unit * nu / (roll ? 1 : 4));
+                                const double cost = P.launch + rounds_us(B, cc, cu, alone, P.hide);
+                                if (us == 0 || cost < us) {
+                                    us = cost;
                                     best = MarchPlan{tx, ty, (w + tx - 1) / tx, (h + ty - 1) / ty, zs[iz], nzs, tx + 2, hp, su, steps,
                                                      (ct + wn - 1) / wn, 27 * c.cin, cch % 2 ? 1 : 2, roll, rt, wm, wx, wn, lds};
                                 }
@@ -113,7 +145,7 @@ inline bool march_search(const MarchKey& c, MarchPlan& best) {
                 }
             }
     }
-    return best_cost > 0;
+    return us > 0;
 }
 
 // the plan of a weight gradient
@@ -129,13 +161,13 @@ struct WgradMarch {
 
 // The plan of a weight gradient, from the sizes alone (the scratch size a caller asks for and the launch agree on
 // any device).  Tiles divide the plane, so that no operand needs masking inside a plane.  Every tile, run length
-// and CF that fits is priced as conv_march prices its plans: a block alone on its CU against the share of the
-// matrix cores, LDS and copies when cc blocks share it, plus the split partials' traffic; constants in clocks,
-// fitted to 22,000 timed plans of 18 layers.  The plan taken is 4% (mean) and at most 29% slower than the best
-// one timed over those.
-inline bool wgrad_march_search(const pvnet_shape& s, int cin, int cout, WgradMarch& best) {
+// and CF that fits is priced as above, with the sum over the splits, and the cheapest is taken; us: its price.  Fitted
+// to 41,000 timed plans of 1,550 layers, rms error 10 %; over 260 other layers the plan taken is 1.7 % (mean) and at
+// most 13 % slower than the best one timed.
+inline bool wgrad_march_search(const pvnet_shape& s, int cin, int cout, WgradMarch& best, double& us) {
     constexpr int WANT = 768;  // blocks: three per CU
-    double best_cost = 0;
+    static const int vgprs[] = {75, 113, 139};  // of CF = 1, 2, 3
+    us = 0;
     static const int cuts[] = {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32, 48};
     const int ft = (cin + 15) / 16, st = (cout + 15) / 16;
     for (int tx = 1; tx <= 256 && tx <= s.w; tx++) {
@@ -148,7 +180,7 @@ inline bool wgrad_march_search(const pvnet_shape& s, int cin, int cout, WgradMar
                 const int lds = 16 * (4 * su + 2 * fu) + 4 * (gr * 32 + 2 * hp + 2 * cf * gr * 32);
                 if (lds > 160 * 1024) continue;
                 const int nf = (ft + cf - 1) / cf;
-                const double c = std::max(1, std::min(160 * 1024 / lds, cf == 3 ? 3 : cf == 2 ? 4 : 6));
+                const int cc = blocks_per_cu(lds, vgprs[cf - 1], 4);
                 for (int cut : cuts) {
                     if (cut > s.d) break;
                     const int zseg = (s.d + cut - 1) / cut, nzs = (s.d + zseg - 1) / zseg;
@@ -156,20 +188,18 @@ inline bool wgrad_march_search(const pvnet_shape& s, int cin, int cout, WgradMar
                     const int want = (int)std::max<int64_t>(1, std::min<int64_t>(units, WANT / (nf * st)));
                     const int per = (int)((units + want - 1) / want), splits = (int)((units + per - 1) / per);
                     const double B = (double)splits * nf * st, za = (double)s.d / nzs;
-                    const double lat = per * (4400 + 6.9 * hp + 830 * (za + 2) + za * gr * (500 + 168.0 * cf));
-                    const double thr = per * za * (gr * std::max(112.0 * cf, 32.6 * (7 + cf)) + 0.81 * (hp + cf * gr * 32));
-                    const double cc = std::min(c, std::ceil(B / 256));
-                    const double cost = (std::max(lat, thr * cc) + 0.36 * (lat + thr * cc)) * std::ceil(B / (256 * c)) +
-                                        0.2 * splits * cout * cin;
-                    if (best_cost == 0 || cost < best_cost) {
-                        best_cost = cost;
+                    const double alone = per * (881 + 7.67 * hp + 1260 * (za + 2) + za * gr * (238 + 218.0 * cf));
+                    const double cu = per * za * (gr * std::max(118.0 * cf, 26.2 * (7 + cf)) + 0.66 * (hp + cf * gr * 32));
+                    const double cost = 7.18 + rounds_us(B, cc, cu, alone, 0.41) + splits * (6.72e-5 * cin * cout + 6.7e-4);
+                    if (us == 0 || cost < us) {
+                        us = cost;
                         best = WgradMarch{tx, ty, s.w / tx, s.h / ty, zseg, nzs, tx + 2, hp, gr, su, fu, cf, st, nf, (int)units, per, splits, lds};
                     }
                 }
             }
         }
     }
-    return best_cost > 0;
+    return us > 0;
 }
 
 // The plan of a shape, a pure function of its key, searched once per thread and kept with the others the thread has
@@ -204,9 +234,17 @@ bool kept_plan(const MarchKey& key, Plan& p, Search search) {
     return slots[i].ok == 1;
 }
 
+inline bool march_plan(const pvnet_shape& s, int cin, int cout, MarchPlan& p) {
+    return kept_plan<MarchPlan>(MarchKey{s, cin, cout}, p, [](const MarchKey& k, MarchPlan& q) {
+        double us;
+        return march_search(k, q, us);
+    });
+}
+
 inline bool wgrad_march_plan(const pvnet_shape& s, int cin, int cout, WgradMarch& p) {
     return kept_plan<WgradMarch>(MarchKey{s, cin, cout}, p, [](const MarchKey& k, WgradMarch& q) {
-        return (int64_t)k.s.nb * k.s.d * k.s.h * k.s.w < (int64_t)1 << 31 && wgrad_march_search(k.s, k.cin, k.cout, q);
+        double us;
+        return (int64_t)k.s.nb * k.s.d * k.s.h * k.s.w < (int64_t)1 << 31 && wgrad_march_search(k.s, k.cin, k.cout, q, us);
     });
 }
 

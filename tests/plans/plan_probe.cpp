@@ -7,31 +7,35 @@ int64_t searches = 0;
 
 extern "C" {
 
-// fields of MarchPlan; 0: no plan
-int probe_conv_plan(const pvnet_shape* s, int32_t cin, int32_t cout, int32_t* out, int32_t n) {
+// fields of MarchPlan and the price; 0: no plan
+int probe_conv_plan(const pvnet_shape* s, int32_t cin, int32_t cout, int32_t* out, int32_t n, double* us) {
     MarchPlan p{};
-    if (n != (int32_t)(sizeof(p) / 4) || !march_search(MarchKey{*s, cin, cout}, p)) return 0;
+    if (n != (int32_t)(sizeof(p) / 4) || !march_search(MarchKey{*s, cin, cout}, p, *us)) return 0;
     std::copy_n(reinterpret_cast<const int32_t*>(&p), n, out);
     return 1;
 }
 
-// fields of WgradMarch; 0: no plan
-int probe_wgrad_plan(const pvnet_shape* s, int32_t cin, int32_t cout, int32_t* out, int32_t n) {
+// fields of WgradMarch and the price; 0: no plan
+int probe_wgrad_plan(const pvnet_shape* s, int32_t cin, int32_t cout, int32_t* out, int32_t n, double* us) {
     WgradMarch p{};
-    if (n != (int32_t)(sizeof(p) / 4) || !wgrad_march_search(*s, cin, cout, p)) return 0;
+    if (n != (int32_t)(sizeof(p) / 4) || !wgrad_march_search(*s, cin, cout, p, *us)) return 0;
     std::copy_n(reinterpret_cast<const int32_t*>(&p), n, out);
     return 1;
 }
+
+int probe_blocks_per_cu(int32_t lds, int32_t vgprs, int32_t waves) { return blocks_per_cu(lds, vgprs, waves); }
 
 // searches of the kept convolution plans so far, after one more lookup; *same: the kept plan is the searched one
 int64_t probe_kept(const pvnet_shape* s, int32_t cin, int32_t cout, int32_t* same) {
     const MarchKey key{*s, cin, cout};
     MarchPlan p{}, q{};
+    double us;
     const bool got = kept_plan<MarchPlan>(key, p, [](const MarchKey& k, MarchPlan& o) {
         searches++;
-        return march_search(k, o);
+        double v;
+        return march_search(k, o, v);
     });
-    *same = got == march_search(key, q) &&
+    *same = got == march_search(key, q, us) &&
             (!got || std::equal(reinterpret_cast<const int32_t*>(&p), reinterpret_cast<const int32_t*>(&p + 1), reinterpret_cast<const int32_t*>(&q)));
     return searches;
 }

@@ -1,4 +1,5 @@
-"""The planner of the marching kernels on the host: plans are searched once and kept."""
+"""The planner of the marching kernels on the host: plans are searched once and kept, and are priced with the blocks
+that a CU holds."""
 import random
 
 import pytest
@@ -44,3 +45,15 @@ def test_table_starts_over_when_full():
 @pytest.mark.parametrize("key", [((0x7fff, 1, 1, 1), 8, 8), ((1, 1, 1, 4096), 8, 8), ((1, 512, 1, 1), 128, 256)])
 def test_odd_shapes_plan_or_not(key):
     assert P.kept(*key)[1]
+
+
+@pytest.mark.parametrize("lds,vgprs,waves,blocks", [
+    (53760, 139, 4, 3),   # 42 pieces of 1,280 bytes, three times within 160 KB
+    (54176, 139, 4, 2),   # 43 pieces: 160 KB divided by the bytes alone would be three
+    (1280, 139, 4, 3),    # registers: 144 of 512 a lane
+    (1280, 256, 4, 2),
+    (160 * 1024, 40, 4, 1),
+    (42496, 92, 5, 3),
+])
+def test_blocks_per_cu(lds, vgprs, waves, blocks):
+    assert P.lib().probe_blocks_per_cu(lds, vgprs, waves) == blocks

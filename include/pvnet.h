@@ -39,9 +39,9 @@ enum { PVNET_RELU = 1, PVNET_F32OUT = 2, PVNET_GATHER = 4 };
  * 3x3x3 convolutions whose rows can be written four channels at a time (cout and ldy multiples of 4,
  * y aligned to 8 bytes, 16 with PVNET_F32OUT, relu_of likewise) march through z with their input
  * planes in LDS; PVNET_GATHER keeps them on the per-tap gathering kernel (the same result bit for
- * bit, for comparison), which also takes the shapes that fit no plan.  Pointwise convolutions with
- * cin <= 32 and cout <= 64 take their matrix-core operands straight from global memory (no LDS); PVNET_GATHER keeps them on the tiled kernel
- * (again the same result bit for bit). */
+ * bit, for comparison), which also takes the shapes that fit no plan or that it is the faster at.
+ * Pointwise convolutions with cin <= 32 and cout <= 64 take their matrix-core operands straight from
+ * global memory (no LDS); PVNET_GATHER keeps them on the tiled kernel (again the same result bit for bit). */
 typedef struct {
     pvnet_shape s;
     int32_t ntaps, cin, cout, kpad;
@@ -72,7 +72,7 @@ int pvnet_conv_split_fwd(const pvnet_conv* c, uint16_t* y0, int32_t ldy0, int32_
  * sums are reduced in a fixed order, so results are deterministic.  3x3x3 layers march through z with
  * the planes of x and dy in LDS, the bias sums in the same pass; flags = PVNET_GATHER keeps them on
  * the per-tap gathering kernel (the same sums in another order, for comparison), which also takes
- * the shapes that fit no plan.  flags = 0 otherwise.  Products with the zeros outside the box are part
+ * the shapes that fit no plan or that it is the faster at.  flags = 0 otherwise.  Products with the zeros outside the box are part
  * of the march's sums: an x that is not finite at a face makes all taps of its channel so, a dy there
  * only the taps whose input lies in the box. */
 typedef struct {

@@ -870,8 +870,6 @@ __global__ __launch_bounds__(256) void k_pack(const PackTable T) {
 // ---------------------------------------------------------------------------------------------
 // host helpers
 
-int64_t voxels(const pvnet_shape& s) { return (int64_t)s.nb * s.d * s.h * s.w; }
-
 bool shape_ok(const pvnet_shape* s) { return s && s->nb > 0 && s->d > 0 && s->h > 0 && s->w > 0; }
 
 bool al16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
@@ -879,41 +877,29 @@ bool al16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 int kpad_of(int ntaps, int c) { return (ntaps * c + BK - 1) / BK * BK; }
 
 struct WgradPlan {
-    int ktiles, ntiles, bn, nsplit, mchunk;
-    int64_t ws_main, ws_total;
-    bool march;  // k_wgrad_march
-    bool pw;     // k_wgrad_pw, chunks per block in mchunk
+    TiledWgrad tiled;    // unless one of
+    bool march;          // k_wgrad_march
+    bool pw;             // k_wgrad_pw
     WgradMarch mp;
+    int pw_chunks;       // per block
+    int nsplit;
+    int64_t ws_main, ws_total;
 };
-
-int wgrad_bn(int cout) { return cout <= 16 ? 16 : (cout <= 32 || cout % 64 != 0) ? 32 : 64; }
 
 WgradPlan plan_wgrad(const pvnet_shape& s, int ntaps, int cin, int cout, int flags) {
     WgradPlan p{};
     const int64_t M = voxels(s);
-    const int K = ntaps * cin;
-    p.bn = wgrad_bn(cout);
-    p.ktiles = (K + 63) / 64;
-    p.ntiles = (cout + p.bn - 1) / p.bn;
-    const int64_t want = 2048 / (p.ktiles * p.ntiles) + 1;
-    int64_t steps = (M + 127) / 128;  // LDS fills of 128 voxels
-    int64_t ns = std::min<int64_t>(std::max<int64_t>(want, 1), std::max<int64_t>(steps, 1));
-    int64_t per = (steps + ns - 1) / ns;
-    p.mchunk = (int)(per * 128);
-    p.nsplit = (int)((M + p.mchunk - 1) / p.mchunk);
-    p.ws_main = (int64_t)p.nsplit * cout * K;
+    p.tiled = tiled_wgrad(M, ntaps, cin, cout);
+    p.nsplit = p.tiled.nsplit;
     p.march = ntaps == 27 && !(flags & PVNET_GATHER) && wgrad_march_plan(s, cin, cout, p.mp);
-    if (p.march) {
-        p.nsplit = p.mp.splits;
-        p.ws_main = (int64_t)p.nsplit * cout * K;
-    }
+    if (p.march) p.nsplit = p.mp.splits;
     p.pw = ntaps == 1 && cin <= 32 && cout <= 16 && !(flags & PVNET_GATHER);
     if (p.pw) {
         const int64_t chunks = (M + WPW_VOX - 1) / WPW_VOX;
-        p.mchunk = 4 * (int)((chunks + 4 * WPW_BLOCKS - 1) / (4 * WPW_BLOCKS));  // whole rounds of the four waves
-        p.nsplit = (int)((chunks + p.mchunk - 1) / p.mchunk);
-        p.ws_main = (int64_t)p.nsplit * cout * K;
+        p.pw_chunks = 4 * (int)((chunks + 4 * WPW_BLOCKS - 1) / (4 * WPW_BLOCKS));  // whole rounds of the four waves
+        p.nsplit = (int)((chunks + p.pw_chunks - 1) / p.pw_chunks);
     }
+    p.ws_main = (int64_t)p.nsplit * cout * ntaps * cin;
     p.ws_total = p.ws_main + (int64_t)p.nsplit * cout;  // and the bias rows
     return p;
 }
@@ -928,20 +914,19 @@ int pool_args(const pvnet_shape* s, int c, const void* a, int lda, const void* b
     return 0;
 }
 
-// the gathering kernel: 256-voxel blocks for narrow outputs on large grids; 64-channel tiles only when the grid
-// still has >= 2048 blocks (the K loop is long, so the device needs many blocks in flight)
 template <bool PARTS>
 void conv_gather(const pvnet_conv& c, const NetParts& pq, int64_t M, hipStream_t st) {
-    const int K = c.ntaps * c.cin, mt = blocks_for(M, 128);
-    if (c.cout <= 16 && M >= (int64_t)256 * 2048) {
-        hipLaunchKernelGGL((k_conv_fwd<16, 64, PARTS>), dim3(blocks_for(M, 256), 1), dim3(256), 0, st, c, (int)M, K, pq);
-    } else if (c.cout <= 16) {
-        hipLaunchKernelGGL((k_conv_fwd<16, 32, PARTS>), dim3(mt, 1), dim3(256), 0, st, c, (int)M, K, pq);
-    } else if (c.cout % 64 == 0 && (int64_t)mt * (c.cout / 64) >= 2048) {
-        hipLaunchKernelGGL((k_conv_fwd<64, 32, PARTS>), dim3(mt, c.cout / 64), dim3(256), 0, st, c, (int)M, K, pq);
-    } else {
-        hipLaunchKernelGGL((k_conv_fwd<32, 32, PARTS>), dim3(mt, (c.cout + 31) / 32), dim3(256), 0, st, c, (int)M, K, pq);
-    }
+    const GatherTile t = gather_tile(M, c.cout);
+    const int K = c.ntaps * c.cin;
+    const dim3 grid(blocks_for(M, t.bm), (c.cout + t.bn - 1) / t.bn);
+    if (t.bm == 256)
+        hipLaunchKernelGGL((k_conv_fwd<16, 64, PARTS>), grid, dim3(256), 0, st, c, (int)M, K, pq);
+    else if (t.bn == 16)
+        hipLaunchKernelGGL((k_conv_fwd<16, 32, PARTS>), grid, dim3(256), 0, st, c, (int)M, K, pq);
+    else if (t.bn == 64)
+        hipLaunchKernelGGL((k_conv_fwd<64, 32, PARTS>), grid, dim3(256), 0, st, c, (int)M, K, pq);
+    else
+        hipLaunchKernelGGL((k_conv_fwd<32, 32, PARTS>), grid, dim3(256), 0, st, c, (int)M, K, pq);
 }
 
 int conv_launch(const pvnet_conv* c, const NetParts& pq, void* stream, const char* who) {
@@ -980,7 +965,7 @@ int conv_launch(const pvnet_conv* c, const NetParts& pq, void* stream, const cha
 }
 
 template <bool PARTS>
-void wgrad_gather(const pvnet_wgrad& a, const NetParts& pq, const WgradPlan& p, int64_t M, int64_t dboff, hipStream_t st) {
+void wgrad_tiled(const pvnet_wgrad& a, const NetParts& pq, const TiledWgrad& p, int64_t M, int64_t dboff, hipStream_t st) {
     const int K = a.ntaps * a.cin;
     const dim3 grid(p.ktiles, p.ntiles, p.nsplit);
     if (p.bn == 16)
@@ -1011,11 +996,11 @@ int wgrad_launch(const pvnet_wgrad* a, const NetParts& pq, void* stream, const c
         hipLaunchKernelGGL(wgrad_march_kernel(p.mp), dim3(p.mp.splits * p.mp.ns * p.mp.nf), dim3(256), p.mp.lds, st, *a, p.mp, pq,
                            dboff);
     } else if (p.pw) {
-        hipLaunchKernelGGL(wgrad_pw_kernel(a->cin, a->cout), dim3(p.nsplit), dim3(256), 0, st, *a, (int)M, p.mchunk, dboff);
+        hipLaunchKernelGGL(wgrad_pw_kernel(a->cin, a->cout), dim3(p.nsplit), dim3(256), 0, st, *a, (int)M, p.pw_chunks, dboff);
     } else if (pq.cup) {
-        wgrad_gather<true>(*a, pq, p, M, dboff, st);
+        wgrad_tiled<true>(*a, pq, p.tiled, M, dboff, st);
     } else {
-        wgrad_gather<false>(*a, pq, p, M, dboff, st);
+        wgrad_tiled<false>(*a, pq, p.tiled, M, dboff, st);
     }
     NET_LAUNCH();
     const int64_t len = (int64_t)a->cout * K;

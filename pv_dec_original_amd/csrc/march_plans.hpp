@@ -54,6 +54,7 @@ struct MarchPrice {
     double plane, unit;                   // a plane and its units
     double hide;                          // of the shorter of the two
 };
+constexpr double CLOCKS_US = 2400;
 constexpr MarchPrice RING_PRICE{2.78, 0.0, 5.31, 26.2, 0.372, 0.188, 0.477, 1.05, {0, 77.7, 79.8}, 784, {20.7, 0, 0}, 0.383, 642, 1.99, 2.2};
 constexpr MarchPrice ROLL_PRICE{2.06, 0.715, 2.59, 36.1, 0.173, 0.656, 0.9, 0.0, {0, 133, 0}, 968, {0, 0, 0}, 0.644, 1490, 2.93, 0.68};
 
@@ -69,11 +70,11 @@ inline int blocks_per_cu(int lds, int vgprs, int waves) {
     return std::max(1, std::min(LDS / ((lds + PIECE - 1) / PIECE * PIECE), 4 * (512 / ((vgprs + 7) / 8 * 8)) / waves));
 }
 
-// us of `blocks` blocks of which a CU holds cc, on 256 CUs
-inline double rounds_us(double blocks, int cc, double cu, double alone, double hide) {
+// time of `blocks` blocks of which a CU holds cc, on 256 CUs, in the unit of cu and alone
+inline double rounds_of(double blocks, int cc, double cu, double alone, double hide) {
     const double rounds = std::ceil(blocks / (256.0 * cc)), rest = std::ceil((blocks - (rounds - 1) * 256 * cc) / 256);
     auto one = [&](double c) { return std::max(alone, cu * c) + hide * std::min(alone, cu * c); };
-    return ((rounds - 1) * one(cc) + one(rest)) / 2400;
+    return (rounds - 1) * one(cc) + one(rest);
 }
 
 // The plan of a convolution: every tile, run length, wave split and place of the weights that fits is priced and the
@@ -133,7 +134,7 @@ inline bool march_search(const MarchKey& c, MarchPlan& best, double& us) {
                                 const double cu = (top + P.share * (m + l + l1 + io - top)) * (1 + P.few / (cc * W)) + 0.5 * wfill;
                                 const double step = P.step[wm] + P.mstep * 16 * mf / nst * std::max(1.0, W / 4.0);
                                 const double alone = P.start + wfill + nst * step + pl * (P.plane + P.unit * nu / (roll ? 1 : 4));
-                                const double cost = P.launch + rounds_us(B, cc, cu, alone, P.hide);
+                                const double cost = P.launch + rounds_of(B, cc, cu, alone, P.hide) / CLOCKS_US;
                                 if (us == 0 || cost < us) {
                                     us = cost;
                                     best = MarchPlan{tx, ty, (w + tx - 1) / tx, (h + ty - 1) / ty, zs[iz], nzs, tx + 2, hp, su, steps,
@@ -146,6 +147,36 @@ inline bool march_search(const MarchKey& c, MarchPlan& best, double& us) {
             }
     }
     return us > 0;
+}
+
+// The gathering convolution's blocks: 256 voxels for narrow outputs on large grids; 64 channels only when the grid still
+// has 2,048 blocks (the K loop is long, so the device needs many blocks in flight).
+struct GatherTile {
+    int32_t bm, bn;
+    int64_t blocks;
+};
+
+inline GatherTile gather_tile(int64_t M, int cout) {
+    const int64_t mt = (M + 127) / 128;
+    if (cout <= 16) return M >= (int64_t)256 * 2048 ? GatherTile{256, 16, (M + 255) / 256} : GatherTile{128, 16, mt};
+    if (cout % 64 == 0 && mt * (cout / 64) >= 2048) return {128, 64, mt * (cout / 64)};
+    return {128, 32, mt * ((cout + 31) / 32)};
+}
+
+// us of a 3x3x3 convolution by gathering, fitted to 5,000 timed layers: rms error 10 % (25 % for 256-voxel blocks, which
+// marching beats by a factor)
+inline double gather_us(int64_t M, int cin, int cout) {
+    struct Price {
+        double launch, step, cu, block, hide;  // us: a step of a block alone, of 256 blocks, the blocks' own cost
+    };
+    const GatherTile t = gather_tile(M, cout);
+    const Price P = t.bm == 256  ? Price{8.84, 0.487, 0.0965, 3.49, 1.71}
+                    : t.bn == 16 ? Price{9.46, 0.396, 0.140, 1.46, 0.289}
+                    : t.bn == 64 ? Price{11.2, 0.657, 0.129, 2.49, 0.866}
+                                 : Price{11.5, 0.408, 0.148, 1.07, 0.467};
+    const double steps = (27 * cin + BK - 1) / BK, rounds = t.blocks / 256.0;
+    const double alone = steps * P.step * std::ceil(rounds / 8), cu = steps * P.cu * rounds;
+    return P.launch + std::max(alone, cu) + P.hide * std::min(alone, cu) + P.block * rounds;
 }
 
 // the plan of a weight gradient
@@ -190,7 +221,7 @@ inline bool wgrad_march_search(const pvnet_shape& s, int cin, int cout, WgradMar
                     const double B = (double)splits * nf * st, za = (double)s.d / nzs;
                     const double alone = per * (881 + 7.67 * hp + 1260 * (za + 2) + za * gr * (238 + 218.0 * cf));
                     const double cu = per * za * (gr * std::max(118.0 * cf, 26.2 * (7 + cf)) + 0.66 * (hp + cf * gr * 32));
-                    const double cost = 7.18 + rounds_us(B, cc, cu, alone, 0.41) + splits * (6.72e-5 * cin * cout + 6.7e-4);
+                    const double cost = 7.18 + rounds_of(B, cc, cu, alone, 0.41) / CLOCKS_US + splits * (6.72e-5 * cin * cout + 6.7e-4);
                     if (us == 0 || cost < us) {
                         us = cost;
                         best = WgradMarch{tx, ty, s.w / tx, s.h / ty, zseg, nzs, tx + 2, hp, gr, su, fu, cf, st, nf, (int)units, per, splits, lds};
@@ -200,6 +231,35 @@ inline bool wgrad_march_search(const pvnet_shape& s, int cin, int cout, WgradMar
         }
     }
     return us > 0;
+}
+
+// The tiled weight-gradient kernel: bn output channels by 64 k-values a block, the voxels in nsplit runs of mchunk (LDS
+// fills of 128 voxels).
+struct TiledWgrad {
+    int32_t bn, ktiles, ntiles, nsplit, mchunk;
+};
+
+inline TiledWgrad tiled_wgrad(int64_t M, int ntaps, int cin, int cout) {
+    const int bn = cout <= 16 ? 16 : (cout <= 32 || cout % 64 != 0) ? 32 : 64;
+    const int ktiles = (ntaps * cin + 63) / 64, ntiles = (cout + bn - 1) / bn;
+    const int64_t want = 2048 / (ktiles * ntiles) + 1, fills = (M + 127) / 128;
+    const int64_t ns = std::min<int64_t>(std::max<int64_t>(want, 1), std::max<int64_t>(fills, 1)), per = (fills + ns - 1) / ns;
+    return {bn, ktiles, ntiles, (int32_t)((M + per * 128 - 1) / (per * 128)), (int32_t)(per * 128)};
+}
+
+// us of a 3x3x3 weight gradient by the tiled kernel and its sum over the splits, fitted to 4,900 timed layers: rms error
+// 7 % (16 channels), 13 %, 11 %
+inline double tiled_wgrad_us(int64_t M, int cin, int cout) {
+    struct Price {
+        double launch, start, fill, cu, hide, sum, split;  // us
+    };
+    const TiledWgrad t = tiled_wgrad(M, 27, cin, cout);
+    const Price P = t.bn == 16   ? Price{5.23, 0.797, 0.251, 0.435, 1.08, 2.13e-6, 3.1e-3}
+                    : t.bn == 32 ? Price{6.07, 0.013, 0.453, 0.425, 1.07, 2.94e-6, 0}
+                                 : Price{9.60, 0.030, 0.775, 0.805, 0.338, 2.07e-6, 0};
+    const double fills = t.mchunk / 128;
+    return P.launch + rounds_of((double)t.ktiles * t.ntiles * t.nsplit, 4, fills * P.cu, P.start + fills * P.fill, P.hide) +
+           t.nsplit * (P.sum * 27 * cin * cout + P.split);
 }
 
 // The plan of a shape, a pure function of its key, searched once per thread and kept with the others the thread has
@@ -234,18 +294,28 @@ bool kept_plan(const MarchKey& key, Plan& p, Search search) {
     return slots[i].ok == 1;
 }
 
-inline bool march_plan(const pvnet_shape& s, int cin, int cout, MarchPlan& p) {
-    return kept_plan<MarchPlan>(MarchKey{s, cin, cout}, p, [](const MarchKey& k, MarchPlan& q) {
-        double us;
-        return march_search(k, q, us);
-    });
+inline int64_t voxels(const pvnet_shape& s) { return (int64_t)s.nb * s.d * s.h * s.w; }
+
+// The route of a layer: marching where a plan fits and costs no more than the kernel it takes the place of.  That one is
+// the cheaper on small or thin planes, where a tile is mostly halo, for deep inputs on few voxels, and for weight
+// gradients of few voxels.  Measured, us, marching and the other: convolutions 8 x 52 x 6 x 12 120 -> 56 161 and 62, 64
+// x 30 x 3 x 2 112 -> 216 524 and 70, 8 x 48^3 96 -> 32 221 and 442; weight gradients 256 x 2^3 96 -> 32 34 and 12, 8 x 6
+// x 2 x 2 160 -> 160 41 and 26, 1 x 88 x 8 x 8 8 -> 16 10.7 and 7.5, 8 x 24^3 64 -> 64 50 and 109.
+inline bool march_route(const MarchKey& k, MarchPlan& p) {
+    double us;
+    return march_search(k, p, us) && us <= gather_us(voxels(k.s), k.cin, k.cout);
 }
 
+inline bool wgrad_route(const MarchKey& k, WgradMarch& p) {
+    const int64_t M = voxels(k.s);
+    double us;
+    return M < (int64_t)1 << 31 && wgrad_march_search(k.s, k.cin, k.cout, p, us) && us <= tiled_wgrad_us(M, k.cin, k.cout);
+}
+
+inline bool march_plan(const pvnet_shape& s, int cin, int cout, MarchPlan& p) { return kept_plan(MarchKey{s, cin, cout}, p, march_route); }
+
 inline bool wgrad_march_plan(const pvnet_shape& s, int cin, int cout, WgradMarch& p) {
-    return kept_plan<WgradMarch>(MarchKey{s, cin, cout}, p, [](const MarchKey& k, WgradMarch& q) {
-        double us;
-        return (int64_t)k.s.nb * k.s.d * k.s.h * k.s.w < (int64_t)1 << 31 && wgrad_march_search(k.s, k.cin, k.cout, q, us);
-    });
+    return kept_plan(MarchKey{s, cin, cout}, p, wgrad_route);
 }
 
 }  // namespace

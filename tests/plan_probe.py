@@ -28,11 +28,11 @@ def lib():
 def _plan(fn, fields, shape, cin, cout):
     out, us = (C.c_int32 * len(fields))(), C.c_double()
     got = fn(C.byref(N.NetShape(*shape)), cin, cout, out, len(fields), C.byref(us))
-    return dict(zip(fields, out), us=us.value) if got else None
+    return dict(zip(fields, out), us=us.value, marches=got == 2) if got else None
 
 
 def conv_plan(shape, cin, cout):
-    """The plan of a 3x3x3 convolution as a dict, with its price in us, or None."""
+    """The plan of a 3x3x3 convolution as a dict, with its price in us and whether the layer takes it, or None."""
     return _plan(lib().probe_conv_plan, CONV, shape, cin, cout)
 
 

@@ -7,20 +7,20 @@ int64_t searches = 0;
 
 extern "C" {
 
-// fields of MarchPlan and the price; 0: no plan
+// fields of MarchPlan and the price; 0: no plan, 1: the gathering kernel is cheaper, 2: marches
 int probe_conv_plan(const pvnet_shape* s, int32_t cin, int32_t cout, int32_t* out, int32_t n, double* us) {
     MarchPlan p{};
     if (n != (int32_t)(sizeof(p) / 4) || !march_search(MarchKey{*s, cin, cout}, p, *us)) return 0;
     std::copy_n(reinterpret_cast<const int32_t*>(&p), n, out);
-    return 1;
+    return march_route(MarchKey{*s, cin, cout}, p) ? 2 : 1;
 }
 
-// fields of WgradMarch and the price; 0: no plan
+// fields of WgradMarch and the price; 0: no plan, 1: the tiled kernel is cheaper, 2: marches
 int probe_wgrad_plan(const pvnet_shape* s, int32_t cin, int32_t cout, int32_t* out, int32_t n, double* us) {
     WgradMarch p{};
     if (n != (int32_t)(sizeof(p) / 4) || !wgrad_march_search(*s, cin, cout, p, *us)) return 0;
     std::copy_n(reinterpret_cast<const int32_t*>(&p), n, out);
-    return 1;
+    return wgrad_route(MarchKey{*s, cin, cout}, p) ? 2 : 1;
 }
 
 int probe_blocks_per_cu(int32_t lds, int32_t vgprs, int32_t waves) { return blocks_per_cu(lds, vgprs, waves); }
@@ -29,13 +29,11 @@ int probe_blocks_per_cu(int32_t lds, int32_t vgprs, int32_t waves) { return bloc
 int64_t probe_kept(const pvnet_shape* s, int32_t cin, int32_t cout, int32_t* same) {
     const MarchKey key{*s, cin, cout};
     MarchPlan p{}, q{};
-    double us;
     const bool got = kept_plan<MarchPlan>(key, p, [](const MarchKey& k, MarchPlan& o) {
         searches++;
-        double v;
-        return march_search(k, o, v);
+        return march_route(k, o);
     });
-    *same = got == march_search(key, q, us) &&
+    *same = got == march_route(key, q) &&
             (!got || std::equal(reinterpret_cast<const int32_t*>(&p), reinterpret_cast<const int32_t*>(&p + 1), reinterpret_cast<const int32_t*>(&q)));
     return searches;
 }

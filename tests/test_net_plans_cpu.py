@@ -57,3 +57,26 @@ def test_odd_shapes_plan_or_not(key):
 ])
 def test_blocks_per_cu(lds, vgprs, waves, blocks):
     assert P.lib().probe_blocks_per_cu(lds, vgprs, waves) == blocks
+
+
+@pytest.mark.parametrize("shape,cin,cout,conv,wgrad", [
+    # where marching costs more than the kernel it takes the place of (both measured, us: marching, the other)
+    ((8, 52, 6, 12), 120, 56, False, None),    # convolution 161, 62
+    ((64, 30, 3, 2), 112, 216, False, None),   # 524, 70
+    ((2, 54, 34, 8), 104, 136, False, None),   # 150, 100
+    ((256, 2, 2, 2), 96, 32, None, False),     # weight gradient 34, 12
+    ((8, 6, 2, 2), 160, 160, None, False),     # 41, 26
+    ((8, 6, 89, 14), 8, 136, None, False),     # 77, 36
+    ((2, 8, 8, 16), 8, 16, True, False),       # convolution 4, 12; weight gradient 9.6, 7.1
+    # and where it is the cheaper
+    ((8, 96, 96, 96), 16, 16, True, True),
+    ((8, 48, 48, 48), 96, 32, True, True),
+    ((8, 12, 12, 12), 160, 160, True, True),
+    ((1, 24, 24, 48), 64, 64, True, True),
+    ((3, 20, 18, 28), 64, 160, True, True),
+])
+def test_route_by_price(shape, cin, cout, conv, wgrad):
+    if conv is not None:
+        assert P.conv_plan(shape, cin, cout)["marches"] == conv
+    if wgrad is not None:
+        assert P.wgrad_plan(shape, cin, cout)["marches"] == wgrad

@@ -72,9 +72,10 @@ int pvnet_conv_split_fwd(const pvnet_conv* c, uint16_t* y0, int32_t ldy0, int32_
  * sums are reduced in a fixed order, so results are deterministic.  3x3x3 layers march through z with
  * the planes of x and dy in LDS, the bias sums in the same pass; flags = PVNET_GATHER keeps them on
  * the per-tap gathering kernel (the same sums in another order, for comparison), which also takes
- * the shapes that fit no plan or that it is the faster at.  flags = 0 otherwise.  Products with the zeros outside the box are part
- * of the march's sums: an x that is not finite at a face makes all taps of its channel so, a dy there
- * only the taps whose input lies in the box. */
+ * the shapes that fit no plan or that it is the faster at.  flags = 0 otherwise.  The march's
+ * sums are those over the pairs inside the box, also where a value is not finite (summed again then,
+ * which takes a pass over x and dy for each 16 columns); the other kernel's hold a dy that is not
+ * finite also against the zeros outside. */
 typedef struct {
     pvnet_shape s;
     int32_t ntaps, cin, cout;

@@ -10,7 +10,8 @@
 // so a block takes 16 output channels of dy (planes z-1 .. z+1 with a halo) against 16 CF input channels of x
 // (its own voxels only), and a wave reads CF + 7 fragments for 7 CF MFMAs.  Wave v owns the shifts v, v + 4, ..
 // (7 of them; the 28th is a repeat that is not written), so every sum is complete within its wave.  Blocks are
-// splits of the voxels, summed by k_sum_splits.  The bias gradient is one more MFMA per dy fragment of the
+// splits of the voxels, summed by k_sum_splits, which also sees to an x that is not finite (here it meets the zeros
+// around dy's box).  The bias gradient is one more MFMA per dy fragment of the
 // centre tap, with ones for x.
 //
 // What bounds it: at CF = 1 the LDS (8 KB of fragments for 7 MFMAs), at CF = 3 the matrix cores and the LDS

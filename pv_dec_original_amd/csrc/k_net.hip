@@ -1222,8 +1222,12 @@ int pvnet_wall_distance(const pvnet_shape* s, const uint8_t* code, float* dist, 
     const int64_t plane = (int64_t)s->h * s->w, nlines = voxels(*s) / s->w, nslab[2] = {(int64_t)s->nb * s->d, s->nb};
     const int64_t ncol[2] = {s->w, plane};
     const int len[2] = {s->h, s->d};
-    hipLaunchKernelGGL(k_edt_row, dim3(blocks_for(nlines, 4)), dim3(256), 0, (hipStream_t)stream, nlines, s->w, code, dist);
-    NET_LAUNCH();
+    constexpr int64_t LINES = (int64_t)1 << 25;  // of one launch: 64 threads each, and a launch has fewer than 2^32
+    for (int64_t l0 = 0; l0 < nlines; l0 += LINES) {
+        const int64_t n = std::min(LINES, nlines - l0);
+        hipLaunchKernelGGL(k_edt_row, dim3(blocks_for(n, 4)), dim3(256), 0, (hipStream_t)stream, n, s->w, code + l0 * s->w, dist + l0 * s->w);
+        NET_LAUNCH();
+    }
     for (int axis = 0; axis < 2; axis++)
         // slabs beyond the grid's y limit go in several launches
         for (int64_t s0 = 0; s0 < nslab[axis]; s0 += 65535) {

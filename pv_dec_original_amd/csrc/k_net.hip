@@ -109,7 +109,7 @@ __global__ __launch_bounds__(256) void k_conv_fwd(pvnet_conv a, int M, int K, Ne
     __shared__ __attribute__((aligned(16))) uint16_t Bs[BN * LP];
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     const int g = lane >> 4, c16 = lane & 15;
-    const int m0 = xcd_tile(blockIdx.x, gridDim.x) * BM, n0 = blockIdx.y * BN;
+    const int m0 = xcd_tile(blockIdx.x + blockIdx.z * gridDim.x, gridDim.x * gridDim.z) * BM, n0 = blockIdx.y * BN;
     const int d = a.s.d, h = a.s.h, w = a.s.w;
 
     // load roles: A rows r + 64 i, 8-wide k chunk q; B row bn (if < BN), same chunk.  Per row, a
@@ -965,7 +965,9 @@ template <bool PARTS>
 void conv_gather(const pvnet_conv& c, const NetParts& pq, int64_t M, hipStream_t st) {
     const GatherTile t = gather_tile(M, c.cout);
     const int K = c.ntaps * c.cin;
-    const dim3 grid(blocks_for(M, t.bm), (c.cout + t.bn - 1) / t.bn);
+    // 2^24 blocks, which a full count of voxels needs, are 2^32 threads, and a launch has fewer along x
+    const int mt = blocks_for(M, t.bm), nz = mt == 1 << 24 ? 2 : 1;
+    const dim3 grid(mt / nz, (c.cout + t.bn - 1) / t.bn, nz);
     if (t.bm == 256)
         hipLaunchKernelGGL((k_conv_fwd<16, 64, PARTS>), grid, dim3(256), 0, st, c, (int)M, K, pq);
     else if (t.bn == 16)

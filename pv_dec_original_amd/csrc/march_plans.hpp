@@ -126,6 +126,7 @@ inline bool march_search(const MarchKey& c, MarchPlan& best, double& us) {
                                 const int nzs = (d + zs[iz] - 1) / zs[iz];
                                 const double za = (double)d / nzs, pl = za + 2;
                                 const double B = tiles * nzs * ((ct + wn - 1) / wn);
+                                if (B * 64 * (W + roll) >= 4294967296.0) continue;  // a launch has fewer than 2^32 threads
                                 const double nst = roll ? sp * pl : steps * za, mf = steps * za * rt;
                                 const double xr = nst * rt, wr = wm == 2 ? 0 : roll ? sp * (3 * za + 2) : steps * za;
                                 const double m = P.mma * mf * W, l = P.lds * (xr + (wm == 1 ? wr : 0)) * W,

@@ -80,3 +80,12 @@ def test_route_by_price(shape, cin, cout, conv, wgrad):
         assert P.conv_plan(shape, cin, cout)["marches"] == conv
     if wgrad is not None:
         assert P.wgrad_plan(shape, cin, cout)["marches"] == wgrad
+
+
+@pytest.mark.parametrize("shape,cin,cout", [((1 << 24, 4, 4, 4), 8, 16), ((1 << 24, 1, 8, 8), 8, 8), ((1 << 27, 2, 2, 2), 8, 16),
+                                            ((3 << 22, 4, 4, 8), 8, 8), ((64, 31, 601, 1801), 8, 8), ((1 << 25, 2, 2, 8), 32, 16)])
+def test_a_plan_fits_a_launch(shape, cin, cout):
+    p = P.conv_plan(shape, cin, cout)
+    if p:
+        blocks = p["ntx"] * p["nty"] * p["nzs"] * p["ng"] * shape[0]
+        assert blocks * 64 * (p["wx"] * p["wn"] + p["roll"]) < 2 ** 32

@@ -99,6 +99,7 @@ double nudge(double v, double lo, double hi) {
 // =============================================================================================
 
 constexpr int32_t GATHER_TILES = 512;  // tiles of one group of a read-out: at most 1 MB of node values
+constexpr int32_t PLAIN_TILES = 640, FIRST_PLAIN_TILES = 2048;  // lattices read out through ordinary memory: always, first
 
 struct pvlbm_sim {
     std::string err;
@@ -133,9 +134,10 @@ struct pvlbm_sim {
     double* d_macro = nullptr;
     double* d_partials = nullptr;
     double* d_red = nullptr;
-    // node values on their way to the host, in two halves of GATHER_TILES tiles each: device, pinned host and the
-    // events of the copies, allocated by the first read-out; position of each group's first node, and their number
-    double *d_gather = nullptr, *h_gather = nullptr;
+    // node values on their way to the host: ordinary memory, or two pinned halves of GATHER_TILES tiles each and the
+    // events of their copies, allocated when first used; position of each group's first node, and their number
+    std::vector<double> v_gather;
+    double* h_gather = nullptr;
     hipEvent_t ev_gather[2] = {nullptr, nullptr};
     std::vector<int64_t> gather_first;
     double* d_expand = nullptr;  // scratch of a start from a coarse field, allocated by the first one
@@ -196,7 +198,7 @@ struct pvlbm_sim {
     ~pvlbm_sim() {
         if (stream) (void)hipStreamSynchronize(stream);
         void* ptrs[] = {d_bq, d_kind, d_aux, d_tdesc, d_pop[0], d_pop[1], d_bmask, d_bclose, d_bprof, d_brho,
-                        d_M, d_nrm, d_wss, d_tau3, d_acc, d_macro, d_partials, d_red, d_expand, d_gather, d_gate};
+                        d_M, d_nrm, d_wss, d_tau3, d_acc, d_macro, d_partials, d_red, d_expand, d_gate};
         for (void* p : ptrs) dfree(p);
         if (h_gather) (void)hipHostFree(h_gather);
         for (hipEvent_t e : ev_gather)
@@ -264,41 +266,52 @@ struct pvlbm_sim {
         return d_expand;
     }
 
-    void ensure_gather() {
-        if (!d_gather) d_gather = dalloc<double>((size_t)2 * GATHER_TILES * 64 * 4);
-        if (!h_gather) HIPCHK(hipHostMalloc((void**)&h_gather, sizeof(double) * 2 * GATHER_TILES * 64 * 4, hipHostMallocDefault));
-        for (hipEvent_t& e : ev_gather)
-            if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    }
+    // Doubles of the read-outs' device part, which lies behind the macro planes
+    int64_t gather_doubles() const { return (int64_t)std::min(2 * GATHER_TILES, ntiles) * 64 * 4; }
 
     // Density and velocity of the nodes into dense box arrays; other points are left alone.  Groups of tiles are
     // gathered on the device and copied while the group before is put in place, so the host reads and writes the
     // nodes and not the box (a vessel of 96^3 points, 250 steps and this: 3.9 ms, 14.3 with the padded planes
     // copied whole into a fresh buffer).  One megabyte a group: long enough a copy for the link, and still in the host's cache when read.
+    // The copies that overlap need pinned memory and events, which take 0.1 to 0.8 ms to make.  Small lattices, and the
+    // first read-out of middling ones, copy into ordinary memory instead, two groups at once.  Us of a handle's first
+    // read-out, in parentheses of the first handle's: tubes of 3,198, 25,353 and 69,495 nodes 64 (116), 131 (135), 342
+    // (454); through pinned memory 131 (161), 218 (840), 334 (1260); the padded planes whole 63 (84), 196 (340), 413
+    // (434).  Later ones 35, 90 and 240 (42, 116, 245 through pinned memory).
     void fill_macros(double* rho, double* u) {
-        const int32_t groups = (ntiles + GATHER_TILES - 1) / GATHER_TILES;
-        if (groups == 0) return;
-        ensure_gather();
-        const int64_t nbox = nx * ny * nz, half = (int64_t)GATHER_TILES * 64 * 4;
+        if (ntiles == 0) return;
+        const bool plain = ntiles <= PLAIN_TILES || (!h_gather && v_gather.empty() && ntiles <= FIRST_PLAIN_TILES);
+        const int32_t step = plain ? 2 : 1, per = step * GATHER_TILES, groups = (ntiles + per - 1) / per;
+        const int64_t nbox = nx * ny * nz, half = plain ? 0 : (int64_t)GATHER_TILES * 64 * 4;
+        if (plain) v_gather.resize((size_t)gather_doubles());
+        else {
+            v_gather = {};
+            if (!h_gather) HIPCHK(hipHostMalloc((void**)&h_gather, sizeof(double) * 2 * half, hipHostMallocDefault));
+            for (hipEvent_t& e : ev_gather)
+                if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        }
+        double *from = d_macro + 4 * ns, *to = plain ? v_gather.data() : h_gather;
+        auto first = [&](int32_t gi) { return gather_first[std::min<size_t>((size_t)gi * step, gather_first.size() - 1)]; };
         auto start = [&](int32_t gi) {
-            const int32_t t0 = gi * GATHER_TILES, cnt = (int32_t)(gather_first[gi + 1] - gather_first[gi]);
-            double* d = d_gather + (gi & 1) * half;
-            HIPCHK(launch_macros_nodes(d_macro, ns, d_tdesc, t0, std::min(GATHER_TILES, ntiles - t0), d, stream));
-            HIPCHK(hipMemcpyAsync(h_gather + (gi & 1) * half, d, sizeof(double) * 4 * cnt, hipMemcpyDeviceToHost, stream));
-            HIPCHK(hipEventRecord(ev_gather[gi & 1], stream));
+            const int32_t t0 = gi * per, cnt = (int32_t)(first(gi + 1) - first(gi));
+            double* d = from + (gi & 1) * half;
+            HIPCHK(launch_macros_nodes(d_macro, ns, d_tdesc, t0, std::min(per, ntiles - t0), d, stream));
+            HIPCHK(hipMemcpyAsync(to + (gi & 1) * half, d, sizeof(double) * 4 * cnt, hipMemcpyDeviceToHost, stream));
+            if (!plain) HIPCHK(hipEventRecord(ev_gather[gi & 1], stream));
         };
         start(0);
         for (int32_t gi = 0; gi < groups; gi++) {
-            HIPCHK(hipEventSynchronize(ev_gather[gi & 1]));
-            if (gi + 1 < groups) start(gi + 1);
-            const double* v = h_gather + (gi & 1) * half;
-            const int64_t* box = lists[PVLBM_LIST_FLUID].data() + gather_first[gi];
-            const int32_t cnt = (int32_t)(gather_first[gi + 1] - gather_first[gi]);
+            HIPCHK(plain ? hipStreamSynchronize(stream) : hipEventSynchronize(ev_gather[gi & 1]));
+            if (!plain && gi + 1 < groups) start(gi + 1);
+            const double* v = to + (gi & 1) * half;
+            const int64_t* box = lists[PVLBM_LIST_FLUID].data() + first(gi);
+            const int32_t cnt = (int32_t)(first(gi + 1) - first(gi));
             for (int32_t i = 0; i < cnt; i++) {
                 const int64_t b = box[i];
                 if (rho) rho[b] = v[4 * i];
                 if (u) u[b] = v[4 * i + 1], u[nbox + b] = v[4 * i + 2], u[2 * nbox + b] = v[4 * i + 3];
             }
+            if (plain && gi + 1 < groups) start(gi + 1);
         }
     }
 
@@ -876,7 +889,7 @@ extern "C" int pvlbm_create(const uint8_t* fluid, const pvlbm_grid* grid, double
         S->d_wss = dalloc<double>((size_t)nw1);
         S->d_tau3 = dalloc<double>((size_t)(3 * nw1));
         S->d_acc = dalloc<double>((size_t)(4 * nw1));
-        S->d_macro = dalloc<double>((size_t)(4 * S->ns));
+        S->d_macro = dalloc<double>((size_t)(4 * S->ns + S->gather_doubles()));
         S->d_partials = dalloc<double>((size_t)(4 * std::max(S->blocks(), 1)));
         S->d_red = dalloc<double>(4);
         S->d_gate = dalloc<unsigned long long>(1);

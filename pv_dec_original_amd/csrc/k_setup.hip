@@ -590,14 +590,14 @@ hipError_t launch_expand_coarse(const float* rho_c, const float* u_c, int cx, in
 // Compact FP32 fields, PT consecutive points of a row per thread (VEC: four, with 16-byte stores).  Bound by the
 // output's 16 bytes a point: most points are not nodes and read one kind byte.  1024 x 512 x 512: 1.03 ms
 // (4.4 TB/s), 1.30 ms with one point and 64-bit divisions per thread.
-template <bool VEC, int PT, class I>
+template <bool VEC, int PT>
 __global__ __launch_bounds__(256) void k_macros_f32(const double* macro, const uint8_t* kind, int64_t nx, uint32_t ny, int64_t nbox,
-                                                    I nq, I quads, int64_t nxp, int64_t nyp, int64_t ns, float* rho, float* u) {
-    const I q = (I)blockIdx.x * 256 + threadIdx.x;
+                                                    uint32_t nq, uint32_t quads, int64_t nxp, int64_t nyp, int64_t ns, float* rho, float* u) {
+    const uint32_t q = blockIdx.x * 256 + threadIdx.x;
     if (q >= quads) return;
-    const I row = q / nq;
+    const uint32_t row = q / nq;
     const int64_t i = PT * (int64_t)(q - row * nq), r = (int64_t)row;
-    const int64_t n = ((int64_t)((uint32_t)row % ny) + nyp * (int64_t)((uint32_t)row / ny)) * nxp + i, b = r * nx + i;
+    const int64_t n = ((int64_t)(row % ny) + nyp * (int64_t)(row / ny)) * nxp + i, b = r * nx + i;
     // rows are padded: four kinds are always within the row
     const uint32_t k4 = PT == 4 ? *reinterpret_cast<const uint32_t*>(kind + n) : kind[n];
     float v[4][PT];
@@ -631,15 +631,14 @@ hipError_t launch_macros_f32(const double* macro, const uint8_t* kind, int64_t n
     // 32-bit indices four, to stay within a launch
     const bool one = !vec && nbox <= 0xffffff00ll;
     const int64_t nq = one ? nx : (nx + 3) / 4, quads = nq * ny * nz;
+    // a thread each, and a launch has fewer than 2^32: boxes of more than 17e9 points, 550 GB of macro planes
+    if (quads > 0xffffff00ll) return hipErrorInvalidValue;
     const dim3 g((unsigned)((quads + 255) / 256));
-    const bool wide = quads > 0xffffff00ll;  // 32-bit quad indices otherwise: their divisions are far cheaper
-#define PV_MACROS(V, PT, I) \
-    hipLaunchKernelGGL((k_macros_f32<V, PT, I>), g, dim3(256), 0, s, macro, kind, nx, (uint32_t)ny, nbox, (I)nq, (I)quads, nxp, nyp, ns, rho, u)
-    if (vec && wide) PV_MACROS(true, 4, int64_t);
-    else if (vec) PV_MACROS(true, 4, uint32_t);
-    else if (one) PV_MACROS(false, 1, uint32_t);
-    else if (wide) PV_MACROS(false, 4, int64_t);
-    else PV_MACROS(false, 4, uint32_t);
+#define PV_MACROS(V, PT) \
+    hipLaunchKernelGGL((k_macros_f32<V, PT>), g, dim3(256), 0, s, macro, kind, nx, (uint32_t)ny, nbox, (uint32_t)nq, (uint32_t)quads, nxp, nyp, ns, rho, u)
+    if (vec) PV_MACROS(true, 4);
+    else if (one) PV_MACROS(false, 1);
+    else PV_MACROS(false, 4);
 #undef PV_MACROS
     return hipGetLastError();
 }

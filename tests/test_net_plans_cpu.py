@@ -5,6 +5,7 @@ import random
 import pytest
 
 from pv_dec_original_amd.warmnet import UNetSpec
+from tests import net_march_cases as K
 from tests import plan_probe as P
 
 
@@ -89,3 +90,37 @@ def test_a_plan_fits_a_launch(shape, cin, cout):
     if p:
         blocks = p["ntx"] * p["nty"] * p["nzs"] * p["ng"] * shape[0]
         assert blocks * 64 * (p["wx"] * p["wn"] + p["roll"]) < 2 ** 32
+
+
+def _conv_instance(p):
+    return p["roll"], p["rt"], p["wm"], p["nsteps"] if p["wm"] == 2 else 0
+
+
+def test_cases_reach_every_convolution_instance():
+    """What test_net_march_plans_gpu.py runs: if the prices change, its cases have to follow."""
+    seen = set()
+    for shape, cin, cout, kernel, rt, wm, wn in K.CONV:
+        p = P.conv_plan(shape, cin, cout)
+        assert p["marches"] and (p["roll"], p["rt"], p["wm"], p["wn"]) == (kernel == "roll", rt, wm, wn), (shape, cin, cout, p)
+        assert p["zseg"] >= 4 and shape[1] % p["zseg"] and p["nzs"] > 1
+        seen.add(_conv_instance(p))
+    want = {(0, rt, wm, 0) for rt in (1, 2, 3, 4, 6) for wm in (0, 1)} | {(1, rt, wm, 0) for rt in (1, 2, 3, 4, 5) for wm in (0, 1)}
+    want |= {(0, rt, 2, n) for rt in (1, 2, 3, 4, 6) for n in (7, 14, 21, 41) if (rt, n) != (6, 41)}
+    assert seen == want, (want - seen, seen - want)
+
+
+def test_cases_in_parts_march():
+    kernels = set()
+    for shape, cup, cs, cout in K.PARTS:
+        f, b, g = P.conv_plan(shape, cup + cs, cout), P.conv_plan(shape, cout, cup + cs), P.wgrad_plan(shape, cup + cs, cout)
+        assert f["marches"] and b["marches"] and g["marches"] and f["zseg"] >= 4 and b["zseg"] >= 4
+        kernels |= {("up", f["roll"], f["wm"]), ("split", b["roll"], b["wm"]), ("wgrad", g["cf"])}
+    assert kernels >= {("up", 0, 0), ("up", 0, 1), ("up", 0, 2), ("up", 1, 0), ("up", 1, 1), ("split", 0, 0), ("split", 0, 1),
+                       ("split", 0, 2), ("split", 1, 0), ("split", 1, 1), ("wgrad", 1), ("wgrad", 2), ("wgrad", 3)}
+
+
+def test_cases_of_weight_gradients():
+    for shape, cin, cout, cf, runs, fewer, part, short in K.WGRAD:
+        p = P.wgrad_plan(shape, cin, cout)
+        got = (p["cf"], p["per"] > 1, -(-cin // 16) % p["cf"] != 0, p["tx"] * p["ty"] % 32 != 0, shape[1] % p["zseg"] != 0)
+        assert p["marches"] and got == (cf, runs, fewer, part, short), (shape, cin, cout, p)

@@ -222,7 +222,8 @@ inline bool wgrad_march_search(const pvnet_shape& s, int cin, int cout, WgradMar
                     const double B = (double)splits * nf * st, za = (double)s.d / nzs;
                     const double alone = per * (881 + 7.67 * hp + 1260 * (za + 2) + za * gr * (238 + 218.0 * cf));
                     const double cu = per * za * (gr * std::max(118.0 * cf, 26.2 * (7 + cf)) + 0.66 * (hp + cf * gr * 32));
-                    const double cost = 7.18 + rounds_of(B, cc, cu, alone, 0.41) / CLOCKS_US + splits * (6.72e-5 * cin * cout + 6.7e-4);
+                    // the last: looking for columns that are not finite
+                    const double cost = 7.28 + rounds_of(B, cc, cu, alone, 0.41) / CLOCKS_US + splits * (6.72e-5 * cin * cout + 6.7e-4) + 8.4e-5 * cin * cout;
                     if (us == 0 || cost < us) {
                         us = cost;
                         best = WgradMarch{tx, ty, s.w / tx, s.h / ty, zseg, nzs, tx + 2, hp, gr, su, fu, cf, st, nf, (int)units, per, splits, lds};
@@ -235,7 +236,8 @@ inline bool wgrad_march_search(const pvnet_shape& s, int cin, int cout, WgradMar
 }
 
 // The tiled weight-gradient kernel: bn output channels by 64 k-values a block, the voxels in nsplit runs of mchunk (LDS
-// fills of 128 voxels).
+// fills of 128 voxels).  At most 2,048 blocks where there are several splits: two rounds of the four that a CU holds
+// (one split more began a third: 27 taps, 8 x 24^3, 64 -> 160 309 us, 274 so; 96 -> 96 287 and 256).
 struct TiledWgrad {
     int32_t bn, ktiles, ntiles, nsplit, mchunk;
 };
@@ -243,7 +245,7 @@ struct TiledWgrad {
 inline TiledWgrad tiled_wgrad(int64_t M, int ntaps, int cin, int cout) {
     const int bn = cout <= 16 ? 16 : (cout <= 32 || cout % 64 != 0) ? 32 : 64;
     const int ktiles = (ntaps * cin + 63) / 64, ntiles = (cout + bn - 1) / bn;
-    const int64_t want = 2048 / (ktiles * ntiles) + 1, fills = (M + 127) / 128;
+    const int64_t want = 2048 / (ktiles * ntiles), fills = (M + 127) / 128;
     const int64_t ns = std::min<int64_t>(std::max<int64_t>(want, 1), std::max<int64_t>(fills, 1)), per = (fills + ns - 1) / ns;
     return {bn, ktiles, ntiles, (int32_t)((M + per * 128 - 1) / (per * 128)), (int32_t)(per * 128)};
 }

@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 CASES = [
     # shape, cin, cout, x tiles per block, runs per block > 1
     ((2, 3, 8, 8), 8, 64, 1, False),
-    ((1, 9, 8, 8), 16, 64, 1, False),      # the last run of planes is short
+    ((2, 5, 18, 48), 64, 8, 1, False),     # the last run of planes is short
     ((2, 5, 15, 16), 32, 64, 1, False),    # part of a 32-voxel group
     ((2, 8, 14, 20), 200, 160, 1, True),
     ((3, 32, 20, 21), 120, 8, 2, False),

@@ -12,16 +12,19 @@
 // others from x; a copied unit then picks its source, and the upsampled half is never written out.  The output
 // may go to two tensors in the same way, so that skips and gradients are dense rows for the layers and poolings
 // that read them (a training step on 8 x 96^3: 7.03 -> 5.77 ms, of which the upsampling was 0.30, the poolings
-// 0.43 and a skip written into the middle of 96-byte rows 0.22).  Both run the k-steps of k_conv_fwd in the same order (k = tap * cin + ci, 32 per MFMA), so every output
-// equals that kernel's bit for bit.  The weights are the MFMA's A operand and the voxels its B operand: a
-// lane then holds four consecutive channels of one voxel and writes them with one 8-byte store.
+// 0.43 and a skip written into the middle of 96-byte rows 0.22).
+// Both run the k-steps of k_conv_fwd in the same order (k = tap * cin + ci, 32 per MFMA), so every output equals that
+// kernel's bit for bit.  The weights are the MFMA's A operand and the voxels its B operand: a lane then holds four
+// consecutive channels of one voxel and writes them with one 8-byte store.
 //
-// What bounds them: the narrow layers the LDS (1 KB of voxels per MFMA when only 16 outputs share it; the
-// weights of the ring kernel sit in registers for that reason) and memory, the deep ones the latency of short
-// runs on few voxels.  Measured against the gathering and brick kernels they replace, bf16, us per call
-// (batch x grid, channels): 8 x 96^3 16->16 231 -> 141, 48->16 748 -> 424, 16->48 562 -> 400, 8->16 152 -> 106;
-// 8 x 48^3 32->32 83 -> 72, 96->32 452 -> 237; 8 x 24^3 64->64 83 -> 57, 224->64 305 -> 133; 8 x 12^3
-// 160->160 96 -> 46; 1 x 24 x 24 x 48 64->64 40 -> 24; 3 x 20 x 18 x 28 160->64 96 -> 40.
+// What bounds them (counters of a training step on 8 x 96^3): in the narrow layers nothing alone.  The matrix cores
+// are busy 28 to 31 % of the time, the LDS 40 to 44 % (1 KB of voxels per MFMA when only 16 outputs share it; the
+// weights of the ring kernel sit in registers for that reason), and the waves wait 33 to 44 % of theirs.  The deep
+// layers, with weights from L2, wait 60 % (matrix cores 18 %): the latency of short runs on few voxels.  Measured
+// against the gathering and brick kernels they replace, bf16, us per call (batch x grid, channels): 8 x 96^3 16->16
+// 231 -> 124, 48->16 748 -> 389, 16->48 562 -> 355, 8->16 152 -> 99; 8 x 48^3 32->32 83 -> 68, 96->32 452 -> 214;
+// 8 x 24^3 64->64 83 -> 57, 224->64 305 -> 132; 8 x 12^3 160->160 96 -> 43; 1 x 24 x 24 x 48 64->64 40 -> 23;
+// 3 x 20 x 18 x 28 160->64 96 -> 37.
 #pragma once
 
 __device__ uint4 g_march_zero[4];  // source of the units outside the box

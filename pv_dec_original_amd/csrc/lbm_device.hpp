@@ -88,7 +88,7 @@ __device__ __forceinline__ void moments(const R (&f)[27], R& rho, R (&u)[3]) {
 // are left out: each adds a signed zero, which changes no later value.  What the left-out products do keep is that an
 // infinite velocity makes every direction not a number: `one` carries that.  The 16-bit steps are bound by vector
 // instructions: 968,846 nodes, D3Q19, FP16, all in cache, with WSS in every step 34.5 -> 31.6 us a step (19.0 M
-// vector instructions of 4 clocks before: 31 us of the chip).
+// vector instructions of 4 clocks before: 31 us of the chip; 15.7 M now).
 template <int Q, int D>
 struct Dir {
     static constexpr int x = Lat<Q>::cx[D], y = Lat<Q>::cy[D], z = Lat<Q>::cz[D];

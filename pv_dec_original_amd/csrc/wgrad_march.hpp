@@ -11,14 +11,14 @@
 // (its own voxels only), and a wave reads CF + 7 fragments for 7 CF MFMAs.  Wave v owns the shifts v, v + 4, ..
 // (7 of them; the 28th is a repeat that is not written), so every sum is complete within its wave.  Blocks are
 // splits of the voxels, summed by k_sum_splits, which also sees to an x that is not finite (here it meets the zeros
-// around dy's box).  The bias gradient is one more MFMA per dy fragment of the
-// centre tap, with ones for x.
+// around dy's box).  The bias gradient is one more MFMA per dy fragment of the centre tap, with ones for x.
 //
-// What bounds it: at CF = 1 the LDS (8 KB of fragments for 7 MFMAs), at CF = 3 the matrix cores and the LDS
-// alike.  Measured against the kernels it replaces (register transposes, one LDS copy of x per x shift or a
-// gather per tap; split sums included), us per call, batch x grid, channels in -> out: 8 x 96^3 48->16
-// 1032 -> 307, 16->16 346 -> 172, 8->16 200 -> 172; 8 x 48^3 96->32 301 -> 163, 32->32 114 -> 80;
-// 8 x 24^3 224->64 339 -> 127, 64->64 115 -> 55; 8 x 12^3 160->160 111 -> 62; 3 x 20 x 18 x 28 64->160 92 -> 50.
+// What bounds it (counters of a training step on 8 x 96^3): at CF = 1 the LDS (8 KB of fragments for 7 MFMAs: busy 49 % of
+// the time, matrix cores 26 %, waits 44 % of the waves'), at CF = 3 the matrix cores first (43 %; LDS 26 %, waits 40 %).
+// Measured against the kernels it replaces (register transposes, one LDS copy of x per x shift or a gather per tap;
+// split sums included), us per call, batch x grid, channels in -> out: 8 x 96^3 48->16 1032 -> 324, 16->16 346 -> 152,
+// 8->16 200 -> 138; 8 x 48^3 96->32 301 -> 163, 32->32 114 -> 73; 8 x 24^3 224->64 339 -> 121, 64->64 115 -> 51;
+// 8 x 12^3 160->160 111 -> 62; 3 x 20 x 18 x 28 64->160 92 -> 43.
 #pragma once
 
 typedef short tr4 __attribute__((ext_vector_type(4)));

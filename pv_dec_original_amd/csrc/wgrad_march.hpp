@@ -18,7 +18,8 @@
 // Measured against the kernels it replaces (register transposes, one LDS copy of x per x shift or a gather per tap;
 // split sums included), us per call, batch x grid, channels in -> out: 8 x 96^3 48->16 1032 -> 324, 16->16 346 -> 152,
 // 8->16 200 -> 138; 8 x 48^3 96->32 301 -> 163, 32->32 114 -> 73; 8 x 24^3 224->64 339 -> 121, 64->64 115 -> 51;
-// 8 x 12^3 160->160 111 -> 62; 3 x 20 x 18 x 28 64->160 92 -> 43.
+// 8 x 12^3 160->160 111 -> 62; 3 x 20 x 18 x 28 64->160 92 -> 43.  With its input in two parts, in a training step,
+// 48->16 takes 266 us (sums apart): the upsampled channels are read from a tensor an eighth the size.
 #pragma once
 
 typedef short tr4 __attribute__((ext_vector_type(4)));
